@@ -166,7 +166,8 @@ struct ContactView {
     // Tet vertices of contact scenes are updated in place; a contact pair may join two vertices
     // of one parallel group, so contact partners of the solving vertex's own group are read from
     // the iteration-start snapshot (their value at the start of the group, as the reference's
-    // positionsNext + copy gives); vgroup: per vertex parallel group (-1: not solved)
+    // positionsNext + copy gives); vgroup: per vertex parallel group (-1: not solved), also in
+    // the snapshot's w lane (as int bits)
     const float4* snap;
     const int* vgroup;
     // 0: cloth contact model (VF / FV / EE repulsion, bounds and truncation); 1: penetration

@@ -69,6 +69,8 @@ hipError_t convergence_scratch_init(int device, double** scratch);
 hipError_t launch_convergence_final_sum(const double* partial, int off0, int n0, int off1, int n1, int off2, int n2,
                                         double* out, hipStream_t stream);
 
+// snap[i] = pos[i] with the int bits of vgroup[i] in w (ContactView::snap).
+hipError_t launch_contact_snapshot(const float4* pos, const int* vgroup, float4* snap, int n, hipStream_t stream);
 // dst[i] = src[i] for n float4 elements (bandwidth / profiler calibration).
 hipError_t launch_stream_copy(const float4* src, float4* dst, int64_t n, hipStream_t stream);
 

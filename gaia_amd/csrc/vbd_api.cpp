@@ -1204,7 +1204,9 @@ void plan_reset_counters(gvbd_context* ctx, PlanObj& p) {
 void plan_contact_snapshot(gvbd_context* ctx, PlanObj& p) {
     for (int32_t sid : p.scenes) {
         SceneObj& s = scene_of(ctx, sid);
-        if (s.cd) hip_check(launch_stream_copy(s.view.pos, s.dev.snap, s.nv, ctx->stream), "snapshot launch");
+        if (s.cd)
+            hip_check(launch_contact_snapshot(s.view.pos, s.dev.vgroup, s.dev.snap, s.nv, ctx->stream),
+                      "snapshot launch");
     }
 }
 
