@@ -1015,6 +1015,7 @@ struct PenView {
     const BvhNode* tNodes;   // tet tree
     int tN;
     const BvhNode* fNodes;   // face tree (current positions)
+    const int* fRight;       // right child of every internal face-tree node
     const int* fMesh;        // per face-tree node: the mesh of its faces, -1 for several
     int fN;
     const BvhNode* sNodes;   // swept-face tree (prev and current positions)
@@ -1281,123 +1282,169 @@ __device__ __forceinline__ float box_far2(V3 p, const BvhNode& n) {
     return dx * dx + dy * dy + dz * dz;
 }
 
-// DCD pass 2, one thread per contained vertex: the closest face of the containing tet's mesh
-// that passes the checks, lower face id on equal distance (DiscreteCollisionDetector.cpp:
-// 514-560). The faces are first taken in ascending (distance, id), the first one passing the
-// checks being the answer: each round is a nearest-face query on the face tree over the faces
-// after the last rejected one, pruning subtrees of other meshes, boxes surely farther than the
-// round's best and boxes surely closer than the rejected face. The nearest face passes for
-// nearly every vertex, so the costly checks run about once per vertex. After kNearestRounds
-// rejected faces the rest is searched in one traversal that checks every face closer than the
-// best valid one so far (each round repeats a traversal, which costs more than the extra checks
-// once many faces are rejected). Both orders give the same answer.
-__global__ __launch_bounds__(64) void pen_closest_kernel(PenView S) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= S.counts[4]) return;
-    const int v = S.list[i];
-    const int ht = S.inTet[v];
-    const V3 p = ld(S.pos, v);
-    const int qm = S.vMesh[v];
-    const int hm = S.tetMesh[ht];
-    float lastD = -1.f;
-    int lastF = -1;
-    int hit = -1;
-    bool exhausted = false;
-    const int firstLeaf = S.fN - 1;
-    for (int round = 0; round < kNearestRounds && hit < 0 && !exhausted; ++round) {
-        float best = FLT_MAX;
-        int bestF = -1, bestType = 0;
-        V3 bestCp = p;
-        const float near2 = lastD * lastD;
-        int node = S.fN > 0 ? 0 : -1;
-        for (int visits = 0; node >= 0; ++visits) {
-            if (visits > 2 * S.fN) {
-                atomicOr(S.error, 1);
-                break;
-            }
-            const BvhNode nd = S.fNodes[node];
-            const int skip = __float_as_int(nd.hi.w);
-            // prune subtrees of other meshes' faces, boxes surely farther than the round's best and
-            // boxes surely closer than the last rejected face (margins for rounding)
-            const int nm = S.fMesh[node];
-            if ((nm >= 0 && nm != hm) || (bestF >= 0 && box_dist2(p, nd) > best * best * 1.0001f + 1e-12f) ||
-                (lastF >= 0 && box_far2(p, nd) * 1.0001f + 1e-12f < near2)) {
-                node = skip;
-                continue;
-            }
-            if (node < firstLeaf) {
-                node = __float_as_int(nd.lo.w);
-                continue;
-            }
-            node = skip;
-            const int f = __float_as_int(nd.lo.w);
-            const int4 fv = S.faces[f];
-            if (fv.w != hm) continue;
-            int type;
-            const V3 cp = closest_point_triangle(p, ld(S.pos, fv.x), ld(S.pos, fv.y), ld(S.pos, fv.z), type);
-            if (hm == qm && type <= AT_C && (type == AT_A ? fv.x : (type == AT_B ? fv.y : fv.z)) == v) continue;
-            const float d = vnorm(p - cp);
-            if (!(d > lastD || (d == lastD && f > lastF))) continue;  // taken in an earlier round
-            if (bestF >= 0 && !(d < best || (d == best && f < bestF))) continue;
-            best = d;
-            bestF = f;
-            bestType = type;
-            bestCp = cp;
+// ---- traversal of a tree by a whole wave ----
+// The nodes to visit lie on a stack in LDS; a step pops up to 64 of them, one per lane, and pushes
+// the children of those that are not pruned. The stack stays sorted by depth, so that it holds little
+// more than 64 nodes per level; when it runs full a step pops fewer, down to one (depth first), which
+// needs at most one entry per level, the reserve. kWaveStack entries are enough for any tree of the
+// refit schedule's depth.
+constexpr int kWaveStack = 1024;
+constexpr int kWaveReserve = kMaxDepth + 2;
+
+// Visits the nodes of a tree of n leaves, each step up to 64 side by side: keep(node, leaf, data) says
+// whether a node is of interest and handles it if it is a leaf; step() is called by every lane after
+// each step. Called by the one wave of a block with `stack` in LDS.
+template <class Keep, class Step>
+__device__ __forceinline__ void wave_traverse(const BvhNode* nodes, const int* right, int n, int* stack, int* error,
+                                              Keep&& keep, Step&& step) {
+    const int lane = threadIdx.x;
+    const int firstLeaf = n - 1;
+    int size = n > 0 ? 1 : 0;
+    if (lane == 0) stack[0] = 0;
+    __syncthreads();
+    while (size > 0) {
+        const int m = min(min(64, size), max(kWaveStack - kWaveReserve - size, 1));
+        const int base = size - m;
+        const int node = lane < m ? stack[base + lane] : -1;
+        __syncthreads();
+        int left = -1, rgt = -1;
+        if (node >= 0) {
+            const bool leaf = node >= firstLeaf;
+            if (!leaf) rgt = right[node];
+            const BvhNode nd = nodes[node];
+            if (keep(node, leaf, nd) && !leaf) left = __float_as_int(nd.lo.w);
         }
-        if (bestF < 0) {
-            exhausted = true;  // no face left
+        const unsigned long long grow = __ballot(left >= 0);
+        const int kids = 2 * __popcll(grow);
+        if (base + kids > kWaveStack) {  // a tree deeper than the refit schedule supports
+            if (lane == 0) atomicOr(error, 1);
             break;
         }
-        if (pen_face_valid(S, qm, hm, ht, p, bestF, bestType, bestCp)) hit = bestF;
-        lastD = best;
-        lastF = bestF;
+        if (left >= 0) {
+            const int at = base + 2 * __popcll(grow & ((1ull << lane) - 1ull));
+            stack[at] = rgt;
+            stack[at + 1] = left;
+        }
+        size = base + kids;
+        step();
+        __syncthreads();
     }
-    if (hit < 0 && !exhausted) {
-        // many near faces rejected (a vertex deep in the other body): one traversal over the faces
-        // after the last rejected one, checking each face closer than the best valid face so far
-        atomicAdd(S.counts + 5, 1);
-        float best = FLT_MAX;
-        const float near2 = lastD * lastD;
-        int node = S.fN > 0 ? 0 : -1;
-        for (int visits = 0; node >= 0; ++visits) {
-            if (visits > 2 * S.fN) {
-                atomicOr(S.error, 1);
-                break;
-            }
-            const BvhNode nd = S.fNodes[node];
-            const int skip = __float_as_int(nd.hi.w);
-            const int nm = S.fMesh[node];
-            if ((nm >= 0 && nm != hm) || (hit >= 0 && box_dist2(p, nd) > best * best * 1.0001f + 1e-12f) ||
-                box_far2(p, nd) * 1.0001f + 1e-12f < near2) {
-                node = skip;
-                continue;
-            }
-            if (node < firstLeaf) {
-                node = __float_as_int(nd.lo.w);
-                continue;
-            }
-            node = skip;
-            const int f = __float_as_int(nd.lo.w);
-            const int4 fv = S.faces[f];
-            if (fv.w != hm) continue;
-            int type;
-            const V3 cp = closest_point_triangle(p, ld(S.pos, fv.x), ld(S.pos, fv.y), ld(S.pos, fv.z), type);
-            if (hm == qm && type <= AT_C && (type == AT_A ? fv.x : (type == AT_B ? fv.y : fv.z)) == v) continue;
-            const float d = vnorm(p - cp);
-            if (!(d > lastD || (d == lastD && f > lastF))) continue;
-            if (hit >= 0 && !(d < best || (d == best && f < hit))) continue;
-            if (!pen_face_valid(S, qm, hm, ht, p, f, type, cp)) continue;
-            best = d;
-            hit = f;
+}
+
+__device__ __forceinline__ float wave_min(float x) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) x = fminf(x, __shfl_xor(x, o, 64));
+    return x;
+}
+
+// A lane's closest face so far (face -1: none) and the closest of the wave's, the lower face id on
+// equal distance.
+struct NearFace {
+    float d;
+    int face, type;
+    V3 cp;
+};
+__device__ __forceinline__ NearFace wave_nearest(NearFace a) {
+    float d = a.face >= 0 ? a.d : FLT_MAX;
+    int f = a.face >= 0 ? a.face : INT_MAX, from = threadIdx.x;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        const float od = __shfl_xor(d, o, 64);
+        const int of = __shfl_xor(f, o, 64), ofrom = __shfl_xor(from, o, 64);
+        if (od < d || (od == d && of < f)) {
+            d = od;
+            f = of;
+            from = ofrom;
         }
     }
-    if (hit < 0) {
-        atomicAdd(S.counts + 1, 1);
-        return;
+    return {__shfl(a.d, from, 64), __shfl(a.face, from, 64), __shfl(a.type, from, 64),
+            V3{__shfl(a.cp.x, from, 64), __shfl(a.cp.y, from, 64), __shfl(a.cp.z, from, 64)}};
+}
+
+// DCD pass 2, one wave per contained vertex: the closest face of the containing tet's mesh that
+// passes the checks, lower face id on equal distance (DiscreteCollisionDetector.cpp:514-560). The
+// faces are first taken in ascending (distance, id), the first one passing the checks being the
+// answer: each round is a nearest-face query on the face tree over the faces after the last
+// rejected one, pruning subtrees of other meshes, boxes surely farther than the round's best and
+// boxes surely closer than the rejected face. The nearest face passes for nearly every vertex, so
+// the costly checks run about once per vertex. After kNearestRounds rejected faces the rest is
+// searched in one traversal that checks every face closer than the best valid one so far. All
+// orders give the same answer.
+// A search is a chain of dependent node loads, and a launch has few of them (the contained
+// vertices: hundreds where the tree has 1e5 nodes), so the wave's 64 lanes share each one: 131 us
+// per launch where one thread per search took 3.87 ms (227 contained vertices, 55,296 faces).
+__global__ __launch_bounds__(64) void pen_closest_kernel(PenView S) {
+    __shared__ int stack[kWaveStack];
+    const int lane = threadIdx.x;
+    const int contained = S.counts[4];
+    for (int i = blockIdx.x; i < contained; i += gridDim.x) {
+        const int v = S.list[i];
+        const int ht = S.inTet[v];
+        const V3 p = ld(S.pos, v);
+        const int qm = S.vMesh[v];
+        const int hm = S.tetMesh[ht];
+        float lastD = -1.f;
+        int lastF = -1;
+        int hit = -1;
+        // the wave's nearest face after (lastD, lastF); with `checked`, its nearest valid one
+        const auto nearest = [&](bool checked) {
+            NearFace mine{FLT_MAX, -1, 0, p};
+            float bound = FLT_MAX;  // the wave's best distance: d > bound cannot win
+            const float near2 = lastD * lastD;
+            wave_traverse(
+                S.fNodes, S.fRight, S.fN, stack, S.error,
+                [&](int node, bool leaf, const BvhNode& nd) {
+                    // subtrees of other meshes' faces, boxes surely farther than the best and boxes
+                    // surely closer than the last rejected face are pruned (margins for rounding)
+                    const int nm = S.fMesh[node];
+                    if ((nm >= 0 && nm != hm) || box_dist2(p, nd) > bound * bound * 1.0001f + 1e-12f ||
+                        (lastF >= 0 && box_far2(p, nd) * 1.0001f + 1e-12f < near2))
+                        return false;
+                    if (!leaf) return true;
+                    const int f = __float_as_int(nd.lo.w);
+                    const int4 fv = S.faces[f];
+                    if (fv.w != hm) return false;
+                    int type;
+                    const V3 cp = closest_point_triangle(p, ld(S.pos, fv.x), ld(S.pos, fv.y), ld(S.pos, fv.z), type);
+                    if (hm == qm && type <= AT_C && (type == AT_A ? fv.x : (type == AT_B ? fv.y : fv.z)) == v) return false;
+                    const float d = vnorm(p - cp);
+                    if (!(d > lastD || (d == lastD && f > lastF))) return false;  // taken in an earlier round
+                    if (d > bound || (mine.face >= 0 && !(d < mine.d || (d == mine.d && f < mine.face)))) return false;
+                    if (checked && !pen_face_valid(S, qm, hm, ht, p, f, type, cp)) return false;
+                    mine = {d, f, type, cp};
+                    return false;
+                },
+                [&]() { bound = wave_min(mine.d); });
+            return wave_nearest(mine);
+        };
+        bool exhausted = false;
+        for (int round = 0; round < kNearestRounds && hit < 0; ++round) {
+            const NearFace best = nearest(false);
+            if (best.face < 0) {
+                exhausted = true;  // no face left
+                break;
+            }
+            int valid = 0;
+            if (lane == 0) valid = pen_face_valid(S, qm, hm, ht, p, best.face, best.type, best.cp) ? 1 : 0;
+            if (__shfl(valid, 0, 64)) hit = best.face;
+            lastD = best.d;
+            lastF = best.face;
+        }
+        if (hit < 0 && !exhausted) {
+            // many near faces rejected (a vertex deep in the other body)
+            if (lane == 0) atomicAdd(S.counts + 5, 1);
+            hit = nearest(true).face;
+        }
+        if (lane == 0) {
+            if (hit < 0) {
+                atomicAdd(S.counts + 1, 1);
+            } else {
+                S.stored[v] = 1;
+                S.rec[(int64_t)v * S.cap].face = hit;
+                atomicAdd(S.counts, 1);
+            }
+        }
     }
-    S.stored[v] = 1;
-    S.rec[(int64_t)v * S.cap].face = hit;
-    atomicAdd(S.counts, 1);
 }
 
 __device__ __forceinline__ float poly3(const float c[4], float x) { return ((c[3] * x + c[2]) * x + c[1]) * x + c[0]; }
@@ -2161,6 +2208,7 @@ void ContactDetector::penetrationDcd(bool rebuild) {
     S.tNodes = tb_.nodes;
     S.tN = tb_.n;
     S.fNodes = fb_.nodes;
+    S.fRight = fb_.right;
     S.fMesh = fb_.mesh;
     S.fN = fb_.n;
     S.P = penHost_.params;
@@ -2174,7 +2222,8 @@ void ContactDetector::penetrationDcd(bool rebuild) {
     S.error = error_;
     if (nSurf_ > 0) {
         hipLaunchKernelGGL(pen_contain_kernel, dim3((nSurf_ + 63) / 64), dim3(64), 0, stream_, S);
-        hipLaunchKernelGGL(pen_closest_kernel, dim3((nSurf_ + 63) / 64), dim3(64), 0, stream_, S);
+        // a wave per contained vertex (their number is only known on the device); 4096 waves fill the chip
+        hipLaunchKernelGGL(pen_closest_kernel, dim3(std::min(nSurf_, 4096)), dim3(64), 0, stream_, S);
     }
     hip_check(hipGetLastError(), "penetration DCD launch");
 }
