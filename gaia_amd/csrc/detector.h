@@ -38,9 +38,16 @@ struct alignas(16) EEContactRec {
     float d;
 };
 
+// Both children of an internal node, side by side for the traversals that test them together: box lo
+// (w: the child's index if it is internal, its leaf word otherwise) and hi (w: 1 for a leaf).
+struct alignas(64) BvhPair {
+    float4 lo0, hi0, lo1, hi1;
+};
+
 struct DeviceBvh {
     int n = 0;                       // primitives
     BvhNode* nodes = nullptr;        // 2n - 1
+    BvhPair* pairs = nullptr;        // n - 1 (1 for a single primitive): set at every refit
     int* parent = nullptr;           // 2n - 1
     int* right = nullptr;            // n - 1: right child of each internal node (refit)
     int* jump = nullptr;             // 4 (n - 1): depth / ancestor buffers of the depth computation
@@ -196,7 +203,7 @@ class ContactDetector {
     void buildBvh(DeviceBvh& b, int kind, const float4* boxes = nullptr);
     void refitBvh(DeviceBvh& b, int kind, hipStream_t stream, const float4* boxes = nullptr,
                   const int* gate = nullptr);
-    void allocBvh(DeviceBvh& b, int n);
+    void allocBvh(DeviceBvh& b, int n, bool pairs);
     void setupPenetrationDevice();
     // the face-side and edge-side work of a pass are independent: side_ runs the edge side
     // between fork() (side_ waits for stream_) and join() (stream_ waits for side_)

@@ -7,8 +7,8 @@
 //           node depths -> internal nodes sorted by depth (the refit schedule)
 //   refit   leaf boxes from the current positions, then one launch per depth level, deepest
 //           first (no atomics, no inter-block waits)
-//   query   one thread per vertex (VF, query box of half-size r around the vertex) or per edge
-//           (EE, half-size r + |e|/2 around the midpoint), stack traversal, exact tests with the
+//   query   waves of up to 64 vertices (VF, query box of half-size r around the vertex) or edges
+//           (EE, the segment's box grown by r), traversal shared by the wave, exact tests with the
 //           reference's predicates (ClothContactDetector.cpp:144-288, 731-813; CollisionGeometry.h:
 //           90-267; TriMeshCollisionGeometry.cpp:7-186)
 //
@@ -186,8 +186,10 @@ struct CDView {
     const int* vvBegin;
     const int* vvNei;
     const BvhNode* fNodes;
+    const BvhPair* fPairs;
     int fN;
     const BvhNode* eNodes;
+    const BvhPair* ePairs;
     int eN;
     float r;
     int vfCap, eeCap;
@@ -256,42 +258,82 @@ __device__ bool edge_feasible(const CDView& S, V3 p, int e) {
     return true;
 }
 
-// VF query of one vertex (ClothContactDetector.cpp:144-288 per candidate face)
-// CAP bounds the per-thread candidate list (the runtime vfCap is at most CAP); only the face
-// id and the packed (type, primitive) key are kept per candidate, the distance is recomputed
-// for the stored ones at the end, so the list costs 2 CAP registers.
-template <bool RECORD, int CAP>
-__global__ __launch_bounds__(256) void vf_query_kernel(CDView S) {
+// The primitive of face f (vertices fv) that a closest point of region `type` lies on: its id, and in
+// `ptype` its kind (0 vertex, 1 edge, 2 the face).
+__device__ __forceinline__ int closest_primitive(const CDView& S, int f, int4 fv, int type, int& ptype) {
+    if (type <= AT_C) {
+        ptype = 0;
+        return type == AT_A ? fv.x : (type == AT_B ? fv.y : fv.z);
+    }
+    if (type == AT_INTERIOR) {
+        ptype = 2;
+        return f;
+    }
+    ptype = 1;
+    const int4 fe = S.faceEdges[f];
+    return type == AT_AB ? fe.x : (type == AT_BC ? fe.y : fe.z);
+}
+
+__device__ __forceinline__ bool primitive_feasible(const CDView& S, V3 p, int ptype, int prim) {
+    return ptype == 0 ? vertex_feasible(S, p, prim) : (ptype == 1 ? edge_feasible(S, p, prim) : true);
+}
+
+// Edge e1 (mesh m1, at p1, p2) against the edge of a leaf (its box and tag): false if
+// they are not closer than r or share a vertex; `contact` if the closest points pass the projection
+// tests (ClothContactDetector.cpp:731-813). The other edge's endpoints come from the leaf's box (the
+// positions of the last refit, which are the query's): no edge or position loads for the many leaves
+// beyond r.
+struct EdgePair {
+    int e2;
+    float mua, mub, d;
+    bool contact;
+};
+__device__ __forceinline__ bool edge_pair(const CDView& S, int e1, int m1, V3 p1, V3 p2, float4 lo, float4 hi,
+                                          EdgePair& out) {
+    const int tag = __float_as_int(lo.w);
+    const int e2 = tag & kLeafPrimMask;
+    const V3 q1 = {(tag >> kLeafPrimBits) & 1 ? hi.x : lo.x, (tag >> (kLeafPrimBits + 1)) & 1 ? hi.y : lo.y,
+                   (tag >> (kLeafPrimBits + 2)) & 1 ? hi.z : lo.z};
+    const V3 q2 = {(tag >> kLeafPrimBits) & 1 ? lo.x : hi.x, (tag >> (kLeafPrimBits + 1)) & 1 ? lo.y : hi.y,
+                   (tag >> (kLeafPrimBits + 2)) & 1 ? lo.z : hi.z};
+    V3 c1, c2;
+    segment_closest_points(p1, p2, q1, q2, c1, c2, out.mua, out.mub);
+    out.d = dist(c1, c2);
+    out.e2 = e2;
+    // minima start at r, so an edge at d >= r (or NaN) leaves them unchanged whether or not the
+    // topology filter below would have skipped it
+    if (!(out.d < S.r)) return false;
+    if (S.eMesh[e2] == m1) {
+        if (e2 == e1) return false;
+        const int4 a = S.edges[e1], b = S.edges[e2];
+        if (a.x == b.x || a.x == b.y || a.y == b.x || a.y == b.y) return false;
+    }
+    const V3 ev1 = p2 - p1, ev2 = q2 - q1;
+    out.contact = (dot(c2 - p1, ev1) >= 0.f && dot(p2 - c2, ev1) >= 0.f) ||
+                  (dot(c1 - q1, ev2) >= 0.f && dot(q2 - c1, ev2) >= 0.f);
+    return true;
+}
+
+// Record pass of one vertex (ClothContactDetector.cpp:144-288 per candidate face): every face within
+// r and every distinct closest primitive, into the segments sized by the query pass's counts, in the
+// tree's depth-first order (the record lists' order). Walks the skip links.
+__global__ __launch_bounds__(256) void vf_record_kernel(CDView S) {
     // vertices in Morton order: a wavefront's queries are spatial neighbours, and so are the
     // blocks of one XCD
-    if (S.gate && !*S.gate) return;
     const int t = xcd_block_index() * blockDim.x + threadIdx.x;
     if (t >= S.nv) return;
     const int v = S.vOrder ? (int)(S.vOrder[t] & 0xFFFFFFFFu) : t;
-    if (S.vQuery && !S.vQuery[v]) {  // not a surface vertex: no VF contacts
-        if (!RECORD) {
-            S.vfMin[v] = S.r;
-            S.vfPairCount[v] = 0;
-            S.vfStored[v] = 0;
-            S.vfOverflow[v] = 0;
-        }
-        return;
-    }
+    if (S.vQuery && !S.vQuery[v]) return;  // not a surface vertex: no VF contacts
     const V3 p = ld(S.pos, v);
     const int mesh = S.vMesh[v];
     const float r = S.r;
     const float rq = r * 1.0001f + 1e-7f;
     const V3 qlo = {p.x - rq, p.y - rq, p.z - rq}, qhi = {p.x + rq, p.y + rq, p.z + rq};
-    float vmin = r;
-    int pairs = 0, stored = 0, overflow = 0;
-    int kKey[CAP], kFace[CAP];  // key: primitive | type << 30
-    int64_t pairBase = 0, keyBase = 0;
-    int recKeys = 0, pairCap = 0;
-    if (RECORD) {
-        pairCap = S.vfPairCount[v];
-        pairBase = S.vfOffset[v];
-        keyBase = pairBase;  // the key segment has the pair segment's size (an upper bound)
-    }
+    int pairs = 0;
+    const int pairCap = S.vfPairCount[v];
+    const int64_t pairBase = S.vfOffset[v];
+    const int64_t keyBase = pairBase;  // the key segment has the pair segment's size (an upper bound)
+    int recKeys = 0;
     const int firstLeaf = S.fN - 1;
     int node = S.fN > 0 ? 0 : -1;
     for (int visits = 0; node >= 0; ++visits) {
@@ -317,95 +359,305 @@ __global__ __launch_bounds__(256) void vf_query_kernel(CDView S) {
         const V3 cp = closest_point_triangle(p, ld(S.pos, fv.x), ld(S.pos, fv.y), ld(S.pos, fv.z), type);
         const float d = dist(p, cp);
         if (!(d < r)) continue;
-        vmin = fminf(d, vmin);
-        atomicMin(S.faceMin + f, __float_as_int(d));
-        if (RECORD) {
-            // the record pass repeats the counting pass's traversal; never write past its count
-            if (pairs >= pairCap) {
-                atomicOr(S.error, 4);
-                break;
-            }
-            S.recVF[pairBase + pairs] = make_int2(v, f);
-            S.recVFd[pairBase + pairs] = d;
+        // the record pass repeats the query pass's tests; never write past its count
+        if (pairs >= pairCap) {
+            atomicOr(S.error, 4);
+            break;
         }
+        S.recVF[pairBase + pairs] = make_int2(v, f);
+        S.recVFd[pairBase + pairs] = d;
         ++pairs;
-        int prim, ptype;
-        if (type <= AT_C) {
-            prim = type == AT_A ? fv.x : (type == AT_B ? fv.y : fv.z);
-            ptype = 0;
-        } else if (type == AT_INTERIOR) {
-            prim = f;
-            ptype = 2;
-        } else {
-            const int4 fe = S.faceEdges[f];
-            prim = type == AT_AB ? fe.x : (type == AT_BC ? fe.y : fe.z);
-            ptype = 1;
-        }
+        int ptype;
+        const int prim = closest_primitive(S, f, fv, type, ptype);
         // dedup on (type, primitive): keep the lowest face id as the representative
         bool dup = false;
-        if (!RECORD) {
-            const int key = prim | (ptype << 30);
-#pragma unroll
-            for (int k = 0; k < CAP; ++k)
-                if (k < stored && !dup && kKey[k] == key) {
-                    if (f < kFace[k]) kFace[k] = f;
-                    dup = true;
+        for (int k = 0; k < recKeys; ++k) {
+            int4& rk = S.recKeys[keyBase + k];
+            if (rk.y == ptype && rk.z == prim) {
+                if (f < rk.w) {
+                    rk.w = f;
+                    S.recKeysD[keyBase + k] = d;
                 }
-        } else {
-            for (int k = 0; k < recKeys; ++k) {
-                int4& rk = S.recKeys[keyBase + k];
-                if (rk.y == ptype && rk.z == prim) {
-                    if (f < rk.w) {
-                        rk.w = f;
-                        S.recKeysD[keyBase + k] = d;
-                    }
-                    dup = true;
-                    break;
-                }
+                dup = true;
+                break;
             }
         }
-        if (dup) continue;
-        bool ok = true;
-        if (ptype == 0)
-            ok = vertex_feasible(S, p, prim);
-        else if (ptype == 1)
-            ok = edge_feasible(S, p, prim);
-        if (!ok) continue;
-        if (RECORD) {
-            S.recKeys[keyBase + recKeys] = make_int4(v, ptype, prim, f);
-            S.recKeysD[keyBase + recKeys] = d;
-            ++recKeys;
-        } else {
-            // keep the vfCap keys with the lowest representative faces (order-free selection)
-            int slot = stored;
-            if (stored == S.vfCap) {
-                overflow = 1;
-                slot = 0;
-                int worst = kFace[0];
-#pragma unroll
-                for (int k = 1; k < CAP; ++k)
-                    if (k < stored && kFace[k] > worst) {
-                        worst = kFace[k];
-                        slot = k;
-                    }
-                if (f > worst) slot = -1;
-            } else {
-                ++stored;
-            }
-#pragma unroll
-            for (int k = 0; k < CAP; ++k)
-                if (k == slot) {
-                    kKey[k] = prim | (ptype << 30);
-                    kFace[k] = f;
+        if (dup || !primitive_feasible(S, p, ptype, prim)) continue;
+        S.recKeys[keyBase + recKeys] = make_int4(v, ptype, prim, f);
+        S.recKeysD[keyBase + recKeys] = d;
+        ++recKeys;
+    }
+    for (int k = recKeys; k < pairs; ++k) S.recKeys[keyBase + k] = make_int4(v, -1, -1, -1);
+}
+
+// Record pass of one edge (ClothContactDetector.cpp:731-813), as the vertices'.
+__global__ __launch_bounds__(256) void ee_record_kernel(CDView S) {
+    const int t = xcd_block_index() * blockDim.x + threadIdx.x;
+    if (t >= S.ne) return;
+    const int e1 = S.eOrder ? (int)(S.eOrder[t] & 0xFFFFFFFFu) : t;
+    const int4 a = S.edges[e1];
+    const int m1 = S.eMesh[e1];
+    const V3 p1 = ld(S.pos, a.x), p2 = ld(S.pos, a.y);
+    const float r = S.r;
+    const float rq = r * 1.0001f + 1e-7f;
+    const V3 qlo = {fminf(p1.x, p2.x) - rq, fminf(p1.y, p2.y) - rq, fminf(p1.z, p2.z) - rq};
+    const V3 qhi = {fmaxf(p1.x, p2.x) + rq, fmaxf(p1.y, p2.y) + rq, fmaxf(p1.z, p2.z) + rq};
+    int count = 0;
+    const int64_t base = S.eeOffset[e1];
+    const int countCap = S.eeCount[e1];
+    const int firstLeaf = S.eN - 1;
+    int node = S.eN > 0 ? 0 : -1;
+    for (int visits = 0; node >= 0; ++visits) {
+        if (visits > 2 * S.eN) {
+            atomicOr(S.error, 1);
+            break;
+        }
+        const BvhNode nd = S.eNodes[node];
+        const int skip = __float_as_int(nd.hi.w);
+        if (!box_overlap(qlo, qhi, nd)) {
+            node = skip;
+            continue;
+        }
+        if (node < firstLeaf) {
+            node = __float_as_int(nd.lo.w);
+            continue;
+        }
+        node = skip;
+        EdgePair e;
+        if (!edge_pair(S, e1, m1, p1, p2, nd.lo, nd.hi, e) || !e.contact) continue;
+        if (count >= countCap) {
+            atomicOr(S.error, 4);
+            break;
+        }
+        S.recEE[base + count] = make_int2(e1, e.e2);
+        S.recEEmu[base + count] = make_float2(e.mua, e.mub);
+        S.recEEd[base + count] = e.d;
+        ++count;
+    }
+}
+
+// ---- traversal of a tree by a whole wave ----
+// Work lies on a stack in LDS: a step pops up to 64 entries, one per lane, and pushes what they lead
+// to. The stack stays sorted by depth (what a step pushes is deeper than all that it left), so that
+// it holds little more than 64 entries per level; when it runs full a step pops fewer, down to one
+// (depth first), which needs at most one more entry per level: the reserve. So a tree of any depth
+// that the refit schedule takes fits.
+constexpr int kWaveReserve = kMaxDepth + 2;
+__device__ __forceinline__ int wave_pop(int size, int cap) {
+    return min(min(64, size), max(cap - kWaveReserve - size, 1));
+}
+__device__ __forceinline__ int lanes_below(unsigned long long mask) {
+    return __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
+}
+
+// Many queries by one wave (a block of 64 threads): Q of them, those whose lane has `active` set,
+// share its lanes. A stack entry is (query, internal node) whose box the query overlaps; the
+// lane that pops it tests both children (one 64-byte BvhPair), so a lane is never idle while any of
+// the wave's queries has a node left, and a query with a long path does not hold up 63 others (one
+// thread per query, following skip links, is bound by the longest chain of dependent node loads and
+// runs the exact tests with few lanes).
+// Leaves go to a queue and are tested 64 at a time: leaf(lane has one, query, lo, hi).
+// Q is a power of two; a stack entry packs the query above the node, a leaf entry has one bit more
+// (which child), so a tree may have 2^(31 - log2 Q) primitives.
+constexpr int kQueryStack = 640;
+constexpr int kLeafQueue = 192;
+template <int Q> constexpr int query_node_bits() {
+    return Q == 32 ? 26 : (Q == 16 ? 27 : 28);
+}
+template <int Q, class Overlap, class Leaf>
+__device__ __forceinline__ void wave_queries(const BvhPair* pairs, int n, bool active, int* stack, int* leaves,
+                                             int* error, Overlap&& overlap, Leaf&& leaf) {
+    constexpr int kBits = query_node_bits<Q>();
+    constexpr unsigned kMask = (1u << kBits) - 1u;
+    const int lane = threadIdx.x;
+    const unsigned long long seeds = __ballot(active && n > 0);
+    if (active && n > 0) stack[lanes_below(seeds)] = (int)((unsigned)lane << kBits);  // the root
+    int size = __popcll(seeds), nl = 0;
+    __syncthreads();
+    while (size > 0 || nl > 0) {
+        if (size > 0) {
+            const int m = wave_pop(size, kQueryStack);
+            const int base = size - m;
+            const unsigned entry = lane < m ? (unsigned)stack[base + lane] : 0u;
+            __syncthreads();
+            const int q = entry >> kBits;
+            bool inA = false, inB = false, lfA = false, lfB = false;
+            unsigned nextA = 0, nextB = 0;
+            if (lane < m) {
+                const BvhPair P = pairs[entry & kMask];
+                if (overlap(q, P.lo0, P.hi0)) {
+                    lfA = __float_as_int(P.hi0.w) != 0;
+                    inA = !lfA;
+                    nextA = ((unsigned)q << kBits) | (unsigned)__float_as_int(P.lo0.w);
                 }
+                if (overlap(q, P.lo1, P.hi1)) {
+                    lfB = __float_as_int(P.hi1.w) != 0;
+                    inB = !lfB;
+                    nextB = ((unsigned)q << kBits) | (unsigned)__float_as_int(P.lo1.w);
+                }
+            }
+            const unsigned long long mA = __ballot(inA), mB = __ballot(inB);
+            const int kids = __popcll(mA) + __popcll(mB);
+            if (base + kids > kQueryStack) {  // a tree deeper than the refit schedule supports
+                if (lane == 0) atomicOr(error, 1);
+                break;
+            }
+            const int at = base + lanes_below(mA) + lanes_below(mB);
+            if (inA) stack[at] = (int)nextA;
+            if (inB) stack[at + (inA ? 1 : 0)] = (int)nextB;
+            size = base + kids;
+            const unsigned long long kA = __ballot(lfA), kB = __ballot(lfB);
+            if (lfA) leaves[nl + lanes_below(kA)] = (int)(entry << 1);
+            nl += __popcll(kA);
+            if (lfB) leaves[nl + lanes_below(kB)] = (int)(entry << 1 | 1u);
+            nl += __popcll(kB);
+            __syncthreads();
+        }
+        while (nl >= 64 || (size == 0 && nl > 0)) {
+            const int m = min(nl, 64);
+            nl -= m;
+            const bool has = lane < m;
+            const unsigned e = has ? (unsigned)leaves[nl + lane] : 0u;
+            const unsigned entry = e >> 1;
+            float4 lo = make_float4(0.f, 0.f, 0.f, 0.f), hi = lo;
+            if (has) {
+                const BvhPair& P = pairs[entry & kMask];
+                lo = e & 1u ? P.lo1 : P.lo0;
+                hi = e & 1u ? P.hi1 : P.hi0;
+            }
+            leaf(has, (int)(entry >> kBits), lo, hi);
+            __syncthreads();
         }
     }
-    if (RECORD) {
-        for (int k = recKeys; k < pairs; ++k) S.recKeys[keyBase + k] = make_int4(v, -1, -1, -1);
-        return;
+}
+
+
+// Contact queries, Q vertices or edges per wave. What a query collects is a set (minima, counts, the
+// CAP lowest ids), so the order in which its leaves are tested does not matter: exact tests of a
+// batch of leaves run one per lane and go to the query's minima and counts in LDS; contacts go to a
+// list in LDS, which the lanes that own the queries take in turn when it is nearly full and at the end.
+constexpr int kHits = 128;
+
+// VF query (ClothContactDetector.cpp:144-288 per candidate face). CAP bounds the owner's candidate
+// list (the runtime vfCap is at most CAP); only the face id and the packed (type, primitive) key are
+// kept per candidate, the distance is recomputed for the stored ones at the end.
+template <int Q, int CAP>
+__global__ __launch_bounds__(64) void vf_query_kernel(CDView S) {
+    if (S.gate && !*S.gate) return;
+    __shared__ int stack[kQueryStack], leaves[kLeafQueue];
+    __shared__ float4 qPos[Q];  // the vertex in w
+    __shared__ int qMesh[Q], qMin[Q], qPairs[Q];
+    __shared__ int hitQuery[kHits], hitKey[kHits], hitFace[kHits];
+    const int lane = threadIdx.x;
+    // vertices in Morton order: a wave's queries are spatial neighbours, and so are the blocks of one XCD
+    const int t = xcd_block_index() * Q + lane;
+    const bool own = lane < Q && t < S.nv;
+    const int v = !own ? -1 : (S.vOrder ? (int)(S.vOrder[t] & 0xFFFFFFFFu) : t);
+    const bool active = own && !(S.vQuery && !S.vQuery[v]);
+    if (own && !active) {  // not a surface vertex: no VF contacts
+        S.vfMin[v] = S.r;
+        S.vfPairCount[v] = 0;
+        S.vfStored[v] = 0;
+        S.vfOverflow[v] = 0;
     }
-    S.vfMin[v] = vmin;
-    S.vfPairCount[v] = pairs;
+    const float r = S.r;
+    const float rq = r * 1.0001f + 1e-7f;
+    V3 p = {0.f, 0.f, 0.f};
+    if (active) {
+        p = ld(S.pos, v);
+        qPos[lane] = make_float4(p.x, p.y, p.z, __int_as_float(v));
+        qMesh[lane] = S.vMesh[v];
+        qMin[lane] = __float_as_int(r);
+        qPairs[lane] = 0;
+    }
+    int stored = 0, overflow = 0;
+    int kKey[CAP], kFace[CAP];  // key: primitive | type << 30
+    // dedup on (type, primitive), keeping the lowest face id as the representative; the vfCap keys with
+    // the lowest representative faces stay
+    const auto insert = [&](int key, int f) {
+        bool dup = false;
+#pragma unroll
+        for (int k = 0; k < CAP; ++k)
+            if (k < stored && !dup && kKey[k] == key) {
+                if (f < kFace[k]) kFace[k] = f;
+                dup = true;
+            }
+        if (dup) return;
+        int slot = stored;
+        if (stored == S.vfCap) {
+            overflow = 1;
+            slot = 0;
+            int worst = kFace[0];
+#pragma unroll
+            for (int k = 1; k < CAP; ++k)
+                if (k < stored && kFace[k] > worst) {
+                    worst = kFace[k];
+                    slot = k;
+                }
+            if (f > worst) slot = -1;
+        } else {
+            ++stored;
+        }
+#pragma unroll
+        for (int k = 0; k < CAP; ++k)
+            if (k == slot) {
+                kKey[k] = key;
+                kFace[k] = f;
+            }
+    };
+    int hits = 0;
+    const auto flush = [&]() {
+        for (int j = 0; j < hits; ++j)
+            if (hitQuery[j] == lane) insert(hitKey[j], hitFace[j]);
+        hits = 0;
+        __syncthreads();
+    };
+    wave_queries<Q>(
+        S.fPairs, S.fN, active, stack, leaves, S.error,
+        [&](int q, float4 lo, float4 hi) {
+            const float4 c = qPos[q];
+            return c.x - rq <= hi.x && c.x + rq >= lo.x && c.y - rq <= hi.y && c.y + rq >= lo.y && c.z - rq <= hi.z &&
+                   c.z + rq >= lo.z;
+        },
+        [&](bool has, int q, float4 lo, float4) {
+            bool hit = false;
+            int f = 0, key = 0;
+            if (has) {
+                const float4 c = qPos[q];
+                const V3 x = {c.x, c.y, c.z};
+                const int u = __float_as_int(c.w);
+                f = __float_as_int(lo.w);
+                const int4 fv = S.faces[f];
+                if (!(fv.w == qMesh[q] && (fv.x == u || fv.y == u || fv.z == u))) {
+                    int type;
+                    const V3 cp = closest_point_triangle(x, ld(S.pos, fv.x), ld(S.pos, fv.y), ld(S.pos, fv.z), type);
+                    const float d = dist(x, cp);
+                    if (d < r) {
+                        atomicMin(&qMin[q], __float_as_int(d));
+                        atomicAdd(&qPairs[q], 1);
+                        atomicMin(S.faceMin + f, __float_as_int(d));
+                        int ptype;
+                        const int prim = closest_primitive(S, f, fv, type, ptype);
+                        hit = primitive_feasible(S, x, ptype, prim);
+                        key = prim | (ptype << 30);
+                    }
+                }
+            }
+            const unsigned long long found = __ballot(hit);
+            if (hit) {
+                const int at = hits + lanes_below(found);
+                hitQuery[at] = q;
+                hitKey[at] = key;
+                hitFace[at] = f;
+            }
+            hits += __popcll(found);
+            __syncthreads();
+            if (hits > kHits - 64) flush();
+        });
+    flush();
+    if (!active) return;
+    S.vfMin[v] = __int_as_float(qMin[lane]);
+    S.vfPairCount[v] = qPairs[lane];
     S.vfStored[v] = stored;
     S.vfOverflow[v] = overflow;
     // stored in ascending face id, whatever the traversal order (so the list, and the solver's sum
@@ -428,113 +680,100 @@ __global__ __launch_bounds__(256) void vf_query_kernel(CDView S) {
     }
 }
 
-// EE query of one edge (ClothContactDetector.cpp:731-813 per candidate edge, :1106-1135 setup)
-// CAP as for the VF query: only the other edge's id is kept per candidate; the closest points and
-// distance of the stored ones are recomputed at the end.
-template <bool RECORD, int CAP>
-__global__ __launch_bounds__(256) void ee_query_kernel(CDView S) {
-    // neighbouring threads take edges that are neighbours in the tree's Morton order, so a
-    // wavefront's traversals share their paths (and cache lines), and an XCD's blocks a range
+// EE query (ClothContactDetector.cpp:731-813 per candidate edge, :1106-1135 setup). Only the other
+// edge's id is kept per candidate; the closest points and distance of the stored ones are recomputed
+// at the end.
+template <int Q, int CAP>
+__global__ __launch_bounds__(64) void ee_query_kernel(CDView S) {
     if (S.gate && !*S.gate) return;
-    const int t = xcd_block_index() * blockDim.x + threadIdx.x;
-    if (t >= S.ne) return;
-    const int e1 = S.eOrder ? (int)(S.eOrder[t] & 0xFFFFFFFFu) : t;
-    const int4 a = S.edges[e1];
-    const int m1 = S.eMesh[e1];
-    const V3 p1 = ld(S.pos, a.x), p2 = ld(S.pos, a.y);
+    __shared__ int stack[kQueryStack], leaves[kLeafQueue];
+    __shared__ float4 qLo[Q], qHi[Q], qP1[Q], qP2[Q];  // qP1.w the edge, qP2.w its mesh
+    __shared__ int qMin[Q], qCount[Q];
+    __shared__ int hitQuery[kHits], hitEdge[kHits];
+    const int lane = threadIdx.x;
+    // neighbouring lanes take edges that are neighbours in the tree's Morton order, and an XCD's blocks a range
+    const int t = xcd_block_index() * Q + lane;
+    const bool active = lane < Q && t < S.ne;
+    const int e1 = !active ? -1 : (S.eOrder ? (int)(S.eOrder[t] & 0xFFFFFFFFu) : t);
     const float r = S.r;
     // Every edge within r of this one overlaps the segment's box grown by r: a tighter region
     // than the box of the reference's sphere (midpoint, r + len / 2), with the same contacts and
     // minimum distances (both are decided by the exact tests below).
     const float rq = r * 1.0001f + 1e-7f;
-    const V3 qlo = {fminf(p1.x, p2.x) - rq, fminf(p1.y, p2.y) - rq, fminf(p1.z, p2.z) - rq};
-    const V3 qhi = {fmaxf(p1.x, p2.x) + rq, fmaxf(p1.y, p2.y) + rq, fmaxf(p1.z, p2.z) + rq};
-    float emin = r;
-    int count = 0, stored = 0, overflow = 0;
-    int cE[CAP];
-    const int64_t base = RECORD ? S.eeOffset[e1] : 0;
-    const int countCap = RECORD ? S.eeCount[e1] : 0;
-    const int firstLeaf = S.eN - 1;
-    const V3 ev1 = p2 - p1;
-    int node = S.eN > 0 ? 0 : -1;
-    for (int visits = 0; node >= 0; ++visits) {
-        if (visits > 2 * S.eN) {
-            atomicOr(S.error, 1);
-            break;
-        }
-        const BvhNode nd = S.eNodes[node];
-        const int skip = __float_as_int(nd.hi.w);
-        if (!box_overlap(qlo, qhi, nd)) {
-            node = skip;
-            continue;
-        }
-        if (node < firstLeaf) {
-            node = __float_as_int(nd.lo.w);
-            continue;
-        }
-        node = skip;
-        // the other edge's endpoints from its leaf (the positions of the last refit, which are
-        // the query's): no edge or position loads for the many leaves beyond r
-        const int tag = __float_as_int(nd.lo.w);
-        const int e2 = tag & kLeafPrimMask;
-        const V3 q1 = {(tag >> kLeafPrimBits) & 1 ? nd.hi.x : nd.lo.x, (tag >> (kLeafPrimBits + 1)) & 1 ? nd.hi.y : nd.lo.y,
-                       (tag >> (kLeafPrimBits + 2)) & 1 ? nd.hi.z : nd.lo.z};
-        const V3 q2 = {(tag >> kLeafPrimBits) & 1 ? nd.lo.x : nd.hi.x, (tag >> (kLeafPrimBits + 1)) & 1 ? nd.lo.y : nd.hi.y,
-                       (tag >> (kLeafPrimBits + 2)) & 1 ? nd.lo.z : nd.hi.z};
-        V3 c1, c2;
-        float mua, mub;
-        segment_closest_points(p1, p2, q1, q2, c1, c2, mua, mub);
-        const float d = dist(c1, c2);
-        // emin starts at r, so an edge at d >= r (or NaN) leaves it unchanged whether or not the
-        // topology filter below would have skipped it
-        if (!(d < r)) continue;
-        if (S.eMesh[e2] == m1) {
-            if (e2 == e1) continue;
-            const int4 b = S.edges[e2];
-            if (a.x == b.x || a.x == b.y || a.y == b.x || a.y == b.y) continue;
-        }
-        emin = fminf(d, emin);
-        const V3 ev2 = q2 - q1;
-        bool ok = false;
-        if (dot(c2 - p1, ev1) >= 0.f && dot(p2 - c2, ev1) >= 0.f)
-            ok = true;
-        else if (dot(c1 - q1, ev2) >= 0.f && dot(q2 - c1, ev2) >= 0.f)
-            ok = true;
-        if (!ok) continue;
-        if (RECORD) {
-            if (count >= countCap) {
-                atomicOr(S.error, 4);
-                break;
-            }
-            S.recEE[base + count] = make_int2(e1, e2);
-            S.recEEmu[base + count] = make_float2(mua, mub);
-            S.recEEd[base + count] = d;
-        } else {
-            // keep the eeCap contacts with the lowest other-edge ids (order-free selection)
-            int slot = stored;
-            if (stored == S.eeCap) {
-                overflow = 1;
-                slot = 0;
-                int worst = cE[0];
-#pragma unroll
-                for (int k = 1; k < CAP; ++k)
-                    if (k < stored && cE[k] > worst) {
-                        worst = cE[k];
-                        slot = k;
-                    }
-                if (e2 > worst) slot = -1;
-            } else {
-                ++stored;
-            }
-#pragma unroll
-            for (int k = 0; k < CAP; ++k)
-                if (k == slot) cE[k] = e2;
-        }
-        ++count;
+    V3 p1 = {0.f, 0.f, 0.f}, p2 = p1;
+    if (active) {
+        const int4 a = S.edges[e1];
+        p1 = ld(S.pos, a.x);
+        p2 = ld(S.pos, a.y);
+        qLo[lane] = make_float4(fminf(p1.x, p2.x) - rq, fminf(p1.y, p2.y) - rq, fminf(p1.z, p2.z) - rq, 0.f);
+        qHi[lane] = make_float4(fmaxf(p1.x, p2.x) + rq, fmaxf(p1.y, p2.y) + rq, fmaxf(p1.z, p2.z) + rq, 0.f);
+        qP1[lane] = make_float4(p1.x, p1.y, p1.z, __int_as_float(e1));
+        qP2[lane] = make_float4(p2.x, p2.y, p2.z, __int_as_float(S.eMesh[e1]));
+        qMin[lane] = __float_as_int(r);
+        qCount[lane] = 0;
     }
-    if (RECORD) return;
-    S.eeMin[e1] = emin;
-    S.eeCount[e1] = count;
+    int stored = 0, overflow = 0;
+    int cE[CAP];
+    // the eeCap contacts with the lowest other-edge ids stay
+    const auto insert = [&](int e2) {
+        int slot = stored;
+        if (stored == S.eeCap) {
+            overflow = 1;
+            slot = 0;
+            int worst = cE[0];
+#pragma unroll
+            for (int k = 1; k < CAP; ++k)
+                if (k < stored && cE[k] > worst) {
+                    worst = cE[k];
+                    slot = k;
+                }
+            if (e2 > worst) slot = -1;
+        } else {
+            ++stored;
+        }
+#pragma unroll
+        for (int k = 0; k < CAP; ++k)
+            if (k == slot) cE[k] = e2;
+    };
+    int hits = 0;
+    const auto flush = [&]() {
+        for (int j = 0; j < hits; ++j)
+            if (hitQuery[j] == lane) insert(hitEdge[j]);
+        hits = 0;
+        __syncthreads();
+    };
+    wave_queries<Q>(
+        S.ePairs, S.eN, active, stack, leaves, S.error,
+        [&](int q, float4 lo, float4 hi) {
+            const float4 ql = qLo[q], qh = qHi[q];
+            return ql.x <= hi.x && qh.x >= lo.x && ql.y <= hi.y && qh.y >= lo.y && ql.z <= hi.z && qh.z >= lo.z;
+        },
+        [&](bool has, int q, float4 lo, float4 hi) {
+            bool hit = false;
+            EdgePair e{};
+            if (has) {
+                const float4 a = qP1[q], b = qP2[q];
+                const int id = __float_as_int(a.w);
+                if (edge_pair(S, id, __float_as_int(b.w), V3{a.x, a.y, a.z}, V3{b.x, b.y, b.z}, lo, hi, e)) {
+                    atomicMin(&qMin[q], __float_as_int(e.d));
+                    hit = e.contact;
+                    if (hit) atomicAdd(&qCount[q], 1);
+                }
+            }
+            const unsigned long long found = __ballot(hit);
+            if (hit) {
+                const int at = hits + lanes_below(found);
+                hitQuery[at] = q;
+                hitEdge[at] = e.e2;
+            }
+            hits += __popcll(found);
+            __syncthreads();
+            if (hits > kHits - 64) flush();
+        });
+    flush();
+    if (!active) return;
+    S.eeMin[e1] = __int_as_float(qMin[lane]);
+    S.eeCount[e1] = qCount[lane];
     S.eeStored[e1] = stored;
     S.eeOverflow[e1] = overflow;
     // stored in ascending other-edge id (independent of the traversal order)
@@ -781,7 +1020,8 @@ __global__ __launch_bounds__(256) void level_nodes_kernel(const uint64_t* keys, 
     if (i == 0 || (int)(keys[i - 1] >> 32) != (int)(keys[i] >> 32)) starts[dk] = i;
 }
 
-__global__ __launch_bounds__(256) void leaf_box_kernel(CDView S, int kind, BvhNode* nodes, int n) {
+__global__ __launch_bounds__(256) void leaf_box_kernel(CDView S, int kind, BvhNode* nodes, BvhPair* pairs,
+                                                       int n) {
     if (S.gate && !*S.gate) return;
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
@@ -810,19 +1050,34 @@ __global__ __launch_bounds__(256) void leaf_box_kernel(CDView S, int kind, BvhNo
     }
     L.lo = make_float4(lo.x, lo.y, lo.z, __int_as_float(tag));
     L.hi = make_float4(hi.x, hi.y, hi.z, L.hi.w);
+    // a tree of one primitive has no internal node: its pair holds the leaf and an empty box
+    if (n == 1 && pairs)
+        pairs[0] = BvhPair{L.lo, make_float4(hi.x, hi.y, hi.z, __int_as_float(1)),
+                           make_float4(FLT_MAX, FLT_MAX, FLT_MAX, 0.f), make_float4(-FLT_MAX, -FLT_MAX, -FLT_MAX, 0.f)};
 }
 
-__global__ __launch_bounds__(256) void internal_box_kernel(const int* levelNodes, int begin, int end,
-                                                           BvhNode* nodes, const int* rightChild, const int* gate) {
-    if (gate && !*gate) return;
-    const int k = begin + blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= end) return;
-    const int i = levelNodes[k];
+// Box of internal node i from its children's, and (trees with wave queries) the children side by side.
+__device__ __forceinline__ void merge_children(BvhNode* nodes, const int* rightChild, BvhPair* pairs, int firstLeaf,
+                                               int i) {
     BvhNode& N = nodes[i];
-    const BvhNode A = nodes[__float_as_int(N.lo.w)];
-    const BvhNode B = nodes[rightChild[i]];
+    const int a = __float_as_int(N.lo.w), b = rightChild[i];
+    const BvhNode A = nodes[a], B = nodes[b];
     N.lo = make_float4(fminf(A.lo.x, B.lo.x), fminf(A.lo.y, B.lo.y), fminf(A.lo.z, B.lo.z), N.lo.w);
     N.hi = make_float4(fmaxf(A.hi.x, B.hi.x), fmaxf(A.hi.y, B.hi.y), fmaxf(A.hi.z, B.hi.z), N.hi.w);
+    if (!pairs) return;
+    const bool la = a >= firstLeaf, lb = b >= firstLeaf;
+    pairs[i] = BvhPair{make_float4(A.lo.x, A.lo.y, A.lo.z, la ? A.lo.w : __int_as_float(a)),
+                       make_float4(A.hi.x, A.hi.y, A.hi.z, __int_as_float(la ? 1 : 0)),
+                       make_float4(B.lo.x, B.lo.y, B.lo.z, lb ? B.lo.w : __int_as_float(b)),
+                       make_float4(B.hi.x, B.hi.y, B.hi.z, __int_as_float(lb ? 1 : 0))};
+}
+
+__global__ __launch_bounds__(256) void internal_box_kernel(const int* levelNodes, int begin, int end, BvhNode* nodes,
+                                                           const int* rightChild, BvhPair* pairs, int firstLeaf,
+                                                           const int* gate) {
+    if (gate && !*gate) return;
+    const int k = begin + blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < end) merge_children(nodes, rightChild, pairs, firstLeaf, levelNodes[k]);
 }
 
 // Several consecutive refit levels of few nodes each in one block: the levels run in order with a
@@ -830,18 +1085,13 @@ __global__ __launch_bounds__(256) void internal_box_kernel(const int* levelNodes
 // before the segment were finished by earlier launches).
 __global__ __launch_bounds__(1024) void internal_box_levels_kernel(const int* levelNodes, const int* levelBegin,
                                                                    int l0, int l1, BvhNode* nodes,
-                                                                   const int* rightChild, const int* gate) {
+                                                                   const int* rightChild, BvhPair* pairs,
+                                                                   int firstLeaf, const int* gate) {
     if (gate && !*gate) return;  // uniform over the block: no barrier is left waiting
     for (int l = l0; l < l1; ++l) {
         const int b = levelBegin[l], e = levelBegin[l + 1];
-        for (int k = b + (int)threadIdx.x; k < e; k += (int)blockDim.x) {
-            const int i = levelNodes[k];
-            BvhNode& N = nodes[i];
-            const BvhNode A = nodes[__float_as_int(N.lo.w)];
-            const BvhNode B = nodes[rightChild[i]];
-            N.lo = make_float4(fminf(A.lo.x, B.lo.x), fminf(A.lo.y, B.lo.y), fminf(A.lo.z, B.lo.z), N.lo.w);
-            N.hi = make_float4(fmaxf(A.hi.x, B.hi.x), fmaxf(A.hi.y, B.hi.y), fmaxf(A.hi.z, B.hi.z), N.hi.w);
-        }
+        for (int k = b + (int)threadIdx.x; k < e; k += (int)blockDim.x)
+            merge_children(nodes, rightChild, pairs, firstLeaf, levelNodes[k]);
         __syncthreads();
     }
 }
@@ -1282,14 +1532,7 @@ __device__ __forceinline__ float box_far2(V3 p, const BvhNode& n) {
     return dx * dx + dy * dy + dz * dz;
 }
 
-// ---- traversal of a tree by a whole wave ----
-// The nodes to visit lie on a stack in LDS; a step pops up to 64 of them, one per lane, and pushes
-// the children of those that are not pruned. The stack stays sorted by depth, so that it holds little
-// more than 64 nodes per level; when it runs full a step pops fewer, down to one (depth first), which
-// needs at most one entry per level, the reserve. kWaveStack entries are enough for any tree of the
-// refit schedule's depth.
 constexpr int kWaveStack = 1024;
-constexpr int kWaveReserve = kMaxDepth + 2;
 
 // Visits the nodes of a tree of n leaves, each step up to 64 side by side: keep(node, leaf, data) says
 // whether a node is of interest and handles it if it is a leaf; step() is called by every lane after
@@ -1303,7 +1546,7 @@ __device__ __forceinline__ void wave_traverse(const BvhNode* nodes, const int* r
     if (lane == 0) stack[0] = 0;
     __syncthreads();
     while (size > 0) {
-        const int m = min(min(64, size), max(kWaveStack - kWaveReserve - size, 1));
+        const int m = wave_pop(size, kWaveStack);
         const int base = size - m;
         const int node = lane < m ? stack[base + lane] : -1;
         __syncthreads();
@@ -1321,7 +1564,7 @@ __device__ __forceinline__ void wave_traverse(const BvhNode* nodes, const int* r
             break;
         }
         if (left >= 0) {
-            const int at = base + 2 * __popcll(grow & ((1ull << lane) - 1ull));
+            const int at = base + 2 * lanes_below(grow);
             stack[at] = rgt;
             stack[at + 1] = left;
         }
@@ -1951,8 +2194,8 @@ void ContactDetector::finalize() {
         vSortTemp_ = dalloc<char>(vSortTempBytes_);
     }
     // BVH storage
-    allocBvh(fb_, nf_);
-    allocBvh(eb_, ne_);
+    allocBvh(fb_, nf_, !pen_);
+    allocBvh(eb_, ne_, !pen_);
     if (pen_ && nf_ > 0) fb_.mesh = dalloc<int>(2 * (size_t)nf_ - 1);
     if (pen_) setupPenetrationDevice();
     hip_check(hipStreamSynchronize(stream_), "detector upload sync");
@@ -1969,11 +2212,12 @@ void ContactDetector::finalize() {
     }
 }
 
-void ContactDetector::allocBvh(DeviceBvh& B, int n) {
+void ContactDetector::allocBvh(DeviceBvh& B, int n, bool pairs) {
     if (n > kLeafPrimMask) fail(GVBD_ERR_INVALID, "a tree of " + std::to_string(n) + " primitives exceeds 2^28 - 1");
     B.n = n;
     if (B.n == 0) return;
     B.nodes = dalloc<BvhNode>(2 * (size_t)B.n - 1);
+    if (pairs) B.pairs = dalloc<BvhPair>(std::max(B.n - 1, 1));
     B.parent = dalloc<int>(2 * (size_t)B.n - 1);
     B.right = dalloc<int>(std::max(B.n - 1, 1));
     B.jump = dalloc<int>(4 * (size_t)std::max(B.n - 1, 1));
@@ -2105,15 +2349,15 @@ void ContactDetector::refitBvh(DeviceBvh& B, int kind, hipStream_t stream, const
     S.edges = edges_;
     S.boxes = boxes;
     S.gate = gate;
-    hipLaunchKernelGGL(leaf_box_kernel, dim3(blocks_for(B.n)), dim3(256), 0, stream, S, kind, B.nodes, B.n);
+    hipLaunchKernelGGL(leaf_box_kernel, dim3(blocks_for(B.n)), dim3(256), 0, stream, S, kind, B.nodes, B.pairs, B.n);
     for (const auto& seg : B.segments) {
         const int b = B.levelBegin[seg.first], e = B.levelBegin[seg.first + 1];
         if (seg.second == seg.first + 1 && e - b > kBlockLevel)
             hipLaunchKernelGGL(internal_box_kernel, dim3(blocks_for(e - b)), dim3(256), 0, stream, B.levelNodes, b,
-                               e, B.nodes, B.right, gate);
+                               e, B.nodes, B.right, B.pairs, B.n - 1, gate);
         else
             hipLaunchKernelGGL(internal_box_levels_kernel, dim3(1), dim3(kBlockLevel), 0, stream, B.levelNodes,
-                               B.dLevelBegin, seg.first, seg.second, B.nodes, B.right, gate);
+                               B.dLevelBegin, seg.first, seg.second, B.nodes, B.right, B.pairs, B.n - 1, gate);
     }
     hip_check(hipGetLastError(), "bvh refit launch");
 }
@@ -2164,8 +2408,8 @@ void ContactDetector::setupPenetrationDevice() {
     hipLaunchKernelGGL(fill_u8_kernel, dim3(std::min(blocks_for(nv_), 4096)), dim3(256), 0, stream_, penFlags_,
                        (int64_t)nv_);
     hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(256), 0, stream_, penCounts_, (int64_t)kPenCounts, 0);
-    allocBvh(tb_, nt_);
-    allocBvh(sb_, nf_);
+    allocBvh(tb_, nt_, false);
+    allocBvh(sb_, nf_, false);
     // tet boxes for the first tree build (at the end of finalize)
     hipLaunchKernelGGL(tet_box_kernel, dim3(blocks_for(nt_)), dim3(256), 0, stream_, pos_, penTets_, nt_, tetBoxes_);
     hip_check(hipGetLastError(), "penetration setup launch");
@@ -2335,6 +2579,50 @@ void ContactDetector::perturb(uint64_t seed, int step, float sigma, const float*
     treeCurrent_ = false;
 }
 
+namespace {
+template <int Q> void launch_vf(const CDView& S, hipStream_t stream) {
+    const dim3 grid((S.nv + Q - 1) / Q);
+    if (S.vfCap <= 8)
+        hipLaunchKernelGGL((vf_query_kernel<Q, 8>), grid, dim3(64), 0, stream, S);
+    else
+        hipLaunchKernelGGL((vf_query_kernel<Q, kMaxCap>), grid, dim3(64), 0, stream, S);
+}
+template <int Q> void launch_ee(const CDView& S, hipStream_t stream) {
+    if (S.ne == 0) return;
+    const dim3 grid((S.ne + Q - 1) / Q);
+    if (S.eeCap <= 8)
+        hipLaunchKernelGGL((ee_query_kernel<Q, 8>), grid, dim3(64), 0, stream, S);
+    else
+        hipLaunchKernelGGL((ee_query_kernel<Q, kMaxCap>), grid, dim3(64), 0, stream, S);
+}
+
+// Queries per wave: few where there are few (more waves, each with a shorter path), more where the
+// waves fill the chip anyway (less of a wave's time goes to its start at the root and its end, with
+// lanes idle). Measured, VF and EE queries together, tori of 8,192 vertices and 24,576 edges, us per
+// pass with 8 / 16 / 32 / 64 queries per wave (one thread per query before: 201, 246, 322, 663, 1472):
+// 8k vertices 63 / 71 / 92 / 121, 36k 123 / 110 / 113 / 148, 65k 233 / 191 / 195 / 208,
+// 221k 702 / 512 / 478 / 500, 524k 1818 / 1285 / 1140 / 1166. A query's bits and a node's share a
+// stack entry, which limits the tree (see wave_queries); 8 take any tree.
+int queries_per_wave(int queries, int prims) {
+    if (queries > 262144 && prims <= (1 << query_node_bits<32>())) return 32;
+    if (queries > 49152 && prims <= (1 << query_node_bits<16>())) return 16;
+    return 8;
+}
+
+void launch_queries(const CDView& S, hipStream_t vfStream, hipStream_t eeStream) {
+    switch (queries_per_wave(S.nv, S.fN)) {
+    case 32: launch_vf<32>(S, vfStream); break;
+    case 16: launch_vf<16>(S, vfStream); break;
+    default: launch_vf<8>(S, vfStream); break;
+    }
+    switch (queries_per_wave(S.ne, S.eN)) {
+    case 32: launch_ee<32>(S, eeStream); break;
+    case 16: launch_ee<16>(S, eeStream); break;
+    default: launch_ee<8>(S, eeStream); break;
+    }
+}
+}  // namespace
+
 void ContactDetector::query(bool record, const int* gate) {
     if (!ready_) fail(GVBD_ERR_STATE, "detector not finalized");
     // the EE query reads the other edge's endpoints from the tree's leaves
@@ -2351,8 +2639,10 @@ void ContactDetector::query(bool record, const int* gate) {
     S.vvBegin = vvBegin_;
     S.vvNei = vvNei_;
     S.fNodes = fb_.nodes;
+    S.fPairs = fb_.pairs;
     S.fN = fb_.n;
     S.eNodes = eb_.nodes;
+    S.ePairs = eb_.pairs;
     S.eN = eb_.n;
     S.eOrder = eb_.n > 0 ? eb_.keysAlt : nullptr;
     S.vOrder = fb_.n > 0 ? vKeysAlt_ : nullptr;  // computed with the face tree
@@ -2377,14 +2667,7 @@ void ContactDetector::query(bool record, const int* gate) {
     hipLaunchKernelGGL(gated_fill_int_kernel, dim3(std::min(blocks_for(nf_), 4096)), dim3(256), 0, stream_, faceMin_,
                        (int64_t)nf_, rbits, gate);
     fork();
-    if (vfCap_ <= 8)
-        hipLaunchKernelGGL((vf_query_kernel<false, 8>), dim3(blocks_for(nv_)), dim3(256), 0, stream_, S);
-    else
-        hipLaunchKernelGGL((vf_query_kernel<false, kMaxCap>), dim3(blocks_for(nv_)), dim3(256), 0, stream_, S);
-    if (eeCap_ <= 8)
-        hipLaunchKernelGGL((ee_query_kernel<false, 8>), dim3(blocks_for(ne_)), dim3(256), 0, side_, S);
-    else
-        hipLaunchKernelGGL((ee_query_kernel<false, kMaxCap>), dim3(blocks_for(ne_)), dim3(256), 0, side_, S);
+    launch_queries(S, stream_, side_);
     join();
     hip_check(hipGetLastError(), "query launch");
     recorded_ = false;
@@ -2423,8 +2706,8 @@ void ContactDetector::query(bool record, const int* gate) {
     S.recEE = recEE_;
     S.recEEmu = recEEmu_;
     S.recEEd = recEEd_;
-    hipLaunchKernelGGL((vf_query_kernel<true, 1>), dim3(blocks_for(nv_)), dim3(256), 0, stream_, S);
-    hipLaunchKernelGGL((ee_query_kernel<true, 1>), dim3(blocks_for(ne_)), dim3(256), 0, stream_, S);
+    hipLaunchKernelGGL(vf_record_kernel, dim3(blocks_for(nv_)), dim3(256), 0, stream_, S);
+    hipLaunchKernelGGL(ee_record_kernel, dim3(blocks_for(ne_)), dim3(256), 0, stream_, S);
     hip_check(hipGetLastError(), "record query launch");
     hip_check(hipStreamSynchronize(stream_), "record query sync");
     recorded_ = true;
