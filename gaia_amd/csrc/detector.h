@@ -50,20 +50,22 @@ struct DeviceBvh {
     BvhPair* pairs = nullptr;        // n - 1 (1 for a single primitive): set at every refit
     int* parent = nullptr;           // 2n - 1
     int* right = nullptr;            // n - 1: right child of each internal node (refit)
-    int* jump = nullptr;             // 4 (n - 1): depth / ancestor buffers of the depth computation
     int* levelNodes = nullptr;       // internal nodes ordered by depth, deepest first
     std::vector<int> levelBegin;     // host: ranges of levelNodes per depth (deepest first)
     int* dLevelBegin = nullptr;      // the same ranges on the device
     std::vector<std::pair<int, int>> segments;  // refit launches: [first, last) level runs
-    uint64_t* keys = nullptr;        // n (sorted Morton keys)
-    uint64_t* keysAlt = nullptr;     // n
-    uint64_t* depthKeys = nullptr;   // n - 1
-    uint64_t* depthKeysAlt = nullptr;
-    int* depth = nullptr;            // n - 1
-    void* sortTemp = nullptr;
-    size_t sortTempBytes = 0;
+    uint64_t* keysAlt = nullptr;     // n (sorted Morton keys)
     int* mesh = nullptr;             // 2n - 1 (face trees of penetration contact): the mesh of every
                                      // face below the node, -1 where faces of several meshes meet
+};
+
+// Buffers of the tree builds (one set per detector).
+struct BvhScratch {
+    int* jump = nullptr;  // 4 (n - 1): depth / ancestor buffers of the depth computation
+    uint64_t *keys = nullptr, *depthKeys = nullptr, *depthKeysAlt = nullptr;
+    int* depth = nullptr;
+    void* sortTemp = nullptr;
+    size_t sortTempBytes = 0;
 };
 
 // Penetration contact of tet meshes (the reference tet solver's DCD and CCD,
@@ -199,9 +201,10 @@ class ContactDetector {
     hipStream_t stream() const { return stream_; }
 
   private:
-    // kind 0 faces, 1 edges, 3 precomputed primitive boxes (`boxes`: lo, hi per primitive)
-    void buildBvh(DeviceBvh& b, int kind, const float4* boxes = nullptr);
-    void refitBvh(DeviceBvh& b, int kind, hipStream_t stream, const float4* boxes = nullptr,
+    // kind 0 faces, 1 edges, 3 tets, 4 faces over their path from `prev`
+    void allocBuildScratch(const std::vector<int>& sizes);
+    void buildBvh(DeviceBvh& b, int kind, const float4* prev = nullptr);
+    void refitBvh(DeviceBvh& b, int kind, hipStream_t stream, const float4* prev = nullptr,
                   const int* gate = nullptr);
     void allocBvh(DeviceBvh& b, int n, bool pairs);
     void setupPenetrationDevice();
@@ -286,7 +289,7 @@ class ContactDetector {
     int4 *penTets_ = nullptr, *penTetNbr_ = nullptr, *penFaceNbr_ = nullptr;
     int *penTetMesh_ = nullptr, *penVNbrBegin_ = nullptr, *penVNbr_ = nullptr, *penSurf_ = nullptr;
     int2* penFaceOwner_ = nullptr;
-    float4 *tetBoxes_ = nullptr, *sweptBoxes_ = nullptr;
+    BvhScratch scratch_;
     uint8_t* penFlags_ = nullptr;
     int* penCounts_ = nullptr;  // kPenCounts: DCD hits, penetrated without a face, CCD hits, walk
                                 // overflows, contained vertices listed by the DCD's first pass

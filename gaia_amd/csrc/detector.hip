@@ -219,7 +219,8 @@ struct CDView {
     const uint8_t* vQuery;   // per vertex: takes VF queries (NULL: every vertex)
     const int* gate;         // device flag: 0 skips the pass's kernels (NULL: always run)
     int* error;
-    const float4* boxes;     // kind 3 primitives: lo, hi per primitive
+    const int4* tets;        // kind 3 primitives
+    const float4* prev;      // kind 4 primitives (faces over their path from prev to pos)
 };
 
 __device__ __forceinline__ bool box_overlap(V3 qlo, V3 qhi, const BvhNode& n) {
@@ -823,6 +824,28 @@ __device__ __forceinline__ float unorder_bits(unsigned int u) {
     return __uint_as_float((u & 0x80000000u) ? (u & 0x7FFFFFFFu) : ~u);
 }
 
+__device__ __forceinline__ void tet_box(const CDView& S, int t, V3& lo, V3& hi) {
+    const int4 tv = S.tets[t];
+    const V3 a = ld(S.pos, tv.x), b = ld(S.pos, tv.y), c = ld(S.pos, tv.z), d = ld(S.pos, tv.w);
+    lo = {fminf(fminf(a.x, b.x), fminf(c.x, d.x)), fminf(fminf(a.y, b.y), fminf(c.y, d.y)),
+          fminf(fminf(a.z, b.z), fminf(c.z, d.z))};
+    hi = {fmaxf(fmaxf(a.x, b.x), fmaxf(c.x, d.x)), fmaxf(fmaxf(a.y, b.y), fmaxf(c.y, d.y)),
+          fmaxf(fmaxf(a.z, b.z), fmaxf(c.z, d.z))};
+}
+
+// box of a face over its path from prev to pos (movingFaceBoundsFunc, ContinuousCollisionDetector.cpp:19-65)
+__device__ __forceinline__ void swept_box(const CDView& S, int f, V3& lo, V3& hi) {
+    const int4 fv = S.faces[f];
+    const V3 q[6] = {ld(S.pos, fv.x),  ld(S.pos, fv.y),  ld(S.pos, fv.z),
+                     ld(S.prev, fv.x), ld(S.prev, fv.y), ld(S.prev, fv.z)};
+    lo = hi = q[0];
+#pragma unroll
+    for (int k = 1; k < 6; ++k) {
+        lo = {fminf(lo.x, q[k].x), fminf(lo.y, q[k].y), fminf(lo.z, q[k].z)};
+        hi = {fmaxf(hi.x, q[k].x), fmaxf(hi.y, q[k].y), fmaxf(hi.z, q[k].z)};
+    }
+}
+
 __device__ __forceinline__ V3 prim_centroid(const CDView& S, int kind, int i) {
     if (kind == 0) {
         const int4 f = S.faces[i];
@@ -834,8 +857,14 @@ __device__ __forceinline__ V3 prim_centroid(const CDView& S, int kind, int i) {
         return 0.5f * (ld(S.pos, e.x) + ld(S.pos, e.y));
     }
     if (kind == 3) {
-        const float4 lo = S.boxes[2 * i], hi = S.boxes[2 * i + 1];
-        return 0.5f * (V3{lo.x, lo.y, lo.z} + V3{hi.x, hi.y, hi.z});
+        V3 lo, hi;
+        tet_box(S, i, lo, hi);
+        return 0.5f * (lo + hi);
+    }
+    if (kind == 4) {
+        V3 lo, hi;
+        swept_box(S, i, lo, hi);
+        return 0.5f * (lo + hi);
     }
     return ld(S.pos, i);  // kind 2: vertices
 }
@@ -1030,9 +1059,9 @@ __global__ __launch_bounds__(256) void leaf_box_kernel(CDView S, int kind, BvhNo
     int tag = prim;
     V3 lo, hi;
     if (kind == 3) {
-        const float4 a = S.boxes[2 * prim], b = S.boxes[2 * prim + 1];
-        lo = {a.x, a.y, a.z};
-        hi = {b.x, b.y, b.z};
+        tet_box(S, prim, lo, hi);
+    } else if (kind == 4) {
+        swept_box(S, prim, lo, hi);
     } else if (kind == 0) {
         const int4 f = S.faces[prim];
         const V3 a = ld(S.pos, f.x), b = ld(S.pos, f.y), c = ld(S.pos, f.z);
@@ -1262,13 +1291,13 @@ struct PenView {
     const int* surfVerts;
     int nSurf;
     const int* vMesh;
-    const BvhNode* tNodes;   // tet tree
+    const BvhPair* tPairs;   // tet tree
     int tN;
     const BvhNode* fNodes;   // face tree (current positions)
     const int* fRight;       // right child of every internal face-tree node
     const int* fMesh;        // per face-tree node: the mesh of its faces, -1 for several
     int fN;
-    const BvhNode* sNodes;   // swept-face tree (prev and current positions)
+    const BvhPair* sPairs;   // swept-face tree (prev and current positions)
     int sN;
     PenetrationParams P;
     int* stored;             // per vertex: 1 with a hit face (the VF record slot's count)
@@ -1452,49 +1481,50 @@ __device__ __forceinline__ float box_dist2(V3 p, const BvhNode& n) {
     return dx * dx + dy * dy + dz * dz;
 }
 
-// DCD pass 1, one thread per surface vertex: the lowest tet containing the vertex (of any mesh;
-// of its own mesh only with self collision, and no tet of its own). Contained vertices are
-// listed for pass 2, so that its waves hold only vertices with a closest-face search to do.
+// DCD pass 1, Q surface vertices per wave: the lowest tet containing each vertex (of any mesh; of its
+// own mesh only with self collision, and no tet of its own). Contained vertices are listed for
+// pass 2, so that its waves hold only vertices with a closest-face search to do.
+template <int Q>
 __global__ __launch_bounds__(64) void pen_contain_kernel(PenView S) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= S.nSurf) return;
-    const int v = S.surfVerts[i];
-    S.stored[v] = 0;
-    S.flags[v] = 0;
-    const V3 p = ld(S.pos, v);
-    if (!S.P.dcd || !(p.y < S.P.offHeight)) return;
-    const int qm = S.vMesh[v];
-    int ht = -1;
-    const int firstLeaf = S.tN - 1;
-    int node = S.tN > 0 ? 0 : -1;
-    for (int visits = 0; node >= 0; ++visits) {
-        if (visits > 2 * S.tN) {
-            atomicOr(S.error, 1);
-            break;
-        }
-        const BvhNode nd = S.tNodes[node];
-        const int skip = __float_as_int(nd.hi.w);
-        if (!(p.x >= nd.lo.x && p.x <= nd.hi.x && p.y >= nd.lo.y && p.y <= nd.hi.y && p.z >= nd.lo.z &&
-              p.z <= nd.hi.z)) {
-            node = skip;
-            continue;
-        }
-        if (node < firstLeaf) {
-            node = __float_as_int(nd.lo.w);
-            continue;
-        }
-        node = skip;
-        const int t = __float_as_int(nd.lo.w);
-        if (ht >= 0 && t > ht) continue;
-        const int m = S.tetMesh[t];
-        if (m == qm && !S.P.self) continue;
-        const int4 tv = S.tets[t];
-        if (m == qm && (tv.x == v || tv.y == v || tv.z == v || tv.w == v)) continue;
-        if (point_in_tet(p, ld(S.pos, tv.x), ld(S.pos, tv.y), ld(S.pos, tv.z), ld(S.pos, tv.w))) ht = t;
+    __shared__ int stack[kQueryStack], leaves[kLeafQueue];
+    __shared__ float4 qPos[Q];  // the vertex in w
+    __shared__ int qMesh[Q], qTet[Q];
+    const int lane = threadIdx.x;
+    const int i = blockIdx.x * Q + lane;
+    const bool own = lane < Q && i < S.nSurf;
+    const int v = own ? S.surfVerts[i] : -1;
+    bool active = false;
+    if (own) {
+        S.stored[v] = 0;
+        S.flags[v] = 0;
+        const V3 p = ld(S.pos, v);
+        active = S.P.dcd && p.y < S.P.offHeight;
+        qPos[lane] = make_float4(p.x, p.y, p.z, __int_as_float(v));
+        qMesh[lane] = S.vMesh[v];
+        qTet[lane] = INT_MAX;
     }
-    if (ht < 0) return;
+    wave_queries<Q>(
+        S.tPairs, S.tN, active, stack, leaves, S.error,
+        [&](int q, float4 lo, float4 hi) {
+            const float4 p = qPos[q];
+            return p.x >= lo.x && p.x <= hi.x && p.y >= lo.y && p.y <= hi.y && p.z >= lo.z && p.z <= hi.z;
+        },
+        [&](bool has, int q, float4 lo, float4) {
+            if (!has) return;
+            const int t = __float_as_int(lo.w);
+            if (t > qTet[q]) return;
+            const int m = S.tetMesh[t], qm = qMesh[q];
+            if (m == qm && !S.P.self) return;
+            const int4 tv = S.tets[t];
+            const float4 p = qPos[q];
+            const int u = __float_as_int(p.w);
+            if (m == qm && (tv.x == u || tv.y == u || tv.z == u || tv.w == u)) return;
+            if (point_in_tet(V3{p.x, p.y, p.z}, ld(S.pos, tv.x), ld(S.pos, tv.y), ld(S.pos, tv.z), ld(S.pos, tv.w)))
+                atomicMin(&qTet[q], t);
+        });
+    if (!active || qTet[lane] == INT_MAX) return;
     S.flags[v] = 1;
-    S.inTet[v] = ht;
+    S.inTet[v] = qTet[lane];
     S.list[atomicAdd(S.counts + 4, 1)] = v;
 }
 
@@ -1799,87 +1829,58 @@ __device__ bool ccd_point_triangle(const V3 f0[3], const V3 f1[3], V3 p0, V3 p1,
     return false;
 }
 
-// CCD of every surface vertex that no tet contained, on its path from prev to pos
-__global__ __launch_bounds__(256) void pen_ccd_kernel(PenView S) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= S.nSurf) return;
-    const int v = S.surfVerts[i];
-    if (S.flags[v] & 1) return;
-    const V3 p1 = ld(S.pos, v);
-    if (!(p1.y < S.P.offHeight)) return;
-    const V3 p0 = ld(S.prev, v);
-    const int qm = S.vMesh[v];
-    const float len = vnorm(p1 - p0);
-    const V3 mid = 0.5f * (p0 + p1);
-    // boxes within the half path length of the midpoint (with a margin for the root's tolerance)
-    const float r = 0.5f * len + 1e-3f * len + 1e-6f;
-    const float r2 = r * r;
-    float best = 0.f;
-    int bestF = -1;
-    const int firstLeaf = S.sN - 1;
-    int node = S.sN > 0 ? 0 : -1;
-    for (int visits = 0; node >= 0; ++visits) {
-        if (visits > 2 * S.sN) {
-            atomicOr(S.error, 1);
-            break;
-        }
-        const BvhNode nd = S.sNodes[node];
-        const int skip = __float_as_int(nd.hi.w);
-        if (box_dist2(mid, nd) > r2) {
-            node = skip;
-            continue;
-        }
-        if (node < firstLeaf) {
-            node = __float_as_int(nd.lo.w);
-            continue;
-        }
-        node = skip;
-        const int f = __float_as_int(nd.lo.w);
-        const int4 fv = S.faces[f];
-        if (fv.w == qm && (fv.x == v || fv.y == v || fv.z == v)) continue;
-        const V3 a0[3] = {ld(S.prev, fv.x), ld(S.prev, fv.y), ld(S.prev, fv.z)};
-        const V3 a1[3] = {ld(S.pos, fv.x), ld(S.pos, fv.y), ld(S.pos, fv.z)};
-        float tt;
-        if (!ccd_point_triangle(a0, a1, p0, p1, tt)) continue;
-        const float depth = tt * len;
-        if (bestF < 0 || depth < best || (depth == best && f < bestF)) {
-            best = depth;
-            bestF = f;
-        }
+// CCD of every surface vertex that no tet contained, on its path from prev to pos, Q vertices per
+// wave: the earliest hit (the lower face on equal depth).
+template <int Q>
+__global__ __launch_bounds__(64) void pen_ccd_kernel(PenView S) {
+    __shared__ int stack[kQueryStack], leaves[kLeafQueue];
+    __shared__ float4 qFrom[Q], qTo[Q];  // the vertex in qFrom.w, the path's length in qTo.w
+    __shared__ float4 qSphere[Q];        // midpoint, squared radius
+    __shared__ int qMesh[Q];
+    __shared__ unsigned long long qHit[Q];  // depth bits (depths are not negative), face
+    const int lane = threadIdx.x;
+    const int i = blockIdx.x * Q + lane;
+    const int v = lane < Q && i < S.nSurf ? S.surfVerts[i] : -1;
+    bool active = v >= 0 && !(S.flags[v] & 1);
+    if (active) {
+        const V3 p1 = ld(S.pos, v);
+        active = p1.y < S.P.offHeight;
+        const V3 p0 = ld(S.prev, v);
+        const float len = vnorm(p1 - p0);
+        const V3 mid = 0.5f * (p0 + p1);
+        // boxes within the half path length of the midpoint (with a margin for the root's tolerance)
+        const float r = 0.5f * len + 1e-3f * len + 1e-6f;
+        qFrom[lane] = make_float4(p0.x, p0.y, p0.z, __int_as_float(v));
+        qTo[lane] = make_float4(p1.x, p1.y, p1.z, len);
+        qSphere[lane] = make_float4(mid.x, mid.y, mid.z, r * r);
+        qMesh[lane] = S.vMesh[v];
+        qHit[lane] = ~0ull;
     }
-    if (bestF < 0) return;
+    wave_queries<Q>(
+        S.sPairs, S.sN, active, stack, leaves, S.error,
+        [&](int q, float4 lo, float4 hi) {
+            const float4 c = qSphere[q];
+            return !(box_dist2(V3{c.x, c.y, c.z}, BvhNode{lo, hi}) > c.w);
+        },
+        [&](bool has, int q, float4 lo, float4) {
+            if (!has) return;
+            const int f = __float_as_int(lo.w);
+            const int4 fv = S.faces[f];
+            const float4 from = qFrom[q], to = qTo[q];
+            const int u = __float_as_int(from.w);
+            if (fv.w == qMesh[q] && (fv.x == u || fv.y == u || fv.z == u)) return;
+            const V3 a0[3] = {ld(S.prev, fv.x), ld(S.prev, fv.y), ld(S.prev, fv.z)};
+            const V3 a1[3] = {ld(S.pos, fv.x), ld(S.pos, fv.y), ld(S.pos, fv.z)};
+            float tt;
+            if (!ccd_point_triangle(a0, a1, V3{from.x, from.y, from.z}, V3{to.x, to.y, to.z}, tt)) return;
+            const float depth = tt * to.w;
+            atomicMin(&qHit[q], ((unsigned long long)__float_as_uint(depth + 0.f) << 32) | (unsigned)f);
+        });
+    if (!active || qHit[lane] == ~0ull) return;
     S.stored[v] = 1;
-    S.rec[(int64_t)v * S.cap].face = bestF;
+    S.rec[(int64_t)v * S.cap].face = (int)(unsigned)qHit[lane];
     S.flags[v] = 2;
     atomicAdd(S.counts + 2, 1);
-}
-
-// boxes of tets (kind 3 primitives): lo, hi per tet
-__global__ __launch_bounds__(256) void tet_box_kernel(const float4* pos, const int4* tets, int n, float4* boxes) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    const int4 tv = tets[t];
-    const V3 a = ld(pos, tv.x), b = ld(pos, tv.y), c = ld(pos, tv.z), d = ld(pos, tv.w);
-    boxes[2 * t] = make_float4(fminf(fminf(a.x, b.x), fminf(c.x, d.x)), fminf(fminf(a.y, b.y), fminf(c.y, d.y)),
-                               fminf(fminf(a.z, b.z), fminf(c.z, d.z)), 0.f);
-    boxes[2 * t + 1] = make_float4(fmaxf(fmaxf(a.x, b.x), fmaxf(c.x, d.x)), fmaxf(fmaxf(a.y, b.y), fmaxf(c.y, d.y)),
-                                   fmaxf(fmaxf(a.z, b.z), fmaxf(c.z, d.z)), 0.f);
-}
-
-// boxes of faces over their path from prev to pos (movingFaceBoundsFunc, ContinuousCollisionDetector.cpp:19-65)
-__global__ __launch_bounds__(256) void swept_box_kernel(const float4* pos, const float4* prev, const int4* faces, int n,
-                                                        float4* boxes) {
-    const int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= n) return;
-    const int4 fv = faces[f];
-    const V3 q[6] = {ld(pos, fv.x), ld(pos, fv.y), ld(pos, fv.z), ld(prev, fv.x), ld(prev, fv.y), ld(prev, fv.z)};
-    V3 lo = q[0], hi = q[0];
-    for (int k = 1; k < 6; ++k) {
-        lo = {fminf(lo.x, q[k].x), fminf(lo.y, q[k].y), fminf(lo.z, q[k].z)};
-        hi = {fmaxf(hi.x, q[k].x), fmaxf(hi.y, q[k].y), fmaxf(hi.z, q[k].z)};
-    }
-    boxes[2 * f] = make_float4(lo.x, lo.y, lo.z, 0.f);
-    boxes[2 * f + 1] = make_float4(hi.x, hi.y, hi.z, 0.f);
 }
 
 __global__ __launch_bounds__(256) void fill_u8_kernel(uint8_t* p, int64_t n) {
@@ -2194,6 +2195,7 @@ void ContactDetector::finalize() {
         vSortTemp_ = dalloc<char>(vSortTempBytes_);
     }
     // BVH storage
+    allocBuildScratch({nf_, ne_, pen_ ? (int)penHost_.tetMesh.size() : 0});
     allocBvh(fb_, nf_, !pen_);
     allocBvh(eb_, ne_, !pen_);
     if (pen_ && nf_ > 0) fb_.mesh = dalloc<int>(2 * (size_t)nf_ - 1);
@@ -2202,12 +2204,10 @@ void ContactDetector::finalize() {
     ready_ = true;
     updateBvh(true);
     if (pen_) {
-        buildBvh(tb_, 3, tetBoxes_);
+        buildBvh(tb_, 3);
         // the swept-face tree over zero-length paths, so that every later pass refits (or
         // rebuilds on schedule) without a first-use build
-        hipLaunchKernelGGL(swept_box_kernel, dim3(blocks_for(nf_)), dim3(256), 0, stream_, pos_, pos_, faces_, nf_,
-                           sweptBoxes_);
-        buildBvh(sb_, 3, sweptBoxes_);
+        buildBvh(sb_, 4, pos_);
         sweptBuilt_ = true;
     }
 }
@@ -2220,21 +2220,34 @@ void ContactDetector::allocBvh(DeviceBvh& B, int n, bool pairs) {
     if (pairs) B.pairs = dalloc<BvhPair>(std::max(B.n - 1, 1));
     B.parent = dalloc<int>(2 * (size_t)B.n - 1);
     B.right = dalloc<int>(std::max(B.n - 1, 1));
-    B.jump = dalloc<int>(4 * (size_t)std::max(B.n - 1, 1));
-    B.keys = dalloc<uint64_t>(B.n);
     B.keysAlt = dalloc<uint64_t>(B.n);
-    B.depthKeys = dalloc<uint64_t>(std::max(B.n - 1, 1));
-    B.depthKeysAlt = dalloc<uint64_t>(std::max(B.n - 1, 1));
-    B.depth = dalloc<int>(std::max(B.n - 1, 1));
     B.levelNodes = dalloc<int>(std::max(B.n - 1, 1));
     B.dLevelBegin = dalloc<int>(kMaxDepth + 1);
-    size_t s1 = 0, s2 = 0;
-    hip_check(rocprim::radix_sort_keys(nullptr, s1, B.keys, B.keysAlt, (size_t)B.n, 0, 62, stream_), "sort size");
-    hip_check(rocprim::radix_sort_keys(nullptr, s2, B.depthKeys, B.depthKeysAlt, (size_t)std::max(B.n - 1, 1), 0, 40,
-                                       stream_),
-              "sort size");
-    B.sortTempBytes = std::max(s1, s2);
-    B.sortTemp = dalloc<char>(B.sortTempBytes);
+}
+
+// Buffers of the tree builds, which run one after another on the detector's stream: one set, enough
+// for trees of any of the sizes.
+void ContactDetector::allocBuildScratch(const std::vector<int>& sizes) {
+    const int n = *std::max_element(sizes.begin(), sizes.end());
+    if (n == 0) return;
+    const size_t ni = (size_t)std::max(n - 1, 1);
+    scratch_.jump = dalloc<int>(4 * ni);
+    scratch_.keys = dalloc<uint64_t>(n);
+    scratch_.depthKeys = dalloc<uint64_t>(ni);
+    scratch_.depthKeysAlt = dalloc<uint64_t>(ni);
+    scratch_.depth = dalloc<int>(ni);
+    // a sort's temporary storage need not grow with its size: the largest over the trees
+    for (int m : sizes) {
+        if (m == 0) continue;
+        size_t s1 = 0, s2 = 0;
+        hip_check(rocprim::radix_sort_keys(nullptr, s1, scratch_.keys, scratch_.keys, (size_t)m, 0, 62, stream_),
+                  "sort size");
+        hip_check(rocprim::radix_sort_keys(nullptr, s2, scratch_.depthKeys, scratch_.depthKeysAlt,
+                                           (size_t)std::max(m - 1, 1), 0, 40, stream_),
+                  "sort size");
+        scratch_.sortTempBytes = std::max(scratch_.sortTempBytes, std::max(s1, s2));
+    }
+    scratch_.sortTemp = dalloc<char>(scratch_.sortTempBytes);
 }
 
 namespace {
@@ -2248,21 +2261,23 @@ CDView make_view(float4* pos, int nv, int nf, int ne) {
 }
 }  // namespace
 
-void ContactDetector::buildBvh(DeviceBvh& B, int kind, const float4* boxes) {
+void ContactDetector::buildBvh(DeviceBvh& B, int kind, const float4* prev) {
     if (B.n == 0) return;
     CDView S = make_view(pos_, nv_, nf_, ne_);
     S.faces = faces_;
     S.edges = edges_;
-    S.boxes = boxes;
+    S.tets = penTets_;
+    S.prev = prev;
     const int n = B.n;
+    BvhScratch& T = scratch_;
     if (blocks_for(n) > boxPartialBlocks_)
         fail(GVBD_ERR_STATE, "tree of " + std::to_string(n) + " primitives exceeds the partial-box buffer");
     unsigned int* box = (unsigned int*)sceneBox_;
     hipLaunchKernelGGL(centroid_box_kernel, dim3(blocks_for(n)), dim3(256), 0, stream_, S, kind, n, boxPartial_);
     hipLaunchKernelGGL(box_final_kernel, dim3(1), dim3(256), 0, stream_, boxPartial_, blocks_for(n), box);
-    hipLaunchKernelGGL(morton_kernel, dim3(blocks_for(n)), dim3(256), 0, stream_, S, kind, n, box, B.keys);
-    size_t tb = B.sortTempBytes;
-    hip_check(rocprim::radix_sort_keys(B.sortTemp, tb, B.keys, B.keysAlt, (size_t)n, 0, 62, stream_), "morton sort");
+    hipLaunchKernelGGL(morton_kernel, dim3(blocks_for(n)), dim3(256), 0, stream_, S, kind, n, box, T.keys);
+    size_t tb = T.sortTempBytes;
+    hip_check(rocprim::radix_sort_keys(T.sortTemp, tb, T.keys, B.keysAlt, (size_t)n, 0, 62, stream_), "morton sort");
     if (kind == 0 && nv_ > 0) {
         // VF query order: vertices sorted by Morton code in the face tree's box
         hipLaunchKernelGGL(morton_kernel, dim3(blocks_for(nv_)), dim3(256), 0, stream_, S, 2, nv_, box, vKeys_);
@@ -2279,23 +2294,23 @@ void ContactDetector::buildBvh(DeviceBvh& B, int kind, const float4* boxes) {
     B.levelBegin.clear();
     const int ni = n - 1;
     if (ni > 0) {
-        int* d0 = B.jump;
-        int* d1 = B.jump + ni;
-        int* a0 = B.jump + 2 * (size_t)ni;
-        int* a1 = B.jump + 3 * (size_t)ni;
+        int* d0 = T.jump;
+        int* d1 = T.jump + ni;
+        int* a0 = T.jump + 2 * (size_t)ni;
+        int* a1 = T.jump + 3 * (size_t)ni;
         hipLaunchKernelGGL(depth_init_kernel, dim3(blocks_for(ni)), dim3(256), 0, stream_, B.parent, ni, d0, a0);
         for (int round = 0; (1 << round) < kMaxDepth; ++round) {
             hipLaunchKernelGGL(depth_jump_kernel, dim3(blocks_for(ni)), dim3(256), 0, stream_, d0, a0, d1, a1, ni);
             std::swap(d0, d1);
             std::swap(a0, a1);
         }
-        hipLaunchKernelGGL(depth_keys_kernel, dim3(blocks_for(ni)), dim3(256), 0, stream_, d0, a0, ni, B.depth,
-                           B.depthKeys, error_);
-        size_t tb2 = B.sortTempBytes;
-        hip_check(rocprim::radix_sort_keys(B.sortTemp, tb2, B.depthKeys, B.depthKeysAlt, (size_t)ni, 0, 40, stream_),
+        hipLaunchKernelGGL(depth_keys_kernel, dim3(blocks_for(ni)), dim3(256), 0, stream_, d0, a0, ni, T.depth,
+                           T.depthKeys, error_);
+        size_t tb2 = T.sortTempBytes;
+        hip_check(rocprim::radix_sort_keys(T.sortTemp, tb2, T.depthKeys, T.depthKeysAlt, (size_t)ni, 0, 40, stream_),
                   "depth sort");
         hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(256), 0, stream_, depthHist_, (int64_t)kMaxDepth, -1);
-        hipLaunchKernelGGL(level_nodes_kernel, dim3(blocks_for(ni)), dim3(256), 0, stream_, B.depthKeysAlt, ni,
+        hipLaunchKernelGGL(level_nodes_kernel, dim3(blocks_for(ni)), dim3(256), 0, stream_, T.depthKeysAlt, ni,
                            B.levelNodes, depthHist_);
         std::vector<int> starts(kMaxDepth, -1);
         hip_check(hipMemcpyAsync(starts.data(), depthHist_, kMaxDepth * sizeof(int), hipMemcpyDeviceToHost, stream_),
@@ -2324,7 +2339,7 @@ void ContactDetector::buildBvh(DeviceBvh& B, int kind, const float4* boxes) {
                                  hipMemcpyHostToDevice, stream_),
                   "level upload");
     }
-    refitBvh(B, kind, stream_, boxes);
+    refitBvh(B, kind, stream_, prev);
     if (B.mesh && kind == 0) {
         // mesh membership changes only with the tree's topology: set at every build
         hipLaunchKernelGGL(node_mesh_leaf_kernel, dim3(blocks_for(n)), dim3(256), 0, stream_, faces_, B.nodes, n,
@@ -2342,12 +2357,13 @@ void ContactDetector::buildBvh(DeviceBvh& B, int kind, const float4* boxes) {
     }
 }
 
-void ContactDetector::refitBvh(DeviceBvh& B, int kind, hipStream_t stream, const float4* boxes, const int* gate) {
+void ContactDetector::refitBvh(DeviceBvh& B, int kind, hipStream_t stream, const float4* prev, const int* gate) {
     if (B.n == 0) return;
     CDView S = make_view(pos_, nv_, nf_, ne_);
     S.faces = faces_;
     S.edges = edges_;
-    S.boxes = boxes;
+    S.tets = penTets_;
+    S.prev = prev;
     S.gate = gate;
     hipLaunchKernelGGL(leaf_box_kernel, dim3(blocks_for(B.n)), dim3(256), 0, stream, S, kind, B.nodes, B.pairs, B.n);
     for (const auto& seg : B.segments) {
@@ -2399,8 +2415,6 @@ void ContactDetector::setupPenetrationDevice() {
     up(penVNbr_, H.vNbr.data(), sizeof(int32_t) * H.vNbr.size());
     penSurf_ = dalloc<int>(std::max(nSurf_, 1));
     up(penSurf_, H.surfVerts.data(), sizeof(int32_t) * H.surfVerts.size());
-    tetBoxes_ = dalloc<float4>(2 * (size_t)std::max(nt_, 1));
-    sweptBoxes_ = dalloc<float4>(2 * (size_t)std::max(nf_, 1));
     penFlags_ = dalloc<uint8_t>(std::max(nv_, 1));
     penCounts_ = dalloc<int>(kPenCounts);
     penInTet_ = dalloc<int>(std::max(nv_, 1));
@@ -2408,12 +2422,47 @@ void ContactDetector::setupPenetrationDevice() {
     hipLaunchKernelGGL(fill_u8_kernel, dim3(std::min(blocks_for(nv_), 4096)), dim3(256), 0, stream_, penFlags_,
                        (int64_t)nv_);
     hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(256), 0, stream_, penCounts_, (int64_t)kPenCounts, 0);
-    allocBvh(tb_, nt_, false);
-    allocBvh(sb_, nf_, false);
-    // tet boxes for the first tree build (at the end of finalize)
-    hipLaunchKernelGGL(tet_box_kernel, dim3(blocks_for(nt_)), dim3(256), 0, stream_, pos_, penTets_, nt_, tetBoxes_);
+    allocBvh(tb_, nt_, true);
+    allocBvh(sb_, nf_, true);
     hip_check(hipGetLastError(), "penetration setup launch");
 }
+
+namespace {
+// Queries per wave: few where there are few (more waves, each with a shorter path), more where the
+// waves fill the chip anyway (less of a wave's time goes to its start at the root and its end, with
+// lanes idle). Measured, VF and EE queries together, tori of 8,192 vertices and 24,576 edges, us per
+// pass with 8 / 16 / 32 / 64 queries per wave (one thread per query before: 201, 246, 322, 663, 1472):
+// 8k vertices 63 / 71 / 92 / 121, 36k 123 / 110 / 113 / 148, 65k 233 / 191 / 195 / 208,
+// 221k 702 / 512 / 478 / 500, 524k 1818 / 1285 / 1140 / 1166. A query's bits and a node's share a
+// stack entry, which limits the tree (see wave_queries); 8 take any tree.
+int queries_per_wave(int queries, int prims) {
+    if (queries > 262144 && prims <= (1 << query_node_bits<32>())) return 32;
+    if (queries > 49152 && prims <= (1 << query_node_bits<16>())) return 16;
+    return 8;
+}
+
+template <int Q> void launch_contain_q(const PenView& S, hipStream_t stream) {
+    hipLaunchKernelGGL(pen_contain_kernel<Q>, dim3((S.nSurf + Q - 1) / Q), dim3(64), 0, stream, S);
+}
+template <int Q> void launch_ccd_q(const PenView& S, hipStream_t stream) {
+    hipLaunchKernelGGL(pen_ccd_kernel<Q>, dim3((S.nSurf + Q - 1) / Q), dim3(64), 0, stream, S);
+}
+
+void launch_contain(const PenView& S, hipStream_t stream) {
+    switch (queries_per_wave(S.nSurf, S.tN)) {
+    case 32: launch_contain_q<32>(S, stream); break;
+    case 16: launch_contain_q<16>(S, stream); break;
+    default: launch_contain_q<8>(S, stream); break;
+    }
+}
+void launch_ccd(const PenView& S, hipStream_t stream) {
+    switch (queries_per_wave(S.nSurf, S.sN)) {
+    case 32: launch_ccd_q<32>(S, stream); break;
+    case 16: launch_ccd_q<16>(S, stream); break;
+    default: launch_ccd_q<8>(S, stream); break;
+    }
+}
+}  // namespace
 
 namespace {
 PenView pen_view(float4* pos, const float4* prev, const int4* faces) {
@@ -2430,12 +2479,11 @@ void ContactDetector::penetrationDcd(bool rebuild) {
     hipLaunchKernelGGL(fill_int_kernel, dim3(std::min(blocks_for(nv_), 4096)), dim3(256), 0, stream_, vfStored_,
                        (int64_t)nv_, 0);
     hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(256), 0, stream_, penCounts_, (int64_t)kPenCounts, 0);
-    hipLaunchKernelGGL(tet_box_kernel, dim3(blocks_for(nt_)), dim3(256), 0, stream_, pos_, penTets_, nt_, tetBoxes_);
     if (rebuild) {
-        buildBvh(tb_, 3, tetBoxes_);
+        buildBvh(tb_, 3);
         buildBvh(fb_, 0);
     } else {
-        refitBvh(tb_, 3, stream_, tetBoxes_);
+        refitBvh(tb_, 3, stream_);
         refitBvh(fb_, 0, stream_);
     }
     PenView S = pen_view(pos_, nullptr, faces_);
@@ -2449,7 +2497,7 @@ void ContactDetector::penetrationDcd(bool rebuild) {
     S.surfVerts = penSurf_;
     S.nSurf = nSurf_;
     S.vMesh = vMesh_;
-    S.tNodes = tb_.nodes;
+    S.tPairs = tb_.pairs;
     S.tN = tb_.n;
     S.fNodes = fb_.nodes;
     S.fRight = fb_.right;
@@ -2465,7 +2513,7 @@ void ContactDetector::penetrationDcd(bool rebuild) {
     S.list = penList_;
     S.error = error_;
     if (nSurf_ > 0) {
-        hipLaunchKernelGGL(pen_contain_kernel, dim3((nSurf_ + 63) / 64), dim3(64), 0, stream_, S);
+        launch_contain(S, stream_);
         // a wave per contained vertex (their number is only known on the device); 4096 waves fill the chip
         hipLaunchKernelGGL(pen_closest_kernel, dim3(std::min(nSurf_, 4096)), dim3(64), 0, stream_, S);
     }
@@ -2475,19 +2523,17 @@ void ContactDetector::penetrationDcd(bool rebuild) {
 void ContactDetector::penetrationCcd(const float4* prev, bool rebuild) {
     if (!ready_ || !pen_) fail(GVBD_ERR_STATE, "detector not finalized for penetration contact");
     if (!penHost_.params.ccd || nf_ == 0) return;
-    hipLaunchKernelGGL(swept_box_kernel, dim3(blocks_for(nf_)), dim3(256), 0, stream_, pos_, prev, faces_, nf_,
-                       sweptBoxes_);
     if (rebuild || !sweptBuilt_) {
-        buildBvh(sb_, 3, sweptBoxes_);
+        buildBvh(sb_, 4, prev);
         sweptBuilt_ = true;
     } else {
-        refitBvh(sb_, 3, stream_, sweptBoxes_);
+        refitBvh(sb_, 4, stream_, prev);
     }
     PenView S = pen_view(pos_, prev, faces_);
     S.surfVerts = penSurf_;
     S.nSurf = nSurf_;
     S.vMesh = vMesh_;
-    S.sNodes = sb_.nodes;
+    S.sPairs = sb_.pairs;
     S.sN = sb_.n;
     S.P = penHost_.params;
     S.stored = vfStored_;
@@ -2496,7 +2542,7 @@ void ContactDetector::penetrationCcd(const float4* prev, bool rebuild) {
     S.flags = penFlags_;
     S.counts = penCounts_;
     S.error = error_;
-    if (nSurf_ > 0) hipLaunchKernelGGL(pen_ccd_kernel, dim3(blocks_for(nSurf_)), dim3(256), 0, stream_, S);
+    if (nSurf_ > 0) launch_ccd(S, stream_);
     hip_check(hipGetLastError(), "penetration CCD launch");
 }
 
@@ -2594,19 +2640,6 @@ template <int Q> void launch_ee(const CDView& S, hipStream_t stream) {
         hipLaunchKernelGGL((ee_query_kernel<Q, 8>), grid, dim3(64), 0, stream, S);
     else
         hipLaunchKernelGGL((ee_query_kernel<Q, kMaxCap>), grid, dim3(64), 0, stream, S);
-}
-
-// Queries per wave: few where there are few (more waves, each with a shorter path), more where the
-// waves fill the chip anyway (less of a wave's time goes to its start at the root and its end, with
-// lanes idle). Measured, VF and EE queries together, tori of 8,192 vertices and 24,576 edges, us per
-// pass with 8 / 16 / 32 / 64 queries per wave (one thread per query before: 201, 246, 322, 663, 1472):
-// 8k vertices 63 / 71 / 92 / 121, 36k 123 / 110 / 113 / 148, 65k 233 / 191 / 195 / 208,
-// 221k 702 / 512 / 478 / 500, 524k 1818 / 1285 / 1140 / 1166. A query's bits and a node's share a
-// stack entry, which limits the tree (see wave_queries); 8 take any tree.
-int queries_per_wave(int queries, int prims) {
-    if (queries > 262144 && prims <= (1 << query_node_bits<32>())) return 32;
-    if (queries > 49152 && prims <= (1 << query_node_bits<16>())) return 16;
-    return 8;
 }
 
 void launch_queries(const CDView& S, hipStream_t vfStream, hipStream_t eeStream) {
