@@ -40,25 +40,23 @@ __global__ __launch_bounds__(kBlock) void residual_kernel(SceneView S, int nslot
         float cmu = 0.f;
         const float4 mat = S.tmat[slot.w >> SLOT_MAT_SHIFT];
         for (int r = slot.y; r < slot.z; ++r) {
-            const TetInc rec = S.tinc[r];
-            const float A = S.tvol[r];
+            float A;
+            TetTerms t;
+            if (S.trow) {
+                const TetRow rec = S.trow[r];
+                A = S.tvol[r];
+                t = tet_terms_rows(x, xyz(S.pos[rec.nb[0]]), xyz(S.pos[rec.nb[1]]), xyz(S.pos[rec.nb[2]]),
+                                   mk(rec.m[0], rec.m[1], rec.m[2]), mk(rec.m[3], rec.m[4], rec.m[5]),
+                                   mk(rec.m[6], rec.m[7], rec.m[8]));
+            } else {
+                const TetInc rec = S.tinc[r];
+                A = rec.A;
+                t = tet_terms(x, xyz(S.pos[rec.nb[0]]), xyz(S.pos[rec.nb[1]]), xyz(S.pos[rec.nb[2]]), rec.c, rec.w[0],
+                              rec.w[1], rec.w[2]);
+            }
             const float Amu = A * mat.x, Alm = A * mat.y;
-            const f3 m0 = mk(rec.m[0], rec.m[1], rec.m[2]);
-            const f3 m1 = mk(rec.m[3], rec.m[4], rec.m[5]);
-            const f3 m2 = mk(rec.m[6], rec.m[7], rec.m[8]);
-            const f3 d0 = xyz(S.pos[rec.nb[0]]) - x;
-            const f3 d1 = xyz(S.pos[rec.nb[1]]) - x;
-            const f3 d2 = xyz(S.pos[rec.nb[2]]) - x;
-            const f3 c0 = m0.x * d0 + m1.x * d1 + m2.x * d2;
-            const f3 c1 = m0.y * d0 + m1.y * d1 + m2.y * d2;
-            const f3 c2 = m0.z * d0 + m1.z * d1 + m2.z * d2;
-            const f3 mv = mk(-(m0.x + m1.x + m2.x), -(m0.y + m1.y + m2.y), -(m0.z + m1.z + m2.z));
-            const f3 k0 = cross(c1, c2), k1 = cross(c2, c0), k2 = cross(c0, c1);
-            const float J = dot(c0, k0);
-            const f3 g = mv.x * k0 + mv.y * k1 + mv.z * k2;
-            const f3 Fm = mv.x * c0 + mv.y * c1 + mv.z * c2;
-            const float s = Alm * (J - mat.z);
-            f = f - (Amu * Fm + s * g);
+            const f3 g = t.g;
+            f = f - (Amu * t.Fm + (Alm * (t.J - mat.z)) * g);
             const f3 ag = Alm * g;
             h.xx += ag.x * g.x;
             h.xy += ag.x * g.y;
@@ -66,7 +64,7 @@ __global__ __launch_bounds__(kBlock) void residual_kernel(SceneView S, int nslot
             h.yy += ag.y * g.y;
             h.yz += ag.y * g.z;
             h.zz += ag.z * g.z;
-            cmu += Amu * dot(mv, mv);
+            cmu += Amu * t.mm;
         }
         if (slot.w & SLOT_DAMPING) {
             // the solve's damping term (VBD_NeoHookean.cpp:562-574)

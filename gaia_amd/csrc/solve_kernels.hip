@@ -15,13 +15,13 @@
 //   velocity update + damping          VBD/VBDPhysics.cpp:2486-2561, VBDCloth/VBDClothPhysics.cpp:2318-2360
 //
 // Design (not a translation of the CUDA kernel): LPV lanes of one wave64 share one vertex
-// and stride over its colour-major incidence records (64 B per tet, 32 B per face or
+// and stride over its colour-major incidence records (32 or 48 B per tet, 32 B per face or
 // bending stencil, streamed with float4 loads) plus float4 neighbour gathers; partial sums
 // are combined with butterfly lane exchanges. Element Hessians are evaluated in contracted
 // closed form instead of the reference's 9x9 / 6x6 assemblies:
 //   tet:  H = A (mu |m|^2 I + lambda g g^T), g = cof(F) m;  f = -A (mu F m + lambda (det F - a) g)
 //         (the second derivative of det F is antisymmetric in the shape indices, so it
-//         vanishes against m (x) m);
+//         vanishes against m (x) m), with F m, g and det F straight from the edges (see TetInc);
 //   StVK: H = A [(m^T S m) I + mu |m|^2 F F^T + (mu + lambda)(F m)(F m)^T];  f = -A F S m.
 // One launch covers one parallel group of every scene of a plan; each block's work item is
 // either tet slots (updated in place: vertices of one colour share no tet, as in the
@@ -175,52 +175,47 @@ __device__ __forceinline__ void tet_block(const SceneView& S, const WorkItem& it
         blockBegin = S.slots[it.slotBegin].y;
         blockEnd = S.slots[it.slotBegin + it.count - 1].z;
     }
-    // the mesh's material (mu, lambda, a); A mu and A lambda are formed per record from its tet's
-    // rest volume, the same float products as precomputed ones
+    // the mesh's material (mu, lambda, a); A mu and A lambda are formed per record
     float4 mat = make_float4(0.f, 0.f, 0.f, 0.f);
     if (active) mat = S.tmat[slot.w >> SLOT_MAT_SHIFT];
-    const float* __restrict__ tvol = S.tvol;
-    for_lane_records<LPV, STAGE, 3>(reinterpret_cast<const float4*>(S.tinc), blockBegin, blockEnd, slot.y + sub,
-                                    slot.z, lds, [&](const float4* r, int k) {
-        const float4 r0 = r[0];
-        const float4 r1 = r[1];
-        const float4 r2 = r[2];
-        const int n0 = __float_as_int(r0.x), n1 = __float_as_int(r0.y), n2 = __float_as_int(r0.z);
-        const f3 m0 = mk(r0.w, r1.x, r1.y);
-        const f3 m1 = mk(r1.z, r1.w, r2.x);
-        const f3 m2 = mk(r2.y, r2.z, r2.w);
-        const float A = tvol[k];
+    const auto add = [&](const TetTerms& t, float A) {
         const float Amu = A * mat.x;
         const float Alm = A * mat.y;
-        const float a = mat.z;
-        const f3 d0 = xyz(pos[n0]) - x;
-        const f3 d1 = xyz(pos[n1]) - x;
-        const f3 d2 = xyz(pos[n2]) - x;
-        // F columns: F e_c = sum_k d_k m_k[c]
-        const f3 c0 = m0.x * d0 + m1.x * d1 + m2.x * d2;
-        const f3 c1 = m0.y * d0 + m1.y * d1 + m2.y * d2;
-        const f3 c2 = m0.z * d0 + m1.z * d1 + m2.z * d2;
-        const f3 mv = mk(-(m0.x + m1.x + m2.x), -(m0.y + m1.y + m2.y), -(m0.z + m1.z + m2.z));
-        // cof(F) columns are c1 x c2, c2 x c0, c0 x c1
-        const f3 k0 = cross(c1, c2);
-        const f3 k1 = cross(c2, c0);
-        const f3 k2 = cross(c0, c1);
-        const float J = dot(c0, k0);
-        const f3 g = mv.x * k0 + mv.y * k1 + mv.z * k2;
-        const f3 Fm = mv.x * c0 + mv.y * c1 + mv.z * c2;
-        const float s = Alm * (J - a);
-        f0 -= Amu * Fm.x + s * g.x;
-        f1 -= Amu * Fm.y + s * g.y;
-        f2 -= Amu * Fm.z + s * g.z;
-        const f3 ag = Alm * g;
-        gxx += ag.x * g.x;
-        gxy += ag.x * g.y;
-        gxz += ag.x * g.z;
-        gyy += ag.y * g.y;
-        gyz += ag.y * g.z;
-        gzz += ag.z * g.z;
-        cmu += Amu * dot(mv, mv);
-    });
+        const float s = Alm * (t.J - mat.z);
+        f0 -= Amu * t.Fm.x + s * t.g.x;
+        f1 -= Amu * t.Fm.y + s * t.g.y;
+        f2 -= Amu * t.Fm.z + s * t.g.z;
+        const f3 ag = Alm * t.g;
+        gxx += ag.x * t.g.x;
+        gxy += ag.x * t.g.y;
+        gxz += ag.x * t.g.z;
+        gyy += ag.y * t.g.y;
+        gyz += ag.y * t.g.z;
+        gzz += ag.z * t.g.z;
+        cmu += Amu * t.mm;
+    };
+    if (S.trow) {
+        const float* __restrict__ tvol = S.tvol;
+        for_lane_records<LPV, STAGE, 3>(reinterpret_cast<const float4*>(S.trow), blockBegin, blockEnd, slot.y + sub,
+                                        slot.z, lds, [&](const float4* r, int k) {
+            const float4 r0 = r[0];
+            const float4 r1 = r[1];
+            const float4 r2 = r[2];
+            add(tet_terms_rows(x, xyz(pos[__float_as_int(r0.x)]), xyz(pos[__float_as_int(r0.y)]),
+                               xyz(pos[__float_as_int(r0.z)]), mk(r0.w, r1.x, r1.y), mk(r1.z, r1.w, r2.x),
+                               mk(r2.y, r2.z, r2.w)),
+                tvol[k]);
+        });
+    } else {
+        for_lane_records<LPV, 2 * STAGE, 2>(reinterpret_cast<const float4*>(S.tinc), blockBegin, blockEnd,
+                                            slot.y + sub, slot.z, lds, [&](const float4* r, int) {
+            const float4 r0 = r[0];
+            const float4 r1 = r[1];
+            add(tet_terms(x, xyz(pos[__float_as_int(r0.x)]), xyz(pos[__float_as_int(r0.y)]),
+                          xyz(pos[__float_as_int(r0.z)]), r0.w, r1.x, r1.y, r1.z),
+                r1.w);
+        });
+    }
     if (LPV > 1) {
         f0 = lane_sum<LPV>(f0);
         f1 = lane_sum<LPV>(f1);
@@ -836,8 +831,8 @@ __device__ __forceinline__ void cloth_block(const SceneView& S, const WorkItem& 
 
 // One launch = one parallel group of every scene referenced by `items`; the block's
 // work kind is uniform, so the branch does not diverge.
-// STAGE > 0 stages the incidence records through LDS, STAGE 64-byte records (or 2 * STAGE cloth
-// records of 32 bytes) per chunk.
+// STAGE > 0 stages the incidence records through LDS, 2 * STAGE records of 32 bytes (or STAGE of 48)
+// per chunk.
 // CONTACT selects the variant for scenes with collision handling (contact forces, bound
 // truncation); the others carry none of that code, so their register use is unchanged by it.
 template <int LPV, int BLOCK, int STAGE, bool CONTACT>

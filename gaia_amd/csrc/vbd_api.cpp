@@ -42,7 +42,8 @@ struct DeviceScene {
     uint8_t* vflag = nullptr;
     int4* slots = nullptr;
     TetInc* tinc = nullptr;
-    float* tvol = nullptr;     // per incidence record: rest volume of its tet
+    TetRow* trow = nullptr;    // instead of tinc (scenes with material damping or the accelerator)
+    float* tvol = nullptr;     // per row record: rest volume of its tet
     float4* tmat = nullptr;    // per tet mesh: (mu, lambda, a, 0)
     ClothSlot* cslots = nullptr;
     FaceInc* cface = nullptr;
@@ -379,34 +380,63 @@ struct TetContactRefs {
     std::vector<int4>* ranges = nullptr;
 };
 
+// Incidence records of a scene's tets: rows in scenes that use them, the short records otherwise.
+struct TetRecords {
+    bool rows = false;
+    std::vector<TetInc> inc;
+    std::vector<TetRow> row;
+    std::vector<float> vol;  // per row record
+    size_t size() const { return rows ? row.size() : inc.size(); }
+};
+
 void emit_tet_slot(const TetMeshHost& m, int32_t off, int32_t lv, int32_t mat, std::vector<int4>& slots,
-                   std::vector<TetInc>& tinc, std::vector<float>& tvol, std::vector<int64_t>& work,
-                   const TetContactRefs* refs) {
+                   TetRecords& recs, std::vector<int64_t>& work, const TetContactRefs* refs) {
     int4 slot;
     slot.x = off + lv;
-    slot.y = (int32_t)tinc.size();
+    slot.y = (int32_t)recs.size();
     for (int32_t k = m.incBegin[lv]; k < m.incBegin[lv + 1]; ++k) {
         const int32_t t = m.incTet[k];
         const int32_t ord = m.incOrder[k];
         const float* D = &m.dminv[9 * (size_t)t];
-        // shape-matrix row j of tet vertex j: j = 0 -> minus column sums, j >= 1 -> row j-1 of DmInv
-        float B[4][3];
-        for (int c = 0; c < 3; ++c) {
-            B[0][c] = -D[0 + 3 * c] - D[1 + 3 * c] - D[2 + 3 * c];
-            for (int j = 1; j < 4; ++j) B[j][c] = D[(j - 1) + 3 * c];
-        }
-        TetInc rec{};
-        int n = 0;
+        int nb[3], row[3], n = 0;
         for (int j = 0; j < 4; ++j) {
             if (j == ord) continue;
-            rec.nb[n] = off + m.tets[4 * (size_t)t + j];
-            for (int c = 0; c < 3; ++c) rec.m[3 * n + c] = B[j][c];
-            ++n;
+            nb[n] = off + m.tets[4 * (size_t)t + j];
+            row[n++] = j;
         }
-        tinc.push_back(rec);
-        tvol.push_back(m.vol[t]);
+        // shape-matrix row j of tet vertex j: j = 0 -> minus column sums, j >= 1 -> row j-1 of DmInv
+        if (recs.rows) {
+            float B[4][3];
+            for (int c = 0; c < 3; ++c) {
+                B[0][c] = -D[0 + 3 * c] - D[1 + 3 * c] - D[2 + 3 * c];
+                for (int j = 1; j < 4; ++j) B[j][c] = D[(j - 1) + 3 * c];
+            }
+            TetRow rec{};
+            for (int i = 0; i < 3; ++i) {
+                rec.nb[i] = nb[i];
+                for (int c = 0; c < 3; ++c) rec.m[3 * i + c] = B[row[i]][c];
+            }
+            recs.row.push_back(rec);
+            recs.vol.push_back(m.vol[t]);
+            continue;
+        }
+        double B[4][3];
+        for (int c = 0; c < 3; ++c) {
+            for (int j = 1; j < 4; ++j) B[j][c] = D[(j - 1) + 3 * c];
+            B[0][c] = -B[1][c] - B[2][c] - B[3][c];
+        }
+        TetInc rec{};
+        for (int i = 0; i < 3; ++i) {
+            const double* r = B[row[i]];
+            rec.nb[i] = nb[i];
+            rec.w[i] = (float)(r[0] * B[ord][0] + r[1] * B[ord][1] + r[2] * B[ord][2]);
+        }
+        // d(6 A det F)/dx_v = +-(x_nb[1] - x_nb[0]) x (x_nb[2] - x_nb[0]): + for vertices 1 and 3
+        rec.c = (float)((ord % 2 ? 1.0 : -1.0) / (6.0 * (double)m.vol[t]));
+        rec.A = m.vol[t];
+        recs.inc.push_back(rec);
     }
-    slot.z = (int32_t)tinc.size();
+    slot.z = (int32_t)recs.size();
     const bool damping = m.mat.dampingHydrostatic != 0.f || m.mat.dampingDeviatoric != 0.f;
     slot.w = (damping ? SLOT_DAMPING : 0) | (mat << SLOT_MAT_SHIFT);
     if (refs) {
@@ -428,8 +458,8 @@ void emit_tet_slot(const TetMeshHost& m, int32_t off, int32_t lv, int32_t mat, s
     }
     slots.push_back(slot);
     // gather model: 72 B per vertex (slot, material, own position, previous position, inertia
-    // target, result) + 88 B per incident tet (48 B record, 4 B rest volume, 3 x 12 B neighbours)
-    work.push_back(72 + 88 * (int64_t)(slot.z - slot.y));
+    // target, result) + 68 B per incident tet (32 B record, 3 x 12 B neighbours; rows 52 B)
+    work.push_back(72 + (recs.rows ? 88 : 68) * (int64_t)(slot.z - slot.y));
 }
 
 // Colour-major cloth slot, face and bending records of one vertex.
@@ -510,8 +540,10 @@ void emit_cloth_slot(const ClothMeshHost& m, int32_t off, int32_t lv, bool inpla
 void upload_scene(gvbd_context* ctx, SceneObj& s, const std::function<void(size_t)>& reserve) {
     const int32_t G = (int32_t)s.groups.size();
     std::vector<int4> slots;
-    std::vector<TetInc> tinc;
-    std::vector<float> tvol;
+    TetRecords recs;
+    recs.rows = s.params.use_accelerator != 0;
+    for (const TetMeshHost& m : s.tets)
+        if (m.mat.dampingHydrostatic != 0.f || m.mat.dampingDeviatoric != 0.f) recs.rows = true;
     std::vector<ClothSlot> cslots;
     std::vector<FaceInc> cface;
     std::vector<BendInc> cbend;
@@ -614,7 +646,7 @@ void upload_scene(gvbd_context* ctx, SceneObj& s, const std::function<void(size_
             if (fixedMask[im][lv]) continue;
             const int32_t off = s.vertexOffset[im];
             if (s.meshes[im].first == MESH_TET) {
-                emit_tet_slot(s.tets[s.meshes[im].second], off, lv, s.meshes[im].second, slots, tinc, tvol,
+                emit_tet_slot(s.tets[s.meshes[im].second], off, lv, s.meshes[im].second, slots, recs,
                               tetWork, contact ? &trefs[im] : nullptr);
             } else {
                 // attachments read other vertices of the group: positionsNext keeps them Jacobi
@@ -737,8 +769,9 @@ void upload_scene(gvbd_context* ctx, SceneObj& s, const std::function<void(size_
     const size_t bV = align(sizeof(float4) * (size_t)std::max(nv, 1));
     const size_t bF = align((size_t)std::max(nv, 1));
     const size_t bS = align(sizeof(int4) * std::max<size_t>(slots.size(), 1));
-    const size_t bI = align(sizeof(TetInc) * std::max<size_t>(tinc.size(), 1));
-    const size_t bIV = align(sizeof(float) * std::max<size_t>(tvol.size(), 1));
+    const size_t bI = recs.rows ? 0 : align(sizeof(TetInc) * std::max<size_t>(recs.inc.size(), 1));
+    const size_t bRow = recs.rows ? align(sizeof(TetRow) * std::max<size_t>(recs.row.size(), 1)) : 0;
+    const size_t bVol = recs.rows ? align(sizeof(float) * std::max<size_t>(recs.vol.size(), 1)) : 0;
     std::vector<float4> tmat(std::max<size_t>(s.tets.size(), 1), make_float4(0.f, 0.f, 0.f, 0.f));
     for (size_t t = 0; t < s.tets.size(); ++t) {
         const auto& mt = s.tets[t].mat;
@@ -771,7 +804,7 @@ void upload_scene(gvbd_context* ctx, SceneObj& s, const std::function<void(size_
     const size_t bDP = dparams.empty() ? 0 : align(sizeof(DeformParams) * dparams.size());
     const size_t bAB = attBegin.empty() ? 0 : align(sizeof(int32_t) * attBegin.size());
     const size_t bAR = att.empty() ? 0 : align(sizeof(AttachRec) * att.size());
-    const size_t total = 6 * bV + bF + bS + bI + bIV + bTM + bCS + bCF + bCB + bFR + bER + bFr + bTF + bTE + bTC + 2 * bA + bW +
+    const size_t total = 6 * bV + bF + bS + bI + bRow + bVol + bTM + bCS + bCF + bCB + bFR + bER + bFr + bTF + bTE + bTC + 2 * bA + bW +
                          bClk + bZ + bDV + bDP + bAB + bAR + bSn + bVG;
     DeviceScene& d = s.dev;
     if (reserve) reserve(total);
@@ -797,8 +830,11 @@ void upload_scene(gvbd_context* ctx, SceneObj& s, const std::function<void(size_
     d.pnext = (float4*)take(bV);
     d.vflag = (uint8_t*)take(bF);
     d.slots = (int4*)take(bS);
-    d.tinc = (TetInc*)take(bI);
-    d.tvol = (float*)take(bIV);
+    if (bI) d.tinc = (TetInc*)take(bI);
+    if (bRow) {
+        d.trow = (TetRow*)take(bRow);
+        d.tvol = (float*)take(bVol);
+    }
     d.tmat = (float4*)take(bTM);
     d.cslots = (ClothSlot*)take(bCS);
     d.cface = (FaceInc*)take(bCF);
@@ -839,8 +875,9 @@ void upload_scene(gvbd_context* ctx, SceneObj& s, const std::function<void(size_
     up(d.vparam, vparam.data(), sizeof(float4) * nv);
     up(d.vflag, vflag.data(), nv);
     up(d.slots, slots.data(), sizeof(int4) * slots.size());
-    up(d.tinc, tinc.data(), sizeof(TetInc) * tinc.size());
-    up(d.tvol, tvol.data(), sizeof(float) * tvol.size());
+    up(d.tinc, recs.inc.data(), sizeof(TetInc) * recs.inc.size());
+    up(d.trow, recs.row.data(), sizeof(TetRow) * recs.row.size());
+    up(d.tvol, recs.vol.data(), sizeof(float) * recs.vol.size());
     up(d.tmat, tmat.data(), sizeof(float4) * tmat.size());
     up(d.cslots, cslots.data(), sizeof(ClothSlot) * cslots.size());
     up(d.cface, cface.data(), sizeof(FaceInc) * cface.size());
@@ -883,6 +920,7 @@ void upload_scene(gvbd_context* ctx, SceneObj& s, const std::function<void(size_
     v.vflag = d.vflag;
     v.slots = d.slots;
     v.tinc = d.tinc;
+    v.trow = d.trow;
     v.tvol = d.tvol;
     v.tmat = d.tmat;
     v.pnext = d.pnext;
@@ -3041,14 +3079,14 @@ static void rebase_scene(SceneObj& s, uintptr_t from, uintptr_t to) {
     };
     DeviceScene& d = s.dev;
     mv(d.pos), mv(d.prev), mv(d.inertia), mv(d.vel), mv(d.vparam), mv(d.pnext), mv(d.vflag), mv(d.slots);
-    mv(d.tinc), mv(d.tvol), mv(d.tmat), mv(d.cslots), mv(d.cface), mv(d.cbend), mv(d.faceRef), mv(d.edgeRef);
+    mv(d.tinc), mv(d.trow), mv(d.tvol), mv(d.tmat), mv(d.cslots), mv(d.cface), mv(d.cbend), mv(d.faceRef), mv(d.edgeRef);
     mv(d.friction);
     mv(d.tFaceRef), mv(d.tEdgeRef), mv(d.tcontact), mv(d.accPrevPrev), mv(d.accPrevIter), mv(d.accOmega);
     mv(d.snap), mv(d.vgroup);
     mv(d.clock), mv(d.vzone), mv(d.dverts), mv(d.dparams), mv(d.attBegin), mv(d.att);
     SceneView& v = s.view;
     mv(v.pos), mv(v.prev), mv(v.inertia), mv(v.vel), mv(v.vparam), mv(v.vflag), mv(v.slots), mv(v.tinc);
-    mv(v.tvol), mv(v.tmat);
+    mv(v.trow), mv(v.tvol), mv(v.tmat);
     mv(v.pnext), mv(v.cslots), mv(v.cface), mv(v.cbend), mv(v.tcontact), mv(v.accPrevPrev), mv(v.accPrevIter);
     mv(v.accOmega), mv(v.clock), mv(v.vzone), mv(v.dverts), mv(v.dparams), mv(v.attBegin), mv(v.att);
     mv(v.solveFail);

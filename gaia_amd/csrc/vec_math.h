@@ -50,4 +50,40 @@ __device__ __forceinline__ bool solve_sym3(const Sym3& h, f3 b, f3& x) {
     return isfinite(x.x) && isfinite(x.y) && isfinite(x.z);
 }
 
+// Force and Hessian parts of one incident tet (TetInc) on its vertex at x, the others at p0..p2:
+// F m_v, g = cof(F) m_v, det F and |m_v|^2.
+struct TetTerms {
+    f3 Fm, g;
+    float J, mm;
+};
+__device__ __forceinline__ TetTerms tet_terms(f3 x, f3 p0, f3 p1, f3 p2, float c, float w0, float w1, float w2) {
+    const f3 d0 = p0 - x;
+    TetTerms t;
+    t.Fm = w0 * d0 + w1 * (p1 - x) + w2 * (p2 - x);
+    t.g = c * cross(p1 - p0, p2 - p0);
+    t.J = -dot(t.g, d0);
+    t.mm = -(w0 + w1 + w2);
+    return t;
+}
+
+// The same by the shape-matrix rows m0..m2 (TetRow).
+__device__ __forceinline__ TetTerms tet_terms_rows(f3 x, f3 p0, f3 p1, f3 p2, f3 m0, f3 m1, f3 m2) {
+    const f3 d0 = p0 - x, d1 = p1 - x, d2 = p2 - x;
+    // F columns: F e_c = sum_k d_k m_k[c]
+    const f3 c0 = m0.x * d0 + m1.x * d1 + m2.x * d2;
+    const f3 c1 = m0.y * d0 + m1.y * d1 + m2.y * d2;
+    const f3 c2 = m0.z * d0 + m1.z * d1 + m2.z * d2;
+    const f3 mv = mk(-(m0.x + m1.x + m2.x), -(m0.y + m1.y + m2.y), -(m0.z + m1.z + m2.z));
+    // cof(F) columns are c1 x c2, c2 x c0, c0 x c1
+    const f3 k0 = cross(c1, c2);
+    const f3 k1 = cross(c2, c0);
+    const f3 k2 = cross(c0, c1);
+    TetTerms t;
+    t.J = dot(c0, k0);
+    t.g = mv.x * k0 + mv.y * k1 + mv.z * k2;
+    t.Fm = mv.x * c0 + mv.y * c1 + mv.z * c2;
+    t.mm = dot(mv, mv);
+    return t;
+}
+
 }  // namespace gvbd
