@@ -2164,7 +2164,8 @@ void ContactDetector::finalize() {
     eeStored_ = dalloc<int>(ne_);
     eeOverflow_ = dalloc<int>(ne_);
     vfRec_ = dalloc<VFContactRec>((size_t)nv_ * vfCap_);
-    eeRec_ = dalloc<EEContactRec>((size_t)ne_ * eeCap_);
+    // penetration contact has no edge queries: no edge tree and no edge lists
+    eeRec_ = dalloc<EEContactRec>(pen_ ? 1 : (size_t)ne_ * eeCap_);
     vfOffset_ = dalloc<int64_t>(nv_ + 1);
     eeOffset_ = dalloc<int64_t>(ne_ + 1);
     error_ = dalloc<int>(64);
@@ -2195,9 +2196,9 @@ void ContactDetector::finalize() {
         vSortTemp_ = dalloc<char>(vSortTempBytes_);
     }
     // BVH storage
-    allocBuildScratch({nf_, ne_, pen_ ? (int)penHost_.tetMesh.size() : 0});
+    allocBuildScratch({nf_, pen_ ? (int)penHost_.tetMesh.size() : ne_});
     allocBvh(fb_, nf_, !pen_);
-    allocBvh(eb_, ne_, !pen_);
+    allocBvh(eb_, pen_ ? 0 : ne_, true);
     if (pen_ && nf_ > 0) fb_.mesh = dalloc<int>(2 * (size_t)nf_ - 1);
     if (pen_) setupPenetrationDevice();
     hip_check(hipStreamSynchronize(stream_), "detector upload sync");
