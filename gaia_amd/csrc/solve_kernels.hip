@@ -37,11 +37,60 @@ namespace gvbd {
 
 namespace {
 
+// A lane's value read by a fixed permutation within its row of 16 lanes: a register move, where
+// __shfl goes through the LDS crossbar with its latency in the solve's serial chain.
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+constexpr int kDppXor1 = 0xB1;         // quad_perm [1, 0, 3, 2]
+constexpr int kDppXor2 = 0x4E;         // quad_perm [2, 3, 0, 1]
+constexpr int kDppXor3 = 0x1B;         // quad_perm [3, 2, 1, 0]
+constexpr int kDppHalfMirror = 0x141;  // lane i of 8 reads 7 - i: xor 7
+constexpr int kDppRor4 = 0x124;        // row rotations by 4 and 8
+constexpr int kDppRor8 = 0x128;
+
+// Sum over the LPV lanes of a vertex (every lane gets it): a butterfly at distances LPV / 2 .. 1.
+// After the exchange at distance 8 lanes i and i ^ 8 hold the same sum, so a rotation by 4 serves as
+// the exchange at distance 4. All lanes of the wave call this.
 template <int LPV>
 __device__ __forceinline__ float lane_sum(float v) {
-#pragma unroll
-    for (int o = LPV / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    if (LPV == 16) {
+        v += dpp<kDppRor8>(v);
+        v += dpp<kDppRor4>(v);
+    }
+    if (LPV == 8) v += dpp<kDppXor3>(dpp<kDppHalfMirror>(v));
+    if (LPV > 2) v += dpp<kDppXor2>(v);
+    if (LPV > 1) v += dpp<kDppXor1>(v);
     return v;
+}
+
+// Per-vertex loads of the solve's tail, issued with its first ones: the lanes of a vertex hold one
+// of a, b and c each (one register quad for all of them), and lane 0 reads the others' after the
+// lane sums. What too few lanes are there for is loaded when it is needed.
+template <int LPV, int N>
+struct TailLoads {
+    float4 own;
+    __device__ __forceinline__ TailLoads(const float4* a, const float4* b, const float4* c, int v, bool active) {
+        own = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (LPV == 1 || !active) return;
+        const int k = threadIdx.x & 3;
+        const float4* p = k & 1 ? b : a;
+        if (LPV >= 4 && N > 2 && k == 2) p = c;
+        own = p[v];
+    }
+    template <int CTRL>
+    __device__ __forceinline__ float4 move() const {
+        return make_float4(dpp<CTRL>(own.x), dpp<CTRL>(own.y), dpp<CTRL>(own.z), dpp<CTRL>(own.w));
+    }
+};
+
+// The value as if it were loaded here: its uses stay after this point. (Products of values known
+// earlier are hoisted over the branches in between and no longer fuse with the sums they go into,
+// which changes the rounding of the result.)
+__device__ __forceinline__ float4 loaded_here(float4 t) {
+    asm volatile("" : "+v"(t.x), "+v"(t.y), "+v"(t.z), "+v"(t.w));
+    return t;
 }
 
 // Plane-ground boundary penalty and IPC-mollified friction for one vertex
@@ -68,7 +117,10 @@ __device__ __forceinline__ void boundary_force(const SolveParams& sp, float k, f
         if (applyFriction) {
             const int d1 = (d + 1) % 3, d2 = (d + 2) % 3;
             const float u0 = dxs[d1], u1 = dxs[d2];
-            const float uNorm = sqrtf(u0 * u0 + u1 * u1);
+            // (which square is rounded before the sum is fixed here, not left to the compiler: a last bit
+            // of it is seen many frames later)
+            const float lo = d1 < d2 ? u0 : u1, hi = d1 < d2 ? u1 : u0;
+            const float uNorm = sqrtf(fmaf(lo, lo, hi * hi));
             if (uNorm > 0.f) {
                 const float f1 = uNorm > frictionEpsU ? 1.0f / uNorm : (-uNorm / frictionEpsU + 2.0f) / frictionEpsU;
                 const float lambda = pen * k;
@@ -164,6 +216,7 @@ __device__ __forceinline__ void tet_block(const SceneView& S, const WorkItem& it
 
     f3 x = mk(0.f, 0.f, 0.f);
     if (active) x = xyz(S.pos[v]);
+    const TailLoads<LPV, 2> tail(S.prev, S.inertia, nullptr, v, active);
 
     float f0 = 0.f, f1 = 0.f, f2 = 0.f;
     float gxx = 0.f, gxy = 0.f, gxz = 0.f, gyy = 0.f, gyz = 0.f, gzz = 0.f;
@@ -239,10 +292,11 @@ __device__ __forceinline__ void tet_block(const SceneView& S, const WorkItem& it
         }
         lane_sum_contact<LPV>(cf, ch);
     }
+    const float4 tail1 = tail.template move<kDppXor1>();
     if (!active || sub != 0) return;
 
     const SolveParams& sp = S.sp;
-    const f3 xp = xyz(S.prev[v]);
+    const f3 xp = xyz(LPV > 1 ? loaded_here(tail.own) : S.prev[v]);
     f3 f = mk(f0, f1, f2);
     Sym3 h{gxx + cmu, gxy, gxz, gyy + cmu, gyz, gzz + cmu};
     if (slot.w & SLOT_DAMPING) {
@@ -255,7 +309,7 @@ __device__ __forceinline__ void tet_block(const SceneView& S, const WorkItem& it
         h.yy += dh.yy; h.yz += dh.yz; h.zz += dh.zz;
     }
     // inertia
-    const float4 yv = S.inertia[v];
+    const float4 yv = LPV > 1 ? loaded_here(tail1) : S.inertia[v];
     const float mass = yv.w;
     f.x += mass * (yv.x - x.x) * sp.dtSqrRecip;
     f.y += mass * (yv.y - x.y) * sp.dtSqrRecip;
@@ -277,7 +331,7 @@ __device__ __forceinline__ void tet_block(const SceneView& S, const WorkItem& it
     if (moved) {
         f3 dx;
         float step = sp.stepSize;
-        if (!solve_sym3(h, f, dx)) {
+        if (!solve_sym3<false>(h, f, dx)) {
             // the 3x3 block is singular: gradient step (VBDPhysics.cpp:2449-2466), counted
             step = sp.stepSizeGD;
             dx = f;
@@ -666,6 +720,7 @@ __device__ __forceinline__ void cloth_block(const SceneView& S, const WorkItem& 
     const int v = sa.x;
     f3 x = mk(0.f, 0.f, 0.f);
     if (active) x = xyz(S.pos[v]);
+    const TailLoads<LPV, 3> tail(S.prev, S.inertia, S.vparam, v, active);
 
     const float4* __restrict__ pos = S.pos;
     int4 first = make_int4(0, 0, 0, 0), last = make_int4(0, 0, 0, 0);
@@ -755,12 +810,13 @@ __device__ __forceinline__ void cloth_block(const SceneView& S, const WorkItem& 
         if (active) contact_forces<LPV>(S, v, sub, S.cv.faceRef, sa.y, sa.z, S.cv.edgeRef, sb.z, sb.w, cf, ch);
         lane_sum_contact<LPV>(cf, ch);
     }
+    const float4 tail1 = tail.template move<kDppXor1>(), tail2 = tail.template move<kDppXor2>();
     if (!active || sub != 0) return;
 
     const SolveParams& sp = S.sp;
-    const f3 xp = xyz(S.prev[v]);
+    const f3 xp = xyz(LPV > 1 ? loaded_here(tail.own) : S.prev[v]);
     const f3 disp = x - xp;
-    const float4 vp = S.vparam[v];  // (exp damping, const damping, StVK damping, bending damping)
+    const float4 vp = LPV > 2 ? loaded_here(tail2) : S.vparam[v];  // (exp damping, const damping, StVK damping, bending damping)
     // membrane + its damping (VBDTriMeshStVK.cpp:904-909): dampingH = H_membrane * gamma / dt
     const float cs = vp.z / sp.dt;
     Sym3 hm{hxx, hxy, hxz, hyy, hyz, hzz};
@@ -774,7 +830,7 @@ __device__ __forceinline__ void cloth_block(const SceneView& S, const WorkItem& 
     h.yy += hbd;
     h.zz += hbd;
     // inertia
-    const float4 yv = S.inertia[v];
+    const float4 yv = LPV > 1 ? loaded_here(tail1) : S.inertia[v];
     const float mass = yv.w;
     f.x += mass * (yv.x - x.x) * sp.dtSqrRecip;
     f.y += mass * (yv.y - x.y) * sp.dtSqrRecip;
@@ -806,7 +862,7 @@ __device__ __forceinline__ void cloth_block(const SceneView& S, const WorkItem& 
     }
     f3 dx;
     f3 xn = x;
-    const bool solved = solve_sym3(h, f, dx);
+    const bool solved = solve_sym3<true>(h, f, dx);
     if (!solved) atomicAdd(S.solveFail, 1);  // singular block: the vertex keeps its position, counted
     if (solved) {
         xn = x + sp.clothStepSize * dx;
@@ -834,9 +890,9 @@ __device__ __forceinline__ void cloth_block(const SceneView& S, const WorkItem& 
 // STAGE > 0 stages the incidence records through LDS, 2 * STAGE records of 32 bytes (or STAGE of 48)
 // per chunk.
 // CONTACT selects the variant for scenes with collision handling (contact forces, bound
-// truncation); the others carry none of that code, so their register use is unchanged by it.
+// truncation); the others carry none of that code and are kept to 64 registers (8 waves per SIMD).
 template <int LPV, int BLOCK, int STAGE, bool CONTACT>
-__global__ __launch_bounds__(BLOCK) void group_solve_kernel(const SceneView* __restrict__ scenes,
+__global__ __launch_bounds__(BLOCK, CONTACT ? 1 : 8) void group_solve_kernel(const SceneView* __restrict__ scenes,
                                                            const WorkItem* __restrict__ items, int iteration,
                                                            int xcdBlocks) {
     __shared__ float4 lds[STAGE > 0 ? 4 * STAGE : 1];
