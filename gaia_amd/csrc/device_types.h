@@ -277,6 +277,18 @@ struct WorkItem {
     int32_t kind;
 };
 
+// A scene stepped whole by one block: one iteration is its `count` items from `first`.
+struct SceneRun {
+    int32_t scene;
+    int32_t first;
+    int32_t count;
+    int32_t pad;
+};
+
+// Set in WorkItem::scene of a SceneRun's item: the last of its parallel group. A WORK_COMMIT item's slots
+// are cloth slots of the group solved through positionsNext.
+enum : int32_t { RUN_GROUP_END = 1 };
+
 // Entry of the flattened (scene, colour, vertex-chunk) work queue of one iteration.
 // kind: WORK_TET / WORK_CLOTH solve chunk, or WORK_COMMIT (pnext -> pos for the cloth
 // slots of one scene colour). The entry may start once `need` earlier entries of its

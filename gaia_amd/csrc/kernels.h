@@ -69,6 +69,13 @@ hipError_t convergence_scratch_init(int device, double** scratch);
 hipError_t launch_convergence_final_sum(const double* partial, int off0, int n0, int off1, int n1, int off2, int n2,
                                         double* out, hipStream_t stream);
 
+// Whole frames (substeps x (initial step, iterations x groups, velocities)) of `nruns` scenes, one
+// block per scene with its positions in LDS: scenes of at most `maxVerts` <= kRunVerts vertices,
+// without deformers and collision handling.
+constexpr int kRunVerts = 4096;
+constexpr int kRunBlock = 1024;
+hipError_t launch_scene_frames(const SceneView* scenes, const SceneRun* runs, int nruns, const WorkItem* items,
+                               int maxVerts, int substeps, int iterations, int lpv, hipStream_t stream);
 // snap[i] = pos[i] with the int bits of vgroup[i] in w (ContactView::snap).
 hipError_t launch_contact_snapshot(const float4* pos, const int* vgroup, float4* snap, int n, hipStream_t stream);
 // dst[i] = src[i] for n float4 elements (bandwidth / profiler calibration).

@@ -204,25 +204,30 @@ __device__ __forceinline__ void lane_sum_contact(f3& f, Sym3& h) {
 // ---------------------------------------------------------------------------
 // Tet vertex block (VBDPhysics.cpp:2402-2483)
 // ---------------------------------------------------------------------------
+// The slot of the vertex that this thread's lanes solve in a work item (zeros beyond the item).
+template <int LPV>
+__device__ __forceinline__ int4 tet_slot(const SceneView& S, const WorkItem& it) {
+    const int local = threadIdx.x / LPV;
+    return local < it.count ? S.slots[it.slotBegin + local] : make_int4(0, 0, 0, 0);
+}
+
 template <int LPV, int STAGE, bool CONTACT>
-__device__ __forceinline__ void tet_block(const SceneView& S, const WorkItem& it, int iteration, float4* lds) {
+__device__ __forceinline__ void tet_block(const SceneView& S, float4* posInOut, const int4& slot, const WorkItem& it,
+                                          int iteration, float4* lds) {
     const int local = threadIdx.x / LPV;
     const int sub = threadIdx.x % LPV;
     const bool active = local < it.count;
-
-    int4 slot = make_int4(0, 0, 0, 0);
-    if (active) slot = S.slots[it.slotBegin + local];
     const int v = slot.x;
 
     f3 x = mk(0.f, 0.f, 0.f);
-    if (active) x = xyz(S.pos[v]);
+    if (active) x = xyz(posInOut[v]);
     const TailLoads<LPV, 2> tail(S.prev, S.inertia, nullptr, v, active);
 
     float f0 = 0.f, f1 = 0.f, f2 = 0.f;
     float gxx = 0.f, gxy = 0.f, gxz = 0.f, gyy = 0.f, gyz = 0.f, gzz = 0.f;
     float cmu = 0.f;
 
-    const float4* __restrict__ pos = S.pos;
+    const float4* __restrict__ pos = posInOut;
     int blockBegin = 0, blockEnd = 0;
     if (STAGE > 0) {
         blockBegin = S.slots[it.slotBegin].y;
@@ -352,7 +357,7 @@ __device__ __forceinline__ void tet_block(const SceneView& S, const WorkItem& it
             atomicOr(S.cv.flag, 1);
         }
     }
-    if (CONTACT || moved) S.pos[v] = make_float4(xn.x, xn.y, xn.z, 0.f);
+    if (CONTACT || moved) posInOut[v] = make_float4(xn.x, xn.y, xn.z, 0.f);
 }
 
 // ---------------------------------------------------------------------------
@@ -705,24 +710,27 @@ __device__ void contact_forces(const SceneView& S, int v, int sub, const int* fa
 // ---------------------------------------------------------------------------
 // Cloth vertex block (VBDClothPhysics.cpp:1026-1154)
 // ---------------------------------------------------------------------------
+template <int LPV>
+__device__ __forceinline__ ClothSlot cloth_slot(const SceneView& S, const WorkItem& it) {
+    const int local = threadIdx.x / LPV;
+    ClothSlot s{make_int4(0, 0, 0, 0), make_int4(0, 0, 0, 0)};
+    if (local < it.count) s = S.cslots[it.slotBegin + local];
+    return s;
+}
+
 template <int LPV, int STAGE, bool CONTACT>
-__device__ __forceinline__ void cloth_block(const SceneView& S, const WorkItem& it, float4* lds) {
+__device__ __forceinline__ void cloth_block(const SceneView& S, float4* posInOut, float4* pnext, const ClothSlot& slot,
+                                            const WorkItem& it, float4* lds) {
     const int local = threadIdx.x / LPV;
     const int sub = threadIdx.x % LPV;
     const bool active = local < it.count;
-
-    int4 sa = make_int4(0, 0, 0, 0), sb = make_int4(0, 0, 0, 0);
-    if (active) {
-        const ClothSlot cs = S.cslots[it.slotBegin + local];
-        sa = cs.a;
-        sb = cs.b;
-    }
+    const int4 sa = slot.a, sb = slot.b;
     const int v = sa.x;
     f3 x = mk(0.f, 0.f, 0.f);
-    if (active) x = xyz(S.pos[v]);
+    if (active) x = xyz(posInOut[v]);
     const TailLoads<LPV, 3> tail(S.prev, S.inertia, S.vparam, v, active);
 
-    const float4* __restrict__ pos = S.pos;
+    const float4* __restrict__ pos = posInOut;
     int4 first = make_int4(0, 0, 0, 0), last = make_int4(0, 0, 0, 0);
     if (STAGE > 0) {
         const ClothSlot c0 = S.cslots[it.slotBegin], c1 = S.cslots[it.slotBegin + it.count - 1];
@@ -849,10 +857,10 @@ __device__ __forceinline__ void cloth_block(const SceneView& S, const WorkItem& 
         // vertex attachments (VBDClothPhysics.cpp:1465-1498)
         for (int r = S.attBegin[v]; r < S.attBegin[v + 1]; ++r) {
             const AttachRec A = S.att[r];
-            const f3 xr = xyz(S.pos[A.ids.w]);
+            const f3 xr = xyz(posInOut[A.ids.w]);
             f3 tgt = mk(A.p.x, A.p.y, A.p.z);
             if (A.ids.x >= 0)
-                tgt = A.p.x * xyz(S.pos[A.ids.x]) + A.p.y * xyz(S.pos[A.ids.y]) + A.p.z * xyz(S.pos[A.ids.z]);
+                tgt = A.p.x * xyz(posInOut[A.ids.x]) + A.p.y * xyz(posInOut[A.ids.y]) + A.p.z * xyz(posInOut[A.ids.z]);
             f = f - A.p.w * (xr - tgt);
             const float hk = A.p.w * A.b;
             h.xx += hk;
@@ -879,7 +887,7 @@ __device__ __forceinline__ void cloth_block(const SceneView& S, const WorkItem& 
             }
         }
     }
-    float4* dst = (sa.w & SLOT_INPLACE) ? S.pos : S.pnext;
+    float4* dst = (sa.w & SLOT_INPLACE) ? posInOut : pnext;
     dst[v] = make_float4(xn.x, xn.y, xn.z, 0.f);
 }
 
@@ -900,9 +908,9 @@ __global__ __launch_bounds__(BLOCK, CONTACT ? 1 : 8) void group_solve_kernel(con
         items[xcdBlocks == 0 ? (int)blockIdx.x : (xcdBlocks == 1 ? xcd_block_index() : xcd_chunk_index(xcdBlocks))];
     const SceneView& S = scenes[it.scene];
     if (it.kind == WORK_TET)
-        tet_block<LPV, STAGE, CONTACT>(S, it, iteration, lds);
+        tet_block<LPV, STAGE, CONTACT>(S, S.pos, tet_slot<LPV>(S, it), it, iteration, lds);
     else
-        cloth_block<LPV, STAGE, CONTACT>(S, it, lds);
+        cloth_block<LPV, STAGE, CONTACT>(S, S.pos, S.pnext, cloth_slot<LPV>(S, it), it, lds);
 }
 
 // After a group's cloth solves: x = positionsNext for the group's cloth vertices
@@ -988,9 +996,9 @@ __global__ __launch_bounds__(BLOCK) void queue_solve_kernel(const SceneView* __r
             for (int p = 0; p < e.count; p += VPB) {
                 const WorkItem it{e.scene, e.slotBegin + p, min(VPB, e.count - p), e.kind};
                 if (e.kind == WORK_TET)
-                    tet_block<LPV, 0, false>(S, it, iteration, nullptr);
+                    tet_block<LPV, 0, false>(S, S.pos, tet_slot<LPV>(S, it), it, iteration, nullptr);
                 else
-                    cloth_block<LPV, 0, false>(S, it, nullptr);
+                    cloth_block<LPV, 0, false>(S, S.pos, S.pnext, cloth_slot<LPV>(S, it), it, nullptr);
             }
         }
         // every thread's stores happen before lane 0's agent-scope release (the completion count
@@ -1024,15 +1032,9 @@ __global__ __launch_bounds__(256) void contact_snapshot_kernel(const float4* __r
 // VBDBaseTriMesh.cpp:163-178; the per-vertex initialisation code is
 // 0: x = y, 1: keep x, 2: x + dt v_prev, 3: (x + y)/2, 4: x + dt v_prev + dt^2 r g,
 // 5: x + (y - x) shortened to the vertex's conservative bound (cloth type 3).
-__global__ __launch_bounds__(256) void initial_step_kernel(const SceneView* __restrict__ scenes,
-                                                           const WorkItem* __restrict__ items) {
-    const WorkItem it = items[blockIdx.x];
-    const int i = threadIdx.x;
-    if (i >= it.count) return;
-    const SceneView& S = scenes[it.scene];
+__device__ __forceinline__ void initial_step(const SceneView& S, float4* pos, int v) {
     const SolveParams& sp = S.sp;
-    const int v = it.slotBegin + i;
-    const float4 p = S.pos[v];
+    const float4 p = pos[v];
     const float4 vel = S.vel[v];
     const uint8_t flag = S.vflag[v];
     const float dt = sp.dt;
@@ -1072,8 +1074,15 @@ __global__ __launch_bounds__(256) void initial_step_kernel(const SceneView* __re
     }
     default: xn = x; break;
     }
-    S.pos[v] = make_float4(xn.x, xn.y, xn.z, 0.f);
+    pos[v] = make_float4(xn.x, xn.y, xn.z, 0.f);
     S.vel[v] = make_float4(vn.x, vn.y, vn.z, 0.f);
+}
+
+__global__ __launch_bounds__(256) void initial_step_kernel(const SceneView* __restrict__ scenes,
+                                                           const WorkItem* __restrict__ items) {
+    const WorkItem it = items[blockIdx.x];
+    const SceneView& S = scenes[it.scene];
+    if ((int)threadIdx.x < it.count) initial_step(S, S.pos, it.slotBegin + threadIdx.x);
 }
 
 // Deformers (VBD/VBDDeformer.h:45-178, VBDCloth/VBDClothDeformer.h:44-196). Items cover one
@@ -1127,53 +1136,47 @@ __global__ __launch_bounds__(256) void deform_kernel(const SceneView* __restrict
 
 // Chebyshev acceleration (runStepGPU, VBDPhysics.cpp:872-906): after the initial step both
 // history buffers take the current positions (recordInitialPositionForAccelerator, :3577-3592).
+__device__ __forceinline__ void accel_init(const SceneView& S, const float4* pos, int v) {
+    if (!S.accOmega || !(S.vflag[v] & VFLAG_ACCEL)) return;
+    const float4 p = pos[v];
+    S.accPrevPrev[v] = p;
+    S.accPrevIter[v] = p;
+}
+
 __global__ __launch_bounds__(256) void accel_init_kernel(const SceneView* __restrict__ scenes,
                                                          const WorkItem* __restrict__ items) {
     const WorkItem it = items[blockIdx.x];
-    const int i = threadIdx.x;
-    if (i >= it.count) return;
     const SceneView& S = scenes[it.scene];
-    if (!S.accOmega) return;
-    const int v = it.slotBegin + i;
-    if (!(S.vflag[v] & VFLAG_ACCEL)) return;
-    const float4 p = S.pos[v];
-    S.accPrevPrev[v] = p;
-    S.accPrevIter[v] = p;
+    if ((int)threadIdx.x < it.count) accel_init(S, S.pos, it.slotBegin + threadIdx.x);
 }
 
 // After iteration k's sweep (VBDSolveParallelGroup_applyAcceleration_kernel,
 // VBDPhysicsCompute.cu:910-944): x <- y_{k-1} + omega_k (x - y_{k-1}); y_{k-1} <- y_k (the positions
 // before this sweep); and the accelerated positions become the next sweep's y_k
 // (recordPrevIterPositionsAccelerator, VBDPhysics.cpp:3594-3606). Fixed vertices are left alone.
-__global__ __launch_bounds__(256) void accel_apply_kernel(const SceneView* __restrict__ scenes,
-                                                          const WorkItem* __restrict__ items, int iteration) {
-    const WorkItem it = items[blockIdx.x];
-    const int i = threadIdx.x;
-    if (i >= it.count) return;
-    const SceneView& S = scenes[it.scene];
+__device__ __forceinline__ void accel_apply(const SceneView& S, float4* pos, int v, int iteration) {
     if (!S.accOmega) return;
-    const int v = it.slotBegin + i;
     const uint8_t flag = S.vflag[v];
     if (!(flag & VFLAG_ACCEL) || (flag & VFLAG_FIXED)) return;
     const float omega = S.accOmega[iteration];
-    const f3 x = xyz(S.pos[v]);
+    const f3 x = xyz(pos[v]);
     const f3 pp = xyz(S.accPrevPrev[v]);
     const f3 xn = pp + omega * (x - pp);
-    S.pos[v] = make_float4(xn.x, xn.y, xn.z, 0.f);
+    pos[v] = make_float4(xn.x, xn.y, xn.z, 0.f);
     S.accPrevPrev[v] = S.accPrevIter[v];
     S.accPrevIter[v] = make_float4(xn.x, xn.y, xn.z, 0.f);
 }
 
-// VBDPhysics.cpp:2486-2561 updateVelocities + dampVelocities (cloth: VBDClothPhysics.cpp:2318-2360).
-__global__ __launch_bounds__(256) void update_velocity_kernel(const SceneView* __restrict__ scenes,
-                                                              const WorkItem* __restrict__ items) {
+__global__ __launch_bounds__(256) void accel_apply_kernel(const SceneView* __restrict__ scenes,
+                                                          const WorkItem* __restrict__ items, int iteration) {
     const WorkItem it = items[blockIdx.x];
-    const int i = threadIdx.x;
-    if (i >= it.count) return;
     const SceneView& S = scenes[it.scene];
-    const int v = it.slotBegin + i;
+    if ((int)threadIdx.x < it.count) accel_apply(S, S.pos, it.slotBegin + threadIdx.x, iteration);
+}
+
+// VBDPhysics.cpp:2486-2561 updateVelocities + dampVelocities (cloth: VBDClothPhysics.cpp:2318-2360).
+__device__ __forceinline__ void update_velocity(const SceneView& S, const float4& p, int v) {
     const float dt = S.sp.dt;
-    const float4 p = S.pos[v];
     const float4 q = S.prev[v];
     f3 vel = mk((p.x - q.x) / dt, (p.y - q.y) / dt, (p.z - q.z) / dt);
     const float vMag = sqrtf(dot(vel, vel));
@@ -1198,6 +1201,83 @@ __global__ __launch_bounds__(256) void update_velocity_kernel(const SceneView* _
     }
     if (flags & VFLAG_FIXED) vel = mk(0.f, 0.f, 0.f);
     S.vel[v] = make_float4(vel.x, vel.y, vel.z, 0.f);
+}
+
+__global__ __launch_bounds__(256) void update_velocity_kernel(const SceneView* __restrict__ scenes,
+                                                              const WorkItem* __restrict__ items) {
+    const WorkItem it = items[blockIdx.x];
+    const SceneView& S = scenes[it.scene];
+    const int v = it.slotBegin + threadIdx.x;
+    if ((int)threadIdx.x < it.count) update_velocity(S, S.pos[v], v);
+}
+
+// Barrier of a block for its LDS accesses alone: loads and stores of global memory stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Whole frames of small scenes, one block per scene: every substep's initial step, iterations x
+// parallel groups and velocity update, with a block barrier where the launches of the other
+// schedules order the work. The same vertex solves in the same order, so the same results.
+// A launch per parallel group costs about 4 us however few vertices it has (2 us of launch and a
+// chain of six dependent loads from cold caches). Here the positions stay in LDS, the next item's
+// slots are loaded during the current item, and a group costs its records' latency, its arithmetic
+// and an LDS barrier: us per frame of 125 / 1,331 tet vertices 332 / 431 -> 226 / 255 (positions in
+// HBM and full barriers: 295 / 380), of 576 cloth vertices 414 -> 291, 4 lanes per vertex.
+template <int LPV, int BLOCK>
+__global__ __launch_bounds__(BLOCK) void scene_frame_kernel(const SceneView* __restrict__ scenes,
+                                                            const SceneRun* __restrict__ runs,
+                                                            const WorkItem* __restrict__ items, int substeps,
+                                                            int iterations) {
+    extern __shared__ float4 pos[];
+    const SceneRun run = runs[blockIdx.x];
+    const SceneView& S = scenes[run.scene];
+    const int tid = threadIdx.x, nv = S.nv;
+    const WorkItem* __restrict__ list = items + run.first;
+    const auto load_slot = [&](const WorkItem& it) {
+        if (it.kind == WORK_CLOTH) return cloth_slot<LPV>(S, it);
+        ClothSlot s{make_int4(0, 0, 0, 0), make_int4(0, 0, 0, 0)};
+        if (it.kind == WORK_TET) s.a = tet_slot<LPV>(S, it);
+        return s;
+    };
+    for (int v = tid; v < nv; v += BLOCK) pos[v] = S.pos[v];
+    for (int sub = 0; sub < substeps; ++sub) {
+        for (int v = tid; v < nv; v += BLOCK) {  // a vertex's LDS entry is this thread's own so far
+            initial_step(S, pos, v);
+            accel_init(S, pos, v);
+        }
+        __syncthreads();
+        WorkItem it = list[0];
+        ClothSlot slot = load_slot(it);
+        for (int iter = 0; iter < iterations; ++iter) {
+            for (int k = 0; k < run.count; ++k) {
+                const WorkItem next = list[k + 1 < run.count ? k + 1 : 0];
+                const ClothSlot nextSlot = load_slot(next);
+                if (it.kind == WORK_TET) {
+                    tet_block<LPV, 0, false>(S, pos, slot.a, it, iter, nullptr);
+                } else if (it.kind == WORK_CLOTH) {
+                    cloth_block<LPV, 0, false>(S, pos, S.pnext, slot, it, nullptr);
+                } else {
+                    __syncthreads();  // the solves' stores to positionsNext
+                    for (int i = tid; i < it.count; i += BLOCK) {
+                        const int v = S.cslots[it.slotBegin + i].a.x;
+                        pos[v] = S.pnext[v];
+                    }
+                }
+                if (it.scene & RUN_GROUP_END) lds_barrier();
+                it = next;
+                slot = nextSlot;
+            }
+            if (S.accOmega) {
+                for (int v = tid; v < nv; v += BLOCK) accel_apply(S, pos, v, iter);
+                lds_barrier();
+            }
+        }
+        for (int v = tid; v < nv; v += BLOCK) update_velocity(S, pos[v], v);
+    }
+    for (int v = tid; v < nv; v += BLOCK) S.pos[v] = pos[v];
 }
 
 // ---------------------------------------------------------------------------
@@ -1287,6 +1367,21 @@ int queue_blocks_per_cu(int lpv, int block) {
     GVBD_SCHEDULES(GVBD_CASE)
 #undef GVBD_CASE
     return 1;
+}
+
+hipError_t launch_scene_frames(const SceneView* scenes, const SceneRun* runs, int nruns, const WorkItem* items,
+                               int maxVerts, int substeps, int iterations, int lpv, hipStream_t stream) {
+    if (nruns <= 0) return hipSuccess;
+    if (maxVerts > kRunVerts) return hipErrorInvalidValue;
+#define GVBD_CASE(L)                                                                                           \
+    if (lpv == L) {                                                                                            \
+        hipLaunchKernelGGL((scene_frame_kernel<L, kRunBlock>), dim3(nruns), dim3(kRunBlock),                   \
+                           sizeof(float4) * maxVerts, stream, scenes, runs, items, substeps, iterations);      \
+        return hipGetLastError();                                                                              \
+    }
+    GVBD_CASE(1) GVBD_CASE(2) GVBD_CASE(4) GVBD_CASE(8) GVBD_CASE(16)
+#undef GVBD_CASE
+    return hipErrorInvalidValue;
 }
 
 hipError_t launch_counter_reset(int* counters, int n, hipStream_t stream) {

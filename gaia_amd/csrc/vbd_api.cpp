@@ -193,6 +193,10 @@ struct PlanObj {
     WorkItem* dDeformPre = nullptr;   // deformed vertices of cloth meshes (before the initial step)
     WorkItem* dDeformPost = nullptr;  // deformed vertices of tet meshes (after it)
     int32_t nDeformPre = 0, nDeformPost = 0;
+    // small scenes: frames stepped whole, one block per scene (see whole_frames)
+    SceneRun* dRuns = nullptr;
+    WorkItem* dRunItems = nullptr;
+    int32_t nRuns = 0, runVerts = 0;
     // work queue (mode GVBD_MODE_WORK_QUEUE)
     QueueEntry* dQueue = nullptr;
     int* dCounters = nullptr;  // tickets[iterations] then progress[scenes]
@@ -342,6 +346,9 @@ void free_plan(PlanObj& p) {
     p.dItems = nullptr;
     p.dCommit = nullptr;
     p.dVItems = nullptr;
+    p.dRuns = nullptr;
+    p.dRunItems = nullptr;
+    p.nRuns = p.runVerts = 0;
     p.dQueue = nullptr;
     p.dCounters = nullptr;
     p.nQueue = p.nCounters = p.queueGrid = p.ticketSlots = p.epoch = 0;
@@ -1017,6 +1024,33 @@ void assign_group_launches(gvbd_context* ctx, PlanObj& p) {
     }
 }
 
+// Whether a plan's frames are stepped whole by one block per scene (scene_frame_kernel) instead of one
+// launch per parallel group: scenes without collision handling and deformers, in group launches read
+// straight from HBM, of at most one pass of the block's 16 waves per launch on average. A launch costs
+// about 4 us and spreads a group over the chip; in the block a group costs 2 to 3 us and every further
+// pass as much again. Measured, launches -> block, us per frame of 10 iterations and 8 groups (waves
+// per iteration): tets, 4 lanes: 729 vertices (46) 392 -> 242, 1,331 (83) 431 -> 255, 2,197 (137)
+// 426 -> 356, 3,375 (211) 433 -> 549; 8 lanes: 729 (91) 336 -> 216, 1,331 (166) 351 -> 349; 16 lanes:
+// 343 (86) 306 -> 190, 729 (182) 309 -> 316; cloth, 4 lanes: 1,600 (100) 470 -> 361, 2,500 (156)
+// 467 -> 537; 8 lanes: 576 (72) 389 -> 284, 1,600 (200) 426 -> 522. Batches of scenes of up to 2,000
+// vertices, 4 lanes, 24 / 100 / 256 / 700 scenes: 609 -> 382, 817 -> 477, 941 -> 511, 2,265 -> 1,366.
+bool whole_frames(gvbd_context* ctx, const PlanObj& p) {
+    if (p.mode != GVBD_MODE_GROUP_LAUNCHES || p.stage != 0) return false;
+    const int vertsPerWave = 64 / p.lpv, wavesPerBlock = kRunBlock / 64;
+    for (int32_t sid : p.scenes) {
+        const SceneObj& s = scene_of(ctx, sid);
+        if (s.cd || s.nDeformPre || s.nDeformPost || s.nv > kRunVerts) return false;
+        if (s.tetGroupOffset.back() + s.clothGroupOffset.back() == 0) return false;  // nothing to solve
+        int64_t waves = 0;
+        for (size_t g = 0; g < s.groups.size(); ++g)
+            for (int n : {s.tetGroupOffset[g + 1] - s.tetGroupOffset[g],
+                          s.clothGroupOffset[g + 1] - s.clothGroupOffset[g]})
+                waves += (n + vertsPerWave - 1) / vertsPerWave;
+        if (waves > (int64_t)wavesPerBlock * p.numGroups) return false;
+    }
+    return true;
+}
+
 void build_plan(gvbd_context* ctx, PlanObj& p) {
     if (!p.dirty) return;
     free_plan(p);
@@ -1130,6 +1164,26 @@ void build_plan(gvbd_context* ctx, PlanObj& p) {
     }
     p.nDeformPre = (int32_t)dpre.size();
     p.nDeformPost = (int32_t)dpost.size();
+    std::vector<SceneRun> runs;
+    std::vector<WorkItem> runItems;
+    if (whole_frames(ctx, p)) {
+        const int verts = kRunBlock / p.lpv;
+        for (size_t si = 0; si < p.scenes.size(); ++si) {
+            const SceneObj& s = scene_of(ctx, p.scenes[si]);
+            const size_t first = runItems.size();
+            for (size_t g = 0; g < s.groups.size(); ++g) {
+                for (int32_t k = s.tetGroupOffset[g], e = s.tetGroupOffset[g + 1]; k < e; k += verts)
+                    runItems.push_back({0, k, std::min(verts, e - k), WORK_TET});
+                for (int32_t k = s.clothGroupOffset[g], e = s.clothGroupOffset[g + 1]; k < e; k += verts)
+                    runItems.push_back({0, k, std::min(verts, e - k), WORK_CLOTH});
+                commit_runs(s, (int)g, s.nv, [&](int32_t k, int32_t n) { runItems.push_back({0, k, n, WORK_COMMIT}); });
+                if (runItems.size() > first) runItems.back().scene |= RUN_GROUP_END;
+            }
+            runs.push_back({(int32_t)si, (int32_t)first, (int32_t)(runItems.size() - first), 0});
+            p.runVerts = std::max(p.runVerts, s.nv);
+        }
+        p.nRuns = (int32_t)runs.size();
+    }
     // one buffer: each array at a 256-byte aligned offset
     struct Part {
         void** dst;
@@ -1142,6 +1196,10 @@ void build_plan(gvbd_context* ctx, PlanObj& p) {
                                {(void**)&p.dItems, items.data(), sizeof(WorkItem) * items.size(), 0},
                                {(void**)&p.dCommit, commits.data(), sizeof(WorkItem) * commits.size(), 0},
                                {(void**)&p.dVItems, vitems.data(), sizeof(WorkItem) * vitems.size(), 0}};
+    if (p.nRuns) {
+        parts.push_back({(void**)&p.dRuns, runs.data(), sizeof(SceneRun) * runs.size(), 0});
+        parts.push_back({(void**)&p.dRunItems, runItems.data(), sizeof(WorkItem) * runItems.size(), 0});
+    }
     if (p.nDeformPre) parts.push_back({(void**)&p.dDeformPre, dpre.data(), sizeof(WorkItem) * dpre.size(), 0});
     if (p.nDeformPost) parts.push_back({(void**)&p.dDeformPost, dpost.data(), sizeof(WorkItem) * dpost.size(), 0});
     if (p.mode == GVBD_MODE_WORK_QUEUE) {
@@ -1428,6 +1486,13 @@ void plan_frame_launches(gvbd_context* ctx, PlanObj& p) {
         // served frames are not timed, so that no event wait slows their launch
         plan_device_contact_frame(ctx, p, !p.capturing && p.scenes.size() == 1);
         if (!p.capturing) contact_frame_done(p, ctx);
+        p.epoch = p.iterations;
+        return;
+    }
+    if (p.nRuns) {
+        hip_check(launch_scene_frames(p.dViews, p.dRuns, p.nRuns, p.dRunItems, p.runVerts, p.substeps, p.iterations,
+                                      p.lpv, ctx->stream),
+                  "frame launch");
         p.epoch = p.iterations;
         return;
     }

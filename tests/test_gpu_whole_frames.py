@@ -1,0 +1,85 @@
+"""Small scenes stepped whole by one block each (group launches without staging) against the work
+queue, which solves the same vertices in the same order: the same bits, for every lane count, one tet,
+groups of several passes, cloth committed through positionsNext with attachments, damping, fixed
+vertices, substeps and the accelerator, scenes on both sides of the sizes that are stepped whole, alone,
+in a batch and captured."""
+import numpy as np
+import pytest
+
+from gaia_amd import Batch, scenes
+from gaia_amd.vbd import physics_dict
+from test_gpu_deformers import hanging_pair_spec
+from vbd_cases import build_gpu, multi_spec
+
+pytestmark = pytest.mark.gpu
+
+
+def tets(n, **physics):
+    if n > 0:
+        pos, t = scenes.cube_tet_mesh(n, 0.1, origin=(0.0, 0.02, 0.0))
+    else:
+        pos, t = 0.1 * np.array([[0, 1, 0], [1, 1, 0], [0, 2, 0], [0, 1, 1.0]]), np.array([[0, 1, 2, 3]], np.int32)
+    return dict(physics=physics_dict(gravity=(0.0, -9.8, 0.0), time_step=1.0 / 60.0, world_lower=(-1e7, 0.0, -1e7),
+                                     **dict(dict(num_substeps=1, iterations=5), **physics)),
+                meshes=[dict(pos=pos, tets=t, material=dict(density=1000.0, mu=1e5, lmbd=1e6), fixed=(), vel=None,
+                             coloring="greedy")])
+
+
+def cloth(n):
+    pos, f = scenes.cloth_sheet(n, 0.6, 0.8)
+    mu, lm = scenes.stvk_lame(1e5, 0.3)
+    return dict(physics=physics_dict(gravity=(0.0, -9.8, 0.0), time_step=1.0 / 60.0, num_substeps=1, iterations=5,
+                                     world_lower=(-1e7, 0.0, -1e7)),
+                meshes=[dict(pos=pos, faces=f, material=dict(density=0.2, mu=mu, lmbd=lm, bending_stiffness=1e-4),
+                             fixed=[0, n - 1], vel=None, coloring="mcs")])
+
+
+def accelerated():
+    spec = multi_spec()
+    spec["physics"] = dict(spec["physics"], use_accelerator=1, accelerator_rho=0.9)
+    return spec
+
+
+# 1,331 and 3,375 tet vertices and 1,600 of cloth are stepped whole with few lanes only
+SPECS = [lambda: tets(0), lambda: tets(3, iterations=0), multi_spec, accelerated, lambda: cloth(12),
+         hanging_pair_spec, lambda: tets(10, num_substeps=2), lambda: tets(14), lambda: cloth(40)]
+
+
+def states(sims):
+    return [a for s in sims for m in range(s.numMeshes()) for a in s.getState(m)]
+
+
+@pytest.mark.parametrize("lanes", [1, 2, 4, 8, 16])
+def test_whole_frames_equal_the_work_queue(gpu_ctx, lanes):
+    runs = {}
+    for mode, graph in (("queue", False), ("group", False), ("group", True)):
+        sims = [build_gpu(gpu_ctx, s()) for s in SPECS]
+        for s in sims:
+            s.setSchedule(lanes, 256, mode=mode)
+            if graph:
+                s.recordVBDSolveGraph(True)
+            for _ in range(3):
+                s.runSteps(1)
+        runs[mode, graph] = states(sims)
+        for s in sims:
+            s.destroy()
+    for got in (runs["group", False], runs["group", True]):
+        assert all(np.isfinite(a).all() and np.array_equal(a, b) for a, b in zip(got, runs["queue", False]))
+
+
+def test_batch_stepped_whole_equals_the_scenes_alone(gpu_ctx):
+    specs = [tets(0), tets(3), tets(7), cloth(5), cloth(12)]
+    runs = []
+    for batched in (False, True):
+        sims = [build_gpu(gpu_ctx, s) for s in specs]
+        for s in sims:
+            s.setSchedule(4, 256, mode="queue" if not batched else "group")
+        if batched:
+            b = Batch(gpu_ctx, sims)
+            b.set_schedule(4, 256)
+            b.run_steps(3)
+        else:
+            for s in sims:
+                s.runSteps(3)
+        runs.append(states(sims))
+    assert all(np.array_equal(a, b) for a, b in zip(*runs))
