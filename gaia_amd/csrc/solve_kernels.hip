@@ -254,7 +254,7 @@ __device__ __forceinline__ void tet_block(const SceneView& S, float4* posInOut, 
     };
     if (S.trow) {
         const float* __restrict__ tvol = S.tvol;
-        for_lane_records<LPV, STAGE, 3>(reinterpret_cast<const float4*>(S.trow), blockBegin, blockEnd, slot.y + sub,
+        for_lane_records<LPV, STAGE, 3>(S.trow.as<const float4>(), blockBegin, blockEnd, slot.y + sub,
                                         slot.z, lds, [&](const float4* r, int k) {
             const float4 r0 = r[0];
             const float4 r1 = r[1];
@@ -265,7 +265,7 @@ __device__ __forceinline__ void tet_block(const SceneView& S, float4* posInOut, 
                 tvol[k]);
         });
     } else {
-        for_lane_records<LPV, 2 * STAGE, 2>(reinterpret_cast<const float4*>(S.tinc), blockBegin, blockEnd,
+        for_lane_records<LPV, 2 * STAGE, 2>(S.tinc.as<const float4>(), blockBegin, blockEnd,
                                             slot.y + sub, slot.z, lds, [&](const float4* r, int) {
             const float4 r0 = r[0];
             const float4 r1 = r[1];
@@ -740,7 +740,7 @@ __device__ __forceinline__ void cloth_block(const SceneView& S, float4* posInOut
     // membrane force and Hessian (kept apart for the StVK damping term)
     float fm0 = 0.f, fm1 = 0.f, fm2 = 0.f;
     float hxx = 0.f, hxy = 0.f, hxz = 0.f, hyy = 0.f, hyz = 0.f, hzz = 0.f;
-    for_lane_records<LPV, 2 * STAGE, 2>(reinterpret_cast<const float4*>(S.cface), first.x, last.x, sa.y + sub, sa.z,
+    for_lane_records<LPV, 2 * STAGE, 2>(S.cface.as<const float4>(), first.x, last.x, sa.y + sub, sa.z,
                                         lds, [&](const float4* r, int) {
         const float4 r0 = r[0];
         const float4 r1 = r[1];
@@ -774,7 +774,7 @@ __device__ __forceinline__ void cloth_block(const SceneView& S, float4* posInOut
     // bending: f -= sum_j kQ(o,j) X_j, H += kQ(o,o) I, skipping degenerate stencils
     float fb0 = 0.f, fb1 = 0.f, fb2 = 0.f, hb = 0.f;
     const float thr2 = S.sp.degenerateThresSq;
-    for_lane_records<LPV, 2 * STAGE, 2>(reinterpret_cast<const float4*>(S.cbend), first.y, last.y, sb.x + sub, sb.y,
+    for_lane_records<LPV, 2 * STAGE, 2>(S.cbend.as<const float4>(), first.y, last.y, sb.x + sub, sb.y,
                                         lds, [&](const float4* r, int) {
         const float4 r0 = r[0];
         const float4 r1 = r[1];
@@ -887,8 +887,11 @@ __device__ __forceinline__ void cloth_block(const SceneView& S, float4* posInOut
             }
         }
     }
-    float4* dst = (sa.w & SLOT_INPLACE) ? posInOut : pnext;
-    dst[v] = make_float4(xn.x, xn.y, xn.z, 0.f);
+    const float4 out = make_float4(xn.x, xn.y, xn.z, 0.f);
+    if (sa.w & SLOT_INPLACE)
+        posInOut[v] = out;
+    else
+        pnext[v] = out;
 }
 
 }  // namespace

@@ -3135,10 +3135,14 @@ static ServerObj& server_of(gvbd_context* ctx, int32_t id) {
     return *it->second;
 }
 
+template <class T> static T*& raw_pointer(T*& p) { return p; }
+template <class T> static T*& raw_pointer(HbmPtr<T>& p) { return reinterpret_cast<T*&>(p); }
+
 // Moves a scene's device pointers from one arena base to another. The arena's arrays hold
 // indices, never addresses, so a copied arena is valid at any base.
 static void rebase_scene(SceneObj& s, uintptr_t from, uintptr_t to) {
-    auto mv = [&](auto*& p) {
+    auto mv = [&](auto& ptr) {
+        auto& p = raw_pointer(ptr);
         using P = std::remove_reference_t<decltype(p)>;
         if (p) p = reinterpret_cast<P>(to + (reinterpret_cast<uintptr_t>(p) - from));
     };
