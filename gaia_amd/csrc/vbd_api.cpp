@@ -638,7 +638,8 @@ void upload_scene(gvbd_context* ctx, SceneObj& s, const std::function<void(size_
         const auto& grp = s.groups[g];
         // A cloth mesh with a single colour in this group can be updated in place: its solved
         // vertices share no element, so the reference's positionsNext + copy (Jacobi over the
-        // group) gives the same result. Without contact, meshes do not interact.
+        // group) gives the same result. Meshes interact by contact alone, whose partners of the own
+        // group are read from the iteration-start snapshot (ContactView::snap).
         std::vector<int32_t> firstColor(s.meshes.size(), -1);
         std::vector<uint8_t> multiColor(s.meshes.size(), 0);
         for (size_t i = 0; i + 1 < grp.size(); i += 2) {
@@ -657,7 +658,7 @@ void upload_scene(gvbd_context* ctx, SceneObj& s, const std::function<void(size_
                               tetWork, contact ? &trefs[im] : nullptr);
             } else {
                 // attachments read other vertices of the group: positionsNext keeps them Jacobi
-                const bool inplace = !multiColor[im] && !s.params.handle_collision && attOf.empty();
+                const bool inplace = !multiColor[im] && attOf.empty();
                 emit_cloth_slot(s.cloths[s.meshes[im].second], off, lv, inplace, cslots, cface, cbend, clothWork,
                                 contact ? &refs[im] : nullptr);
                 if (!attOf.empty() && !attOf[off + lv].empty()) cslots.back().a.w |= SLOT_ATTACH;
