@@ -44,16 +44,38 @@ struct alignas(64) BvhPair {
     float4 lo0, hi0, lo1, hi1;
 };
 
+// Refit (see refit_blocks_kernel): one launch does the nodes within blocks of kRefitLeaves consecutive
+// leaves, one more per tier those within windows of kRefitFan times as many.
+constexpr int kRefitLeaves = 1024;
+constexpr int kRefitFan = 64;
+constexpr int kMaxRefitDepth = 62;  // keys of 30 Morton bits and 32 index bits
+struct RefitTiers {
+    int count;
+    int windows[4];
+    int firstList[4], firstEntry[4];
+    int capacity[4];  // entries per list
+    int lists() const { return count ? firstList[count - 1] + windows[count - 1] : 0; }
+};
+struct RefitTop {
+    int node, left, right;
+    int parentAt, leftAt, rightAt;  // places in the same list, or -1
+    int pad[2];
+};
+
 struct DeviceBvh {
     int n = 0;                       // primitives
     BvhNode* nodes = nullptr;        // 2n - 1
     BvhPair* pairs = nullptr;        // n - 1 (1 for a single primitive): set at every refit
     int* parent = nullptr;           // 2n - 1
     int* right = nullptr;            // n - 1: right child of each internal node (refit)
+    RefitTiers tiers{};
+    RefitTop* top = nullptr;         // the tiers' lists
+    int* topCount = nullptr;         // per list: its entries
+    int topMost[4] = {0, 0, 0, 0};   // host: longest list per tier
     int* levelNodes = nullptr;       // internal nodes ordered by depth, deepest first
     std::vector<int> levelBegin;     // host: ranges of levelNodes per depth (deepest first)
     int* dLevelBegin = nullptr;      // the same ranges on the device
-    std::vector<std::pair<int, int>> segments;  // refit launches: [first, last) level runs
+    std::vector<std::pair<int, int>> segments;  // launches over the levels: [first, last) level runs
     uint64_t* keysAlt = nullptr;     // n (sorted Morton keys)
     int* mesh = nullptr;             // 2n - 1 (face trees of penetration contact): the mesh of every
                                      // face below the node, -1 where faces of several meshes meet

@@ -951,8 +951,12 @@ __device__ __forceinline__ int common_prefix(const uint64_t* keys, int n, int i,
 
 // Binary radix tree over sorted unique keys (Karras 2012): internal node i covers a key range
 // starting or ending at i; its split is the highest differing bit in the range.
+// Nodes whose leaves lie in several blocks of kRefitLeaves get a list: of the smallest window of
+// kRefitLeaves * kRefitFan^t leaves (t >= 1) that holds all their leaves; topList and topSlot: a node's list
+// (-1: none) and its place there.
 __global__ __launch_bounds__(256) void build_tree_kernel(const uint64_t* keys, int n, BvhNode* nodes, int* parent,
-                                                         int* rightChild) {
+                                                         int* rightChild, RefitTiers tiers, int* topCount,
+                                                         int* topList, int* topSlot) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) {  // leaves
         BvhNode& L = nodes[n - 1 + i];
@@ -982,6 +986,36 @@ __global__ __launch_bounds__(256) void build_tree_kernel(const uint64_t* keys, i
     rightChild[i] = right;
     parent[left] = i;
     parent[right] = i;
+    int list = -1, slot = 0;
+    int a = lo / kRefitLeaves, b = hi / kRefitLeaves;
+    for (int t = 0; a != b && t < tiers.count; ++t) {
+        a /= kRefitFan;
+        b /= kRefitFan;
+        if (a == b) {
+            list = tiers.firstList[t] + a;
+            slot = atomicAdd(topCount + list, 1);
+        }
+    }
+    topList[i] = list;
+    topSlot[i] = slot;
+}
+
+// Entries of the lists: a node's children and parent, by their places where they are in the same list.
+__global__ __launch_bounds__(256) void refit_top_entries_kernel(const BvhNode* nodes, const int* parent,
+                                                                const int* rightChild, int nInternal,
+                                                                RefitTiers tiers, const int* topList,
+                                                                const int* topSlot, RefitTop* entries) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= nInternal) return;
+    const int list = topList[i];
+    if (list < 0) return;
+    int t = 0;
+    while (t + 1 < tiers.count && list >= tiers.firstList[t + 1]) ++t;
+    if (topSlot[i] >= tiers.capacity[t]) return;  // (a list holds every node that crosses its windows' borders)
+    const auto place = [&](int c) { return c >= 0 && c < nInternal && topList[c] == list ? topSlot[c] : -1; };
+    const int left = __float_as_int(nodes[i].lo.w), right = rightChild[i];
+    entries[tiers.firstEntry[t] + (int64_t)(list - tiers.firstList[t]) * tiers.capacity[t] + topSlot[i]] =
+        RefitTop{i, left, right, place(parent[i]), place(left), place(right), {0, 0}};
 }
 
 // Skip link of every node (written to hi.w): the right sibling of the nearest node on the path
@@ -1049,15 +1083,10 @@ __global__ __launch_bounds__(256) void level_nodes_kernel(const uint64_t* keys, 
     if (i == 0 || (int)(keys[i - 1] >> 32) != (int)(keys[i] >> 32)) starts[dk] = i;
 }
 
-__global__ __launch_bounds__(256) void leaf_box_kernel(CDView S, int kind, BvhNode* nodes, BvhPair* pairs,
-                                                       int n) {
-    if (S.gate && !*S.gate) return;
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    BvhNode& L = nodes[n - 1 + k];
-    const int prim = __float_as_int(L.lo.w) & kLeafPrimMask;
-    int tag = prim;
-    V3 lo, hi;
+// Box of a tree's primitive and its leaf word (the primitive; for an edge also which endpoint gives
+// each bound).
+__device__ __forceinline__ void prim_box(const CDView& S, int kind, int prim, V3& lo, V3& hi, int& tag) {
+    tag = prim;
     if (kind == 3) {
         tet_box(S, prim, lo, hi);
     } else if (kind == 4) {
@@ -1077,51 +1106,172 @@ __global__ __launch_bounds__(256) void leaf_box_kernel(CDView S, int kind, BvhNo
         hi = {sx ? a.x : b.x, sy ? a.y : b.y, sz ? a.z : b.z};
         tag = prim | ((int)sx | (int)sy << 1 | (int)sz << 2) << kLeafPrimBits;
     }
-    L.lo = make_float4(lo.x, lo.y, lo.z, __int_as_float(tag));
-    L.hi = make_float4(hi.x, hi.y, hi.z, L.hi.w);
-    // a tree of one primitive has no internal node: its pair holds the leaf and an empty box
-    if (n == 1 && pairs)
-        pairs[0] = BvhPair{L.lo, make_float4(hi.x, hi.y, hi.z, __int_as_float(1)),
-                           make_float4(FLT_MAX, FLT_MAX, FLT_MAX, 0.f), make_float4(-FLT_MAX, -FLT_MAX, -FLT_MAX, 0.f)};
 }
 
-// Box of internal node i from its children's, and (trees with wave queries) the children side by side.
-__device__ __forceinline__ void merge_children(BvhNode* nodes, const int* rightChild, BvhPair* pairs, int firstLeaf,
-                                               int i) {
-    BvhNode& N = nodes[i];
-    const int a = __float_as_int(N.lo.w), b = rightChild[i];
-    const BvhNode A = nodes[a], B = nodes[b];
-    N.lo = make_float4(fminf(A.lo.x, B.lo.x), fminf(A.lo.y, B.lo.y), fminf(A.lo.z, B.lo.z), N.lo.w);
-    N.hi = make_float4(fmaxf(A.hi.x, B.hi.x), fmaxf(A.hi.y, B.hi.y), fmaxf(A.hi.z, B.hi.z), N.hi.w);
+struct Box {
+    V3 lo, hi;
+};
+__device__ __forceinline__ Box merge(const Box& A, const Box& B) {
+    return {{fminf(A.lo.x, B.lo.x), fminf(A.lo.y, B.lo.y), fminf(A.lo.z, B.lo.z)},
+            {fmaxf(A.hi.x, B.hi.x), fmaxf(A.hi.y, B.hi.y), fmaxf(A.hi.z, B.hi.z)}};
+}
+__device__ __forceinline__ Box node_box(const BvhNode& N) {
+    return {{N.lo.x, N.lo.y, N.lo.z}, {N.hi.x, N.hi.y, N.hi.z}};
+}
+
+// Boxes in LDS, one array per bound (the lanes' accesses go to different banks).
+struct LdsBoxes {
+    float* p;
+    int n;
+    __device__ __forceinline__ Box get(int i) const {
+        return {{p[i], p[n + i], p[2 * n + i]}, {p[3 * n + i], p[4 * n + i], p[5 * n + i]}};
+    }
+    __device__ __forceinline__ void set(int i, const Box& b) const {
+        p[i] = b.lo.x, p[n + i] = b.lo.y, p[2 * n + i] = b.lo.z;
+        p[3 * n + i] = b.hi.x, p[4 * n + i] = b.hi.y, p[5 * n + i] = b.hi.z;
+    }
+};
+
+// Writes an internal node's box (its child and skip links stay) and, for trees with wave queries, its
+// children side by side: refA, refB are the children's node, or a leaf's word.
+__device__ __forceinline__ void store_node(BvhNode* nodes, BvhPair* pairs, int i, const Box& N, const Box& A,
+                                           const Box& B, float refA, float refB, bool leafA, bool leafB) {
+    BvhNode& n = nodes[i];
+    n.lo.x = N.lo.x, n.lo.y = N.lo.y, n.lo.z = N.lo.z;
+    n.hi.x = N.hi.x, n.hi.y = N.hi.y, n.hi.z = N.hi.z;
     if (!pairs) return;
-    const bool la = a >= firstLeaf, lb = b >= firstLeaf;
-    pairs[i] = BvhPair{make_float4(A.lo.x, A.lo.y, A.lo.z, la ? A.lo.w : __int_as_float(a)),
-                       make_float4(A.hi.x, A.hi.y, A.hi.z, __int_as_float(la ? 1 : 0)),
-                       make_float4(B.lo.x, B.lo.y, B.lo.z, lb ? B.lo.w : __int_as_float(b)),
-                       make_float4(B.hi.x, B.hi.y, B.hi.z, __int_as_float(lb ? 1 : 0))};
+    pairs[i] = BvhPair{make_float4(A.lo.x, A.lo.y, A.lo.z, refA),
+                       make_float4(A.hi.x, A.hi.y, A.hi.z, __int_as_float(leafA ? 1 : 0)),
+                       make_float4(B.lo.x, B.lo.y, B.lo.z, refB),
+                       make_float4(B.hi.x, B.hi.y, B.hi.z, __int_as_float(leafB ? 1 : 0))};
 }
 
-__global__ __launch_bounds__(256) void internal_box_kernel(const int* levelNodes, int begin, int end, BvhNode* nodes,
-                                                           const int* rightChild, BvhPair* pairs, int firstLeaf,
-                                                           const int* gate) {
-    if (gate && !*gate) return;
-    const int k = begin + blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < end) merge_children(nodes, rightChild, pairs, firstLeaf, levelNodes[k]);
+__device__ __forceinline__ int lds_count(int* p, int d) {
+    return __hip_atomic_fetch_add(p, d, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// Several consecutive refit levels of few nodes each in one block: the levels run in order with a
-// block barrier between them, so a level reads children finished by the previous ones (levels
-// before the segment were finished by earlier launches).
-__global__ __launch_bounds__(1024) void internal_box_levels_kernel(const int* levelNodes, const int* levelBegin,
-                                                                   int l0, int l1, BvhNode* nodes,
-                                                                   const int* rightChild, BvhPair* pairs,
-                                                                   int firstLeaf, const int* gate) {
-    if (gate && !*gate) return;  // uniform over the block: no barrier is left waiting
-    for (int l = l0; l < l1; ++l) {
-        const int b = levelBegin[l], e = levelBegin[l + 1];
-        for (int k = b + (int)threadIdx.x; k < e; k += (int)blockDim.x)
-            merge_children(nodes, rightChild, pairs, firstLeaf, levelNodes[k]);
-        __syncthreads();
+// Refit of one block of kRefitLeaves leaves (in tree order): their boxes, then every internal node all of
+// whose leaves are among them. The internal node of a radix tree has the number of its first or last
+// leaf, so these nodes are in the block's own range of numbers. A leaf's thread climbs in LDS while it
+// is the second to arrive at a node: a node with leaves elsewhere gets one arrival at most and is left to
+// refit_top_kernel. Bound by the climb's chain of LDS accesses (13 us for trees of 10k to 40k leaves, 45 us
+// for 663k, where the nodes' stores count) and by the launches. With a launch per level (small levels
+// together in one block, from HBM) a refit of two such trees took 75 us for 7 large levels, now 25.
+__global__ __launch_bounds__(kRefitLeaves) void refit_blocks_kernel(CDView S, int kind, BvhNode* nodes,
+                                                                    const int* parent, const int* rightChild,
+                                                                    BvhPair* pairs, int n) {
+    constexpr int L = kRefitLeaves, kElsewhere = 0xFFFF;
+    // entries 0 .. L - 1: the internal nodes of the block's numbers; L .. 2 L - 1: its leaves
+    __shared__ float boxes[6 * 2 * L];
+    __shared__ unsigned int children[L];  // left | right << 16
+    __shared__ unsigned short up[2 * L];
+    __shared__ int arrived[L], word[L];
+    if (S.gate && !*S.gate) return;  // uniform over the block
+    const LdsBoxes box{boxes, 2 * L};
+    const int tid = threadIdx.x, base = blockIdx.x * L, k = base + tid;
+    const auto local = [&](int c) {
+        const unsigned int d = (unsigned int)((c >= n - 1 ? c - (n - 1) : c) - base);
+        return c < 0 || d >= (unsigned int)L ? kElsewhere : (int)d + (c >= n - 1 ? L : 0);
+    };
+    int left = 0, right = 0;
+    if (k < n - 1) {
+        left = __float_as_int(nodes[k].lo.w);
+        right = rightChild[k];
+        up[tid] = (unsigned short)local(parent[k]);
+        children[tid] = (unsigned int)local(left) | (unsigned int)local(right) << 16;
+    }
+    arrived[tid] = 0;
+    if (k < n) {
+        BvhNode& leaf = nodes[n - 1 + k];
+        V3 lo, hi;
+        int tag;
+        prim_box(S, kind, __float_as_int(leaf.lo.w) & kLeafPrimMask, lo, hi, tag);
+        up[L + tid] = (unsigned short)local(parent[n - 1 + k]);
+        box.set(L + tid, {lo, hi});
+        word[tid] = tag;
+        leaf.lo = make_float4(lo.x, lo.y, lo.z, __int_as_float(tag));
+        leaf.hi.x = hi.x, leaf.hi.y = hi.y, leaf.hi.z = hi.z;
+        // a tree of one primitive has no internal node: its pair holds the leaf and an empty box
+        if (n == 1 && pairs)
+            pairs[0] = BvhPair{make_float4(lo.x, lo.y, lo.z, __int_as_float(tag)),
+                               make_float4(hi.x, hi.y, hi.z, __int_as_float(1)),
+                               make_float4(FLT_MAX, FLT_MAX, FLT_MAX, 0.f),
+                               make_float4(-FLT_MAX, -FLT_MAX, -FLT_MAX, 0.f)};
+    }
+    __syncthreads();
+    if (k < n) {
+        for (int p = up[L + tid]; p != kElsewhere && lds_count(arrived + p, 1) == 1; p = up[p]) {
+            const unsigned int c = children[p];
+            box.set(p, merge(box.get(c & 0xFFFF), box.get(c >> 16)));
+        }
+    }
+    __syncthreads();
+    if (k < n - 1 && arrived[tid] == 2) {
+        const int a = children[tid] & 0xFFFF, b = children[tid] >> 16;
+        const bool la = a >= L, lb = b >= L;
+        store_node(nodes, pairs, k, box.get(tid), box.get(a), box.get(b), __int_as_float(la ? word[a - L] : left),
+                   __int_as_float(lb ? word[b - L] : right), la, lb);
+    }
+}
+
+// LDS bytes of refit_top_kernel for lists of up to m nodes.
+constexpr size_t refit_top_lds(int m) { return (size_t)m * (6 * sizeof(float) + sizeof(int) + 3 * sizeof(short)); }
+
+// Refit of one window's list of nodes (see build_tree_kernel): children outside the list were finished by
+// earlier launches. A node without children in the list starts a climb; a node with one keeps the other
+// child's box in its own place until the climb arrives.
+__global__ __launch_bounds__(1024) void refit_top_kernel(const RefitTop* entries, int capacity, const int* counts,
+                                                         int most, BvhNode* nodes, BvhPair* pairs, int firstLeaf,
+                                                         const int* gate) {
+    constexpr int kNone = 0xFFFF;
+    extern __shared__ float topLds[];
+    if (gate && !*gate) return;  // uniform over the block
+    const LdsBoxes box{topLds, most};
+    int* missing = (int*)(topLds + 6 * (size_t)most);
+    unsigned short* up = (unsigned short*)(missing + most);
+    unsigned short *leftAt = up + most, *rightAt = leftAt + most;
+    const RefitTop* list = entries + (int64_t)blockIdx.x * capacity;
+    const int m = min(counts[blockIdx.x], most);
+    for (int e = threadIdx.x; e < m; e += blockDim.x) {
+        const RefitTop E = list[e];
+        up[e] = (unsigned short)E.parentAt;  // -1 becomes kNone
+        leftAt[e] = (unsigned short)E.leftAt;
+        rightAt[e] = (unsigned short)E.rightAt;
+        missing[e] = (E.leftAt >= 0) + (E.rightAt >= 0);
+        if (E.leftAt < 0 && E.rightAt < 0)
+            box.set(e, merge(node_box(nodes[E.left]), node_box(nodes[E.right])));
+        else if (E.leftAt < 0 || E.rightAt < 0)
+            box.set(e, node_box(nodes[E.leftAt < 0 ? E.left : E.right]));
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < m; e += blockDim.x) {
+        if (leftAt[e] != kNone || rightAt[e] != kNone) continue;
+        for (int p = up[e]; p != kNone && lds_count(missing + p, -1) == 1; p = up[p]) {
+            const int a = leftAt[p], b = rightAt[p];
+            box.set(p, merge(box.get(a != kNone ? a : p), box.get(b != kNone ? b : p)));
+        }
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < m; e += blockDim.x) {
+        const RefitTop E = list[e];
+        const bool la = E.left >= firstLeaf, lb = E.right >= firstLeaf;
+        Box A, B;
+        float refA = __int_as_float(E.left), refB = __int_as_float(E.right);
+        if (E.leftAt >= 0) {
+            A = box.get(E.leftAt);
+        } else {
+            const BvhNode c = nodes[E.left];
+            A = node_box(c);
+            if (la) refA = c.lo.w;
+        }
+        if (E.rightAt >= 0) {
+            B = box.get(E.rightAt);
+        } else {
+            const BvhNode c = nodes[E.right];
+            B = node_box(c);
+            if (lb) refB = c.lo.w;
+        }
+        store_node(nodes, pairs, E.node, box.get(e), A, B, refA, refB, la, lb);
     }
 }
 
@@ -2224,6 +2374,29 @@ void ContactDetector::allocBvh(DeviceBvh& B, int n, bool pairs) {
     B.keysAlt = dalloc<uint64_t>(B.n);
     B.levelNodes = dalloc<int>(std::max(B.n - 1, 1));
     B.dLevelBegin = dalloc<int>(kMaxDepth + 1);
+    // refit lists: windows of kRefitLeaves * kRefitFan^(t + 1) leaves; a node in a window's list crosses
+    // one of its inner borders, and at most kMaxRefitDepth nodes cross one border
+    int64_t entries = 0;
+    int lists = 0;
+    B.tiers = RefitTiers{};
+    for (int64_t parts = (B.n + kRefitLeaves - 1) / kRefitLeaves; parts > 1;) {
+        const int t = B.tiers.count++;
+        const int64_t windows = (parts + kRefitFan - 1) / kRefitFan;
+        B.tiers.windows[t] = (int)windows;
+        B.tiers.firstList[t] = lists;
+        B.tiers.firstEntry[t] = (int)entries;
+        B.tiers.capacity[t] = (int)(std::min<int64_t>(parts, kRefitFan) - 1) * kMaxRefitDepth;
+        lists += (int)windows;
+        entries += windows * B.tiers.capacity[t];
+        parts = windows;
+    }
+    if (lists) {
+        B.top = dalloc<RefitTop>((size_t)entries);
+        B.topCount = dalloc<int>(lists);
+        hip_check(hipFuncSetAttribute((const void*)refit_top_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      (int)refit_top_lds(kRefitFan * kMaxRefitDepth)),
+                  "refit LDS");
+    }
 }
 
 // Buffers of the tree builds, which run one after another on the detector's stream: one set, enough
@@ -2286,14 +2459,21 @@ void ContactDetector::buildBvh(DeviceBvh& B, int kind, const float4* prev) {
         hip_check(rocprim::radix_sort_keys(vSortTemp_, tv, vKeys_, vKeysAlt_, (size_t)nv_, 0, 62, stream_),
                   "vertex order sort");
     }
+    const int ni = n - 1;
+    int *topList = T.jump, *topSlot = T.jump + ni;
+    const int lists = B.tiers.lists();
+    if (lists)
+        hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(256), 0, stream_, B.topCount, (int64_t)lists, 0);
     hipLaunchKernelGGL(build_tree_kernel, dim3(blocks_for(n)), dim3(256), 0, stream_, B.keysAlt, n, B.nodes, B.parent,
-                       B.right);
+                       B.right, B.tiers, B.topCount, topList, topSlot);
+    if (lists)
+        hipLaunchKernelGGL(refit_top_entries_kernel, dim3(blocks_for(ni)), dim3(256), 0, stream_, B.nodes, B.parent,
+                           B.right, ni, B.tiers, topList, topSlot, B.top);
     hipLaunchKernelGGL(skip_kernel, dim3(blocks_for(2 * (int64_t)n - 1)), dim3(256), 0, stream_, B.nodes, B.parent,
                        B.right, 2 * n - 1, error_);
     hip_check(hipGetLastError(), "bvh build launch");
-    // refit schedule: internal nodes by depth, deepest first
+    // internal nodes by depth, deepest first
     B.levelBegin.clear();
-    const int ni = n - 1;
     if (ni > 0) {
         int* d0 = T.jump;
         int* d1 = T.jump + ni;
@@ -2316,13 +2496,22 @@ void ContactDetector::buildBvh(DeviceBvh& B, int kind, const float4* prev) {
         std::vector<int> starts(kMaxDepth, -1);
         hip_check(hipMemcpyAsync(starts.data(), depthHist_, kMaxDepth * sizeof(int), hipMemcpyDeviceToHost, stream_),
                   "level read");
+        std::vector<int> counts(lists);
+        if (lists)
+            hip_check(hipMemcpyAsync(counts.data(), B.topCount, lists * sizeof(int), hipMemcpyDeviceToHost, stream_),
+                      "list sizes");
         hip_check(hipStreamSynchronize(stream_), "bvh build sync");
+        for (int t = 0; t < B.tiers.count; ++t) {
+            const int* c = counts.data() + B.tiers.firstList[t];
+            B.topMost[t] = *std::max_element(c, c + B.tiers.windows[t]);
+            if (B.topMost[t] > B.tiers.capacity[t]) fail(GVBD_ERR_STATE, "a refit list is longer than its bound");
+        }
         // runs are stored deepest first
         for (int d = kMaxDepth - 1; d >= 0; --d)
             if (starts[d] >= 0) B.levelBegin.push_back(starts[d]);
         B.levelBegin.push_back(ni);
-        // refit launches: every level of more than kBlockLevel nodes alone, runs of smaller levels
-        // together in one block
+        // launches over the levels: every level of more than kBlockLevel nodes alone, runs of smaller
+        // levels together in one block
         B.segments.clear();
         const int nl = (int)B.levelBegin.size() - 1;
         for (int l = 0; l < nl;) {
@@ -2366,15 +2555,13 @@ void ContactDetector::refitBvh(DeviceBvh& B, int kind, hipStream_t stream, const
     S.tets = penTets_;
     S.prev = prev;
     S.gate = gate;
-    hipLaunchKernelGGL(leaf_box_kernel, dim3(blocks_for(B.n)), dim3(256), 0, stream, S, kind, B.nodes, B.pairs, B.n);
-    for (const auto& seg : B.segments) {
-        const int b = B.levelBegin[seg.first], e = B.levelBegin[seg.first + 1];
-        if (seg.second == seg.first + 1 && e - b > kBlockLevel)
-            hipLaunchKernelGGL(internal_box_kernel, dim3(blocks_for(e - b)), dim3(256), 0, stream, B.levelNodes, b,
-                               e, B.nodes, B.right, B.pairs, B.n - 1, gate);
-        else
-            hipLaunchKernelGGL(internal_box_levels_kernel, dim3(1), dim3(kBlockLevel), 0, stream, B.levelNodes,
-                               B.dLevelBegin, seg.first, seg.second, B.nodes, B.right, B.pairs, B.n - 1, gate);
+    hipLaunchKernelGGL(refit_blocks_kernel, dim3((B.n + kRefitLeaves - 1) / kRefitLeaves), dim3(kRefitLeaves), 0,
+                       stream, S, kind, B.nodes, B.parent, B.right, B.pairs, B.n);
+    for (int t = 0; t < B.tiers.count; ++t) {
+        if (B.topMost[t] == 0) continue;
+        hipLaunchKernelGGL(refit_top_kernel, dim3(B.tiers.windows[t]), dim3(1024), refit_top_lds(B.topMost[t]), stream,
+                           B.top + B.tiers.firstEntry[t], B.tiers.capacity[t], B.topCount + B.tiers.firstList[t],
+                           B.topMost[t], B.nodes, B.pairs, B.n - 1, gate);
     }
     hip_check(hipGetLastError(), "bvh refit launch");
 }
