@@ -7,6 +7,8 @@
 #include <cstdint>
 #include <vector>
 
+#include "host_stage.h"
+
 namespace gvbd {
 
 // One BVH node: box lo/hi; lo.w (int bits) holds an internal node's left child or a leaf's
@@ -149,7 +151,7 @@ struct DetectorDeviceView {
 
 class ContactDetector {
   public:
-    ContactDetector(int device, hipStream_t stream, float maxQueryDis, int vfCap, int eeCap);
+    ContactDetector(int device, hipStream_t stream, HostStage& stage, float maxQueryDis, int vfCap, int eeCap);
     ~ContactDetector();
     ContactDetector(const ContactDetector&) = delete;
     ContactDetector& operator=(const ContactDetector&) = delete;
@@ -239,6 +241,7 @@ class ContactDetector {
 
     int device_;
     hipStream_t stream_;
+    HostStage& stage_;
     hipStream_t side_ = nullptr;  // default priority, created at finalize
     hipEvent_t forkEv_ = nullptr, joinEv_ = nullptr;
     float r_;

@@ -2130,8 +2130,9 @@ template <class T> T* ContactDetector::dalloc(size_t n) {
     return (T*)p;
 }
 
-ContactDetector::ContactDetector(int device, hipStream_t stream, float maxQueryDis, int vfCap, int eeCap)
-    : device_(device), stream_(stream), r_(maxQueryDis), vfCap_(vfCap), eeCap_(eeCap) {
+ContactDetector::ContactDetector(int device, hipStream_t stream, HostStage& stage, float maxQueryDis, int vfCap,
+                                 int eeCap)
+    : device_(device), stream_(stream), stage_(stage), r_(maxQueryDis), vfCap_(vfCap), eeCap_(eeCap) {
     require(maxQueryDis > 0.f && std::isfinite(maxQueryDis), "max_query_distance must be positive");
     require(vfCap >= 1 && vfCap <= kMaxCap && eeCap >= 1 && eeCap <= kMaxCap,
             "contact capacities must be in [1, 16]");
@@ -2778,10 +2779,7 @@ void ContactDetector::setPositions(int mesh, const float* pos) {
     if (!ready_) fail(GVBD_ERR_STATE, "detector not finalized");
     require(mesh >= 0 && mesh < numMeshes(), "mesh index out of range");
     const int off = meshV_[mesh], n = meshV_[mesh + 1] - off;
-    std::vector<float4> p4(n);
-    for (int i = 0; i < n; ++i) p4[i] = make_float4(pos[3 * i], pos[3 * i + 1], pos[3 * i + 2], 0.f);
-    hip_check(hipMemcpyAsync(pos_ + off, p4.data(), sizeof(float4) * n, hipMemcpyHostToDevice, stream_), "positions");
-    hip_check(hipStreamSynchronize(stream_), "positions sync");
+    stage_.upload({{StagePart::VEC3, const_cast<float*>(pos), pos_ + off, n}});
     treeCurrent_ = false;
 }
 
@@ -2789,14 +2787,7 @@ void ContactDetector::getPositions(int mesh, float* pos) const {
     if (!ready_) fail(GVBD_ERR_STATE, "detector not finalized");
     require(mesh >= 0 && mesh < numMeshes(), "mesh index out of range");
     const int off = meshV_[mesh], n = meshV_[mesh + 1] - off;
-    std::vector<float4> p4(n);
-    hip_check(hipMemcpyAsync(p4.data(), pos_ + off, sizeof(float4) * n, hipMemcpyDeviceToHost, stream_), "positions");
-    hip_check(hipStreamSynchronize(stream_), "positions sync");
-    for (int i = 0; i < n; ++i) {
-        pos[3 * i] = p4[i].x;
-        pos[3 * i + 1] = p4[i].y;
-        pos[3 * i + 2] = p4[i].z;
-    }
+    stage_.download({{StagePart::VEC3, pos, const_cast<float4*>(pos_) + off, n}});
 }
 
 void ContactDetector::perturb(uint64_t seed, int step, float sigma, const float* drift) {
@@ -3030,45 +3021,33 @@ void ContactDetector::eeContactsAll(int32_t* ee, float* mu, float* d) {
 }
 
 void ContactDetector::vfContactsCapped(int32_t* count, VFContactRec* rec) {
-    if (count) {
-        const auto c = download(vfStored_, nv_, stream_);
-        std::memcpy(count, c.data(), sizeof(int) * nv_);
-    }
-    if (rec) {
-        const auto r = download(vfRec_, (size_t)nv_ * vfCap_, stream_);
-        std::memcpy(rec, r.data(), sizeof(VFContactRec) * r.size());
-    }
+    if (!ready_) fail(GVBD_ERR_STATE, "detector not finalized");
+    std::vector<StagePart> parts;
+    if (count) parts.push_back({StagePart::WORDS, count, vfStored_, nv_});
+    if (rec) parts.push_back({StagePart::WORDS, rec, vfRec_, (int64_t)nv_ * vfCap_ * (int64_t)(sizeof(VFContactRec) / 4)});
+    if (!parts.empty()) stage_.download(parts);
 }
 
 void ContactDetector::eeContactsCapped(int32_t* count, EEContactRec* rec) {
-    if (count) {
-        const auto c = download(eeStored_, ne_, stream_);
-        std::memcpy(count, c.data(), sizeof(int) * ne_);
-    }
-    if (rec) {
-        const auto r = download(eeRec_, (size_t)ne_ * eeCap_, stream_);
-        std::memcpy(rec, r.data(), sizeof(EEContactRec) * r.size());
-    }
+    if (!ready_) fail(GVBD_ERR_STATE, "detector not finalized");
+    std::vector<StagePart> parts;
+    if (count) parts.push_back({StagePart::WORDS, count, eeStored_, ne_});
+    if (rec) parts.push_back({StagePart::WORDS, rec, eeRec_, (int64_t)ne_ * eeCap_ * (int64_t)(sizeof(EEContactRec) / 4)});
+    if (!parts.empty()) stage_.download(parts);
 }
 
 void ContactDetector::minDistances(float* vf, float* face, float* edge) {
-    if (vf) {
-        const auto a = download(vfMin_, nv_, stream_);
-        std::memcpy(vf, a.data(), sizeof(float) * nv_);
-    }
-    if (face) {
-        const auto a = download(faceMin_, nf_, stream_);
-        std::memcpy(face, a.data(), sizeof(float) * nf_);
-    }
-    if (edge) {
-        const auto a = download(eeMin_, ne_, stream_);
-        std::memcpy(edge, a.data(), sizeof(float) * ne_);
-    }
+    if (!ready_) fail(GVBD_ERR_STATE, "detector not finalized");
+    std::vector<StagePart> parts;
+    if (vf) parts.push_back({StagePart::WORDS, vf, vfMin_, nv_});
+    if (face) parts.push_back({StagePart::WORDS, face, faceMin_, nf_});
+    if (edge) parts.push_back({StagePart::WORDS, edge, eeMin_, ne_});
+    if (!parts.empty()) stage_.download(parts);
 }
 
 void ContactDetector::boundsOut(float* b) {
-    const auto a = download(bounds_, nv_, stream_);
-    std::memcpy(b, a.data(), sizeof(float) * nv_);
+    if (!ready_) fail(GVBD_ERR_STATE, "detector not finalized");
+    stage_.download({{StagePart::WORDS, b, bounds_, nv_}});
 }
 
 }  // namespace gvbd

@@ -20,6 +20,7 @@
 #include "detector.h"
 #include "device_types.h"
 #include "errors.h"
+#include "host_stage.h"
 #include "kernels.h"
 #include "mesh_prep.h"
 #include "scene_io.h"
@@ -267,6 +268,8 @@ struct gvbd_context {
     int numCUs = 0;
     hipStream_t stream = nullptr;
     int* dStatus = nullptr;  // set by work-queue kernels when a dependency wait exceeds its limit
+    bool queueUsed = false;  // whether any work-queue kernel was launched or captured
+    std::unique_ptr<gvbd::HostStage> stage;
     double* convScratch = nullptr;  // this device's scratch of the allocation-free convergence evaluation
     hipEvent_t events[64] = {};
     std::string lastError;
@@ -368,6 +371,7 @@ void release_plan(PlanObj& p) {
 
 // Work-queue status: reports (and clears) a dependency wait that hit its spin limit.
 void check_queue_status(gvbd_context* ctx) {
+    if (!ctx->queueUsed) return;  // nothing has written it
     int st = 0;
     hip_check(hipMemcpy(&st, ctx->dStatus, sizeof(int), hipMemcpyDeviceToHost), "status read");
     if (st != 0) {
@@ -1310,6 +1314,7 @@ void plan_contact_snapshot(gvbd_context* ctx, PlanObj& p) {
 void plan_iteration(gvbd_context* ctx, PlanObj& p, int it, int epoch) {
     if (p.contact) plan_contact_snapshot(ctx, p);
     if (p.mode == GVBD_MODE_WORK_QUEUE) {
+        ctx->queueUsed = true;
         hip_check(launch_queue_solve(queue_args(ctx, p), it, epoch, p.queueGrid, p.lpv, p.block, ctx->stream),
                   "work-queue solve launch");
     } else {
@@ -1725,7 +1730,8 @@ void initialize_scene(gvbd_context* ctx, SceneObj& s, const std::function<void(s
     if (contact) {
         // ClothContactDetector over the scene's own positions (VBDClothPhysics initialize ->
         // ClothContactDetector::initialize, ClothContactDetector.cpp:944-1050)
-        s.cd = std::make_unique<ContactDetector>(ctx->device, ctx->stream, s.params.contact_query_radius, 8, 8);
+        s.cd = std::make_unique<ContactDetector>(ctx->device, ctx->stream, *ctx->stage, s.params.contact_query_radius,
+                                                 8, 8);
         s.cd->useExternalPositions(s.dev.pos);
         for (auto& mk : s.meshes) {
             if (mk.first == MESH_TET) {
@@ -1876,6 +1882,7 @@ int gvbd_context_create(int32_t device, gvbd_context** out) {
         hip_check(hipMalloc((void**)&ctx->dStatus, 256), "hipMalloc status");
         hip_check(hipMemset(ctx->dStatus, 0, 256), "status clear");
         hip_check(gvbd::convergence_scratch_init(device, &ctx->convScratch), "convergence scratch address");
+        ctx->stage = std::make_unique<gvbd::HostStage>(device, ctx->stream);
         *out = ctx.release();
     });
 }
@@ -1897,6 +1904,7 @@ int gvbd_context_destroy(gvbd_context* ctx) {
     for (auto& e : ctx->events)
         if (e) (void)hipEventDestroy(e);
     if (ctx->dStatus) (void)hipFree(ctx->dStatus);
+    ctx->stage.reset();
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return GVBD_OK;
@@ -2731,32 +2739,33 @@ static void mesh_state_io(gvbd_context* ctx, int32_t scene, int32_t mesh, float*
     if (!s.initialized) fail(GVBD_ERR_STATE, "scene not initialised");
     require(mesh >= 0 && mesh < (int32_t)s.meshes.size(), "mesh index out of range");
     const int32_t off = s.vertexOffset[mesh], n = s.meshVertices(mesh);
-    std::vector<float4> tmp(n);
-    hip_check(hipStreamSynchronize(ctx->stream), "sync");
-    check_queue_status(ctx);
     float4* dev[2] = {s.dev.pos + off, s.dev.vel + off};
     float* host[2] = {pos, vel};
+    if (s.dev.arena) {
+        if (ctx->queueUsed) {
+            hip_check(hipStreamSynchronize(ctx->stream), "sync");
+            check_queue_status(ctx);
+        }
+        std::vector<StagePart> parts;
+        for (int a = 0; a < 2; ++a)
+            if (host[a]) parts.push_back({StagePart::VEC3, host[a], dev[a], n});
+        if (get)
+            ctx->stage->download(parts);
+        else
+            ctx->stage->upload(parts);
+        return;
+    }
     // a scene its server holds in host memory is read and written there
-    const bool resident = s.dev.arena != nullptr;
-    auto held = [&](float4* d) { return s.hostCopy.data() + ((uintptr_t)d - s.hostCopyBase); };
+    hip_check(hipStreamSynchronize(ctx->stream), "sync");
+    check_queue_status(ctx);
     for (int a = 0; a < 2; ++a) {
         if (!host[a]) continue;
-        if (get) {
-            if (resident)
-                hip_check(hipMemcpy(tmp.data(), dev[a], sizeof(float4) * n, hipMemcpyDeviceToHost), "download");
+        float4* held = reinterpret_cast<float4*>(s.hostCopy.data() + ((uintptr_t)dev[a] - s.hostCopyBase));
+        for (int32_t i = 0; i < n; ++i) {
+            if (get)
+                std::memcpy(host[a] + 3 * (int64_t)i, held + i, 3 * sizeof(float));
             else
-                std::memcpy(tmp.data(), held(dev[a]), sizeof(float4) * n);
-            for (int32_t i = 0; i < n; ++i) {
-                host[a][3 * i] = tmp[i].x;
-                host[a][3 * i + 1] = tmp[i].y;
-                host[a][3 * i + 2] = tmp[i].z;
-            }
-        } else {
-            for (int32_t i = 0; i < n; ++i) tmp[i] = make_float4(host[a][3 * i], host[a][3 * i + 1], host[a][3 * i + 2], 0.f);
-            if (resident)
-                hip_check(hipMemcpy(dev[a], tmp.data(), sizeof(float4) * n, hipMemcpyHostToDevice), "upload");
-            else
-                std::memcpy(held(dev[a]), tmp.data(), sizeof(float4) * n);
+                held[i] = make_float4(host[a][3 * i], host[a][3 * i + 1], host[a][3 * i + 2], 0.f);
         }
     }
 }
@@ -3540,8 +3549,8 @@ int gvbd_cd_create(gvbd_context* ctx, float max_query_distance, int32_t vf_capac
     return guard(ctx, [&] {
         require(ctx != nullptr && cd_out != nullptr, "NULL argument");
         hip_check(hipSetDevice(ctx->device), "hipSetDevice");
-        auto d = std::make_unique<ContactDetector>(ctx->device, ctx->stream, max_query_distance, vf_capacity,
-                                                   ee_capacity);
+        auto d = std::make_unique<ContactDetector>(ctx->device, ctx->stream, *ctx->stage, max_query_distance,
+                                                   vf_capacity, ee_capacity);
         const int32_t id = ctx->nextDetector++;
         ctx->detectors[id] = std::move(d);
         *cd_out = id;
