@@ -772,6 +772,11 @@ def main():
         t = json.load(open(side)).get("schedules", {}).get(key)
         if t:
             roof["traffic"] = t["hbm_bytes_per_launch"]
+            # the gather model counts neighbour positions that the caches serve: the DRAM rate is the
+            # measured traffic's
+            roof["gather_model_gbs"] = roof["achieved"]
+            roof["achieved"] = round(t["hbm_bytes_per_launch"] / (roof["avg_launch_us"] * 1e-6) / 1e9, 1)
+            roof["frac"] = round(roof["achieved"] / HBM_PEAK_GBS, 4)
     # achievable-bandwidth reference points: the library's streaming copy kernel and the runtime's
     # device-to-device copy (each moves 2 x copy_bytes per copy)
     copy_ms = ctx.stream_copy_ms(args.copy_bytes, reps=5)

@@ -4,10 +4,11 @@
 //   build   scene box of primitive centroids -> 30-bit Morton codes in the box (the 10-bit-per-
 //           axis interleave of BVH/MortonCode.h:9-31) with the primitive id in the low 32 bits ->
 //           device radix sort -> binary radix tree from the sorted keys (Karras 2012, HPG) ->
-//           node depths -> internal nodes sorted by depth (the refit schedule)
-//   refit   leaf boxes from the current positions, then one launch per depth level, deepest
-//           first (no atomics, no inter-block waits)
-//   query   waves of up to 64 vertices (VF, query box of half-size r around the vertex) or edges
+//           lists of the nodes that cross blocks of leaves (the refit), node depths
+//   refit   a block per 1,024 leaves: their boxes from the current positions and all nodes within
+//           them, climbing in LDS; then a launch per tier for nodes that cross blocks (no
+//           inter-block waits)
+//   query   waves of 8 to 32 vertices (VF, query box of half-size r around the vertex) or edges
 //           (EE, the segment's box grown by r), traversal shared by the wave, exact tests with the
 //           reference's predicates (ClothContactDetector.cpp:144-288, 731-813; CollisionGeometry.h:
 //           90-267; TriMeshCollisionGeometry.cpp:7-186)
@@ -442,7 +443,7 @@ __global__ __launch_bounds__(256) void ee_record_kernel(CDView S) {
 // to. The stack stays sorted by depth (what a step pushes is deeper than all that it left), so that
 // it holds little more than 64 entries per level; when it runs full a step pops fewer, down to one
 // (depth first), which needs at most one more entry per level: the reserve. So a tree of any depth
-// that the refit schedule takes fits.
+// that the build takes fits.
 constexpr int kWaveReserve = kMaxDepth + 2;
 __device__ __forceinline__ int wave_pop(int size, int cap) {
     return min(min(64, size), max(cap - kWaveReserve - size, 1));
@@ -499,7 +500,7 @@ __device__ __forceinline__ void wave_queries(const BvhPair* pairs, int n, bool a
             }
             const unsigned long long mA = __ballot(inA), mB = __ballot(inB);
             const int kids = __popcll(mA) + __popcll(mB);
-            if (base + kids > kQueryStack) {  // a tree deeper than the refit schedule supports
+            if (base + kids > kQueryStack) {  // a tree deeper than the build lets pass
                 if (lane == 0) atomicOr(error, 1);
                 break;
             }
@@ -1739,7 +1740,7 @@ __device__ __forceinline__ void wave_traverse(const BvhNode* nodes, const int* r
         }
         const unsigned long long grow = __ballot(left >= 0);
         const int kids = 2 * __popcll(grow);
-        if (base + kids > kWaveStack) {  // a tree deeper than the refit schedule supports
+        if (base + kids > kWaveStack) {  // a tree deeper than the build lets pass
             if (lane == 0) atomicOr(error, 1);
             break;
         }
