@@ -337,7 +337,7 @@ __device__ __forceinline__ void tet_block(const SceneView& S, float4* posInOut, 
     if (moved) {
         f3 dx;
         float step = sp.stepSize;
-        if (!solve_sym3<false>(h, f, dx)) {
+        if (!solve_sym3<CONTACT>(h, f, dx)) {
             // the 3x3 block is singular: gradient step (VBDPhysics.cpp:2449-2466), counted
             step = sp.stepSizeGD;
             dx = f;

@@ -43,7 +43,7 @@ struct DeviceScene {
     uint8_t* vflag = nullptr;
     int4* slots = nullptr;
     TetInc* tinc = nullptr;
-    TetRow* trow = nullptr;    // instead of tinc (scenes with material damping or the accelerator)
+    TetRow* trow = nullptr;    // instead of tinc (scenes that use rows, see TetRow)
     float* tvol = nullptr;     // per row record: rest volume of its tet
     float4* tmat = nullptr;    // per tet mesh: (mu, lambda, a, 0)
     ClothSlot* cslots = nullptr;
@@ -552,7 +552,7 @@ void upload_scene(gvbd_context* ctx, SceneObj& s, const std::function<void(size_
     const int32_t G = (int32_t)s.groups.size();
     std::vector<int4> slots;
     TetRecords recs;
-    recs.rows = s.params.use_accelerator != 0;
+    recs.rows = s.params.use_accelerator != 0 || s.params.handle_collision != 0;
     for (const TetMeshHost& m : s.tets)
         if (m.mat.dampingHydrostatic != 0.f || m.mat.dampingDeviatoric != 0.f) recs.rows = true;
     std::vector<ClothSlot> cslots;

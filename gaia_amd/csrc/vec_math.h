@@ -33,10 +33,11 @@ __device__ __forceinline__ f3 sym_mul(const Sym3& h, f3 v) {
 // VBDPhysicsCompute.cu:896), whose source is not available: failure iff the
 // determinant is not finite or |det| <= 1e-12 |h_xx h_yy h_zz|. Returns false on
 // failure, and then the caller takes a gradient step (VBDPhysics.cpp:2452-2459).
-// CLOTH: the order in which the determinant's products fuse. Left to the compiler, which of two
-// products it fuses with their sum differs between the tet and the cloth kernels and from build to
-// build; each keeps the one it had.
-template <bool CLOTH>
+// XX_FIRST: the order in which the determinant's products fuse. Left to the compiler, which of two
+// products it fuses with their sum differs between kernels and from build to build; each keeps the one it
+// had: h_xx C00 rounded first in the cloth solve and in the tet solve of contact scenes, h_xy C01 in the
+// plain tet solve.
+template <bool XX_FIRST>
 __device__ __forceinline__ bool solve_sym3(const Sym3& h, f3 b, f3& x) {
     const float C00 = h.yy * h.zz - h.yz * h.yz;
     const float C01 = h.yz * h.xz - h.xy * h.zz;
@@ -44,7 +45,7 @@ __device__ __forceinline__ bool solve_sym3(const Sym3& h, f3 b, f3& x) {
     const float C11 = h.xx * h.zz - h.xz * h.xz;
     const float C12 = h.xy * h.xz - h.xx * h.yz;
     const float C22 = h.xx * h.yy - h.xy * h.xy;
-    const float det = fmaf(h.xz, C02, CLOTH ? fmaf(h.xy, C01, h.xx * C00) : fmaf(h.xx, C00, h.xy * C01));
+    const float det = fmaf(h.xz, C02, XX_FIRST ? fmaf(h.xy, C01, h.xx * C00) : fmaf(h.xx, C00, h.xy * C01));
     const float scale = fabsf(h.xx * h.yy * h.zz);
     if (!isfinite(det) || !(fabsf(det) > 1e-12f * scale)) return false;
     const float inv = 1.0f / det;

@@ -448,8 +448,8 @@ GVBD_API int gvbd_batch_update_velocities(gvbd_context* ctx, int32_t batch);
 GVBD_API int gvbd_batch_solve_parallel_group(gvbd_context* ctx, int32_t batch, int32_t group, int32_t iteration);
 GVBD_API int gvbd_batch_num_parallel_groups(gvbd_context* ctx, int32_t batch, int32_t* n);
 /* algorithmic bytes of one solve launch `group` and its vertex count (gather model: per tet
- * vertex 72 B + 68 B per incident tet (88 B in scenes with material damping or the accelerator),
- * per cloth vertex 60 B + 56 B per face + 116 B per bending stencil) */
+ * vertex 72 B + 68 B per incident tet (88 B in scenes with material damping, the accelerator or
+ * collision handling), per cloth vertex 60 B + 56 B per face + 116 B per bending stencil) */
 GVBD_API int gvbd_batch_group_work(gvbd_context* ctx, int32_t batch, int32_t group, int64_t* bytes, int64_t* vertices);
 
 /* ---- serving loop: continuous batching of step requests ----
