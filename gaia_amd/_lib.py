@@ -250,6 +250,7 @@ _SIGNATURES = {
     "gvbd_scene_set_schedule": [_P, _I, _I, _I],
     "gvbd_scene_set_schedule_ex": [_P, _I, _SCHED],
     "gvbd_scene_get_schedule": [_P, _I, _SCHED],
+    "gvbd_scene_plan_info": [_P, _I, c_int32_p, c_int32_p],
     "gvbd_scene_run_step": [_P, _I],
     "gvbd_scene_run_steps": [_P, _I, _I],
     "gvbd_scene_apply_initial_step": [_P, _I],
@@ -283,6 +284,7 @@ _SIGNATURES = {
     "gvbd_batch_set_schedule_ex": [_P, _I, _SCHED],
     "gvbd_batch_get_schedule": [_P, _I, _SCHED],
     "gvbd_batch_queue_info": [_P, _I, c_int32_p, c_int32_p],
+    "gvbd_batch_plan_info": [_P, _I, c_int32_p, c_int32_p],
     "gvbd_batch_record_graph": [_P, _I, _I],
     "gvbd_batch_run_steps": [_P, _I, _I],
     "gvbd_batch_apply_initial_step": [_P, _I],

@@ -202,8 +202,8 @@ struct ContactView {
     HbmPtr<const float> bound;       // per vertex conservative bound
     HbmPtr<const float4> xAtCD;      // positions at the last detection
     HbmPtr<int> flag;                // set when a vertex is truncated: detect before the next iteration
-    // Vertices of contact scenes are updated in place (cloth with one colour per group, and no
-    // attachments; a launch per group that copies positionsNext costs 4.7 us); a contact pair may join two
+    // Vertices of contact scenes are updated in place (cloth with one colour per group that
+    // shares no element, and no attachments; a launch per group that copies positionsNext costs 4.7 us); a contact pair may join two
     // of one parallel group, so contact partners of the solving vertex's own group are read from
     // the iteration-start snapshot (their value at the start of the group, as the reference's
     // positionsNext + copy gives); vgroup: per vertex parallel group (-1: not solved), also in

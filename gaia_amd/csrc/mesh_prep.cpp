@@ -570,6 +570,15 @@ bool prepare_cloth_mesh(ClothMeshHost& m, std::string& err) {
     return true;
 }
 
+bool colors_separate_elements(const ClothMeshHost& m) {
+    for (const TriEdge& e : m.edges) {
+        if (m.colors[e.v1] == m.colors[e.v2]) return false;
+        // (the edges of a stencil's two faces are in the list themselves)
+        if (e.v21Next >= 0 && e.v21Next != e.v12Next && m.colors[e.v12Next] == m.colors[e.v21Next]) return false;
+    }
+    return true;
+}
+
 Graph tri_vertex_graph(int32_t nv, int32_t nf, const int32_t* faces, bool withBending) {
     std::vector<std::pair<uint64_t, int32_t>> occ;  // (edge key, opposite vertex)
     occ.reserve(3 * (size_t)nf);

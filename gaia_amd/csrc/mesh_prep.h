@@ -124,6 +124,9 @@ struct ClothMeshHost {
 // (Q = 3 K0 K0^T / (|n1| + |n2|)). Fails on degenerate faces or non-manifold / inconsistently
 // oriented meshes.
 bool prepare_cloth_mesh(ClothMeshHost& m, std::string& err);
+// Whether no two vertices of one colour share an element of a prepared mesh (a face, or the stencil of an
+// interior edge). Colours from outside need not keep them apart.
+bool colors_separate_elements(const ClothMeshHost& m);
 
 // Edges of a triangle mesh numbered by first appearance over the faces (TriMesh.cpp:481-560):
 // v1 -> v2 is the edge's direction in its first face f1, v12Next that face's third vertex,

@@ -25,8 +25,9 @@
 //   StVK: H = A [(m^T S m) I + mu |m|^2 F F^T + (mu + lambda)(F m)(F m)^T];  f = -A F S m.
 // One launch covers one parallel group of every scene of a plan; each block's work item is
 // either tet slots (updated in place: vertices of one colour share no tet, as in the
-// reference CPU path) or cloth slots (in place too where a mesh has one colour in the group, else
-// written to pnext and copied back after the group, the reference's positionsNext scheme). Plans of
+// reference CPU path) or cloth slots (in place too where a mesh has one colour in the group and its
+// colours keep the vertices of every element apart, else written to pnext and copied back after the group, the
+// reference's positionsNext scheme). Plans of
 // small scenes take one block per scene and one launch per frame.
 #include <hip/hip_runtime.h>
 

@@ -198,6 +198,7 @@ struct PlanObj {
     SceneRun* dRuns = nullptr;
     WorkItem* dRunItems = nullptr;
     int32_t nRuns = 0, runVerts = 0;
+    int32_t nCommitSlots = 0;  // cloth slots solved through positionsNext, per iteration
     // work queue (mode GVBD_MODE_WORK_QUEUE)
     QueueEntry* dQueue = nullptr;
     int* dCounters = nullptr;  // tickets[iterations] then progress[scenes]
@@ -638,12 +639,17 @@ void upload_scene(gvbd_context* ctx, SceneObj& s, const std::function<void(size_
             attBegin.push_back((int32_t)att.size());
         }
     }
+    std::vector<uint8_t> separate(s.meshes.size(), 0);
+    for (size_t im = 0; im < s.meshes.size(); ++im)
+        if (s.meshes[im].first == MESH_CLOTH) separate[im] = colors_separate_elements(s.cloths[s.meshes[im].second]);
     for (int32_t g = 0; g < G; ++g) {
         const auto& grp = s.groups[g];
-        // A cloth mesh with a single colour in this group can be updated in place: its solved
-        // vertices share no element, so the reference's positionsNext + copy (Jacobi over the
-        // group) gives the same result. Meshes interact by contact alone, whose partners of the own
-        // group are read from the iteration-start snapshot (ContactView::snap).
+        // A cloth mesh with a single colour in this group can be updated in place if its colours keep
+        // the vertices of every element apart: the reference's positionsNext + copy (Jacobi over the
+        // group) gives the same result then. (Given colours may leave the bending stencils out; in place,
+        // a vertex would then be read by one wave and written by another.) Meshes interact by contact
+        // alone, whose partners of the own group are read from the iteration-start snapshot
+        // (ContactView::snap).
         std::vector<int32_t> firstColor(s.meshes.size(), -1);
         std::vector<uint8_t> multiColor(s.meshes.size(), 0);
         for (size_t i = 0; i + 1 < grp.size(); i += 2) {
@@ -662,7 +668,7 @@ void upload_scene(gvbd_context* ctx, SceneObj& s, const std::function<void(size_
                               tetWork, contact ? &trefs[im] : nullptr);
             } else {
                 // attachments read other vertices of the group: positionsNext keeps them Jacobi
-                const bool inplace = !multiColor[im] && attOf.empty();
+                const bool inplace = separate[im] && !multiColor[im] && attOf.empty();
                 emit_cloth_slot(s.cloths[s.meshes[im].second], off, lv, inplace, cslots, cface, cbend, clothWork,
                                 contact ? &refs[im] : nullptr);
                 if (!attOf.empty() && !attOf[off + lv].empty()) cslots.back().a.w |= SLOT_ATTACH;
@@ -1064,8 +1070,10 @@ void build_plan(gvbd_context* ctx, PlanObj& p) {
     p.numGroups = 0;
     p.accel = false;
     p.contact = p.clothContact = false;
+    p.nCommitSlots = 0;
     for (int32_t sid : p.scenes) {
         SceneObj& s = scene_of(ctx, sid);
+        p.nCommitSlots += (int32_t)std::count(s.clothSlotInplace.begin(), s.clothSlotInplace.end(), 0);
         if (s.cd) {
             p.contact = true;
             if (!s.cd->penetration()) p.clothContact = true;
@@ -3037,6 +3045,23 @@ int gvbd_batch_queue_info(gvbd_context* ctx, int32_t batch, int32_t* entries, in
         build_plan(ctx, p);
         if (entries) *entries = p.nQueue;
         if (grid) *grid = p.queueGrid;
+    });
+}
+
+static void plan_info(gvbd_context* ctx, PlanObj& p, int32_t* whole_frames, int32_t* commit_slots) {
+    build_plan(ctx, p);
+    if (whole_frames) *whole_frames = p.nRuns > 0 ? 1 : 0;
+    if (commit_slots) *commit_slots = p.nCommitSlots;
+}
+
+int gvbd_scene_plan_info(gvbd_context* ctx, int32_t scene, int32_t* whole_frames, int32_t* commit_slots) {
+    return guard(ctx, [&] { plan_info(ctx, scene_plan(ctx, scene), whole_frames, commit_slots); });
+}
+
+int gvbd_batch_plan_info(gvbd_context* ctx, int32_t batch, int32_t* whole_frames, int32_t* commit_slots) {
+    return guard(ctx, [&] {
+        require(ctx != nullptr, "ctx is NULL");
+        plan_info(ctx, batch_plan(ctx, batch), whole_frames, commit_slots);
     });
 }
 

@@ -598,6 +598,13 @@ class VBDPhysics:
         self.ctx.check(lib().gvbd_scene_get_schedule(self.ctx.handle, self.scene, ctypes.byref(sc)))
         return schedule_dict(sc)
 
+    def planInfo(self):
+        """(whether frames are stepped whole by one block, cloth vertices per iteration solved through
+        positionsNext and copied back) of the current schedule."""
+        w, c = ctypes.c_int32(), ctypes.c_int32()
+        self.ctx.check(lib().gvbd_scene_plan_info(self.ctx.handle, self.scene, ctypes.byref(w), ctypes.byref(c)))
+        return bool(w.value), c.value
+
     def runIteration(self, iIter):
         """One VBD iteration (every parallel group in order) after applyInitialStep."""
         self.ctx.check(lib().gvbd_scene_run_iteration(self.ctx.handle, self.scene, iIter))
@@ -769,6 +776,12 @@ class Batch:
         e, g = ctypes.c_int32(), ctypes.c_int32()
         self.ctx.check(lib().gvbd_batch_queue_info(self.ctx.handle, self.batch, ctypes.byref(e), ctypes.byref(g)))
         return e.value, g.value
+
+    def plan_info(self):
+        """VBDPhysics.planInfo of the batch (one block per scene)."""
+        w, c = ctypes.c_int32(), ctypes.c_int32()
+        self.ctx.check(lib().gvbd_batch_plan_info(self.ctx.handle, self.batch, ctypes.byref(w), ctypes.byref(c)))
+        return bool(w.value), c.value
 
     def record_graph(self, enable=True):
         self.ctx.check(lib().gvbd_batch_record_graph(self.ctx.handle, self.batch, 1 if enable else 0))

@@ -327,6 +327,10 @@ GVBD_API int gvbd_scene_set_schedule(gvbd_context* ctx, int32_t scene, int32_t l
 /* full schedule (mode, work-queue entry size, persistent grid); drops a recorded graph */
 GVBD_API int gvbd_scene_set_schedule_ex(gvbd_context* ctx, int32_t scene, const gvbd_schedule* schedule);
 GVBD_API int gvbd_scene_get_schedule(gvbd_context* ctx, int32_t scene, gvbd_schedule* schedule);
+/* how the current schedule steps the scene: whether its frames are stepped whole by one block (one launch
+ * per frame), and how many cloth vertices an iteration solves through a second position array and a copy
+ * (those of meshes whose colours put two vertices of an element into one group, or with attachments) */
+GVBD_API int gvbd_scene_plan_info(gvbd_context* ctx, int32_t scene, int32_t* whole_frames, int32_t* commit_slots);
 
 /* ---- stepping (asynchronous on the context stream) ---- */
 GVBD_API int gvbd_scene_run_step(gvbd_context* ctx, int32_t scene);               /* all substeps of one frame */
@@ -434,6 +438,8 @@ GVBD_API int gvbd_batch_set_schedule_ex(gvbd_context* ctx, int32_t batch, const 
 GVBD_API int gvbd_batch_get_schedule(gvbd_context* ctx, int32_t batch, gvbd_schedule* schedule);
 /* work-queue size of one iteration and the persistent grid (blocks) of the current schedule */
 GVBD_API int gvbd_batch_queue_info(gvbd_context* ctx, int32_t batch, int32_t* entries, int32_t* grid);
+/* as gvbd_scene_plan_info, one block per scene */
+GVBD_API int gvbd_batch_plan_info(gvbd_context* ctx, int32_t batch, int32_t* whole_frames, int32_t* commit_slots);
 GVBD_API int gvbd_batch_record_graph(gvbd_context* ctx, int32_t batch, int32_t enable);
 GVBD_API int gvbd_batch_run_steps(gvbd_context* ctx, int32_t batch, int32_t n);
 /* per-iteration hooks over every scene of the batch (as the gvbd_scene_ forms) */
