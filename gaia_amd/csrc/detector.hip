@@ -494,7 +494,9 @@ __device__ __forceinline__ void wave_queries(const BvhPair* pairs, int n, bool a
                 }
                 if (overlap(q, P.lo1, P.hi1)) {
                     lfB = __float_as_int(P.hi1.w) != 0;
-                    inB = !lfB;
+                    // (the root is nobody's child: the empty second child of a one-leaf tree, whose box a
+                    // query of infinite extent overlaps too)
+                    inB = !lfB && __float_as_int(P.lo1.w) != 0;
                     nextB = ((unsigned)q << kBits) | (unsigned)__float_as_int(P.lo1.w);
                 }
             }

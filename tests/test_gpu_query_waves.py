@@ -33,6 +33,23 @@ CASES = {
 }
 
 
+def test_one_face_within_the_largest_distance(gpu_ctx):
+    """A tree of one leaf, and query boxes that overflow to infinity in every direction."""
+    tri = np.array([[0, 0, 0], [1, 0, 0], [0, 1, 0]], np.float32)
+    points = np.array([[0.25, 0.25, 2.0], [-3.0, 0.0, 0.0], [1.5, 1.5, 0.0]], np.float32)
+    cd = ContactDetector(gpu_ctx, [(tri, np.array([[0, 1, 2]], np.int32)), (points, np.zeros((0, 3), np.int32))],
+                         max_query_dis=np.finfo(np.float32).max)
+    cd.updateBVH(True)
+    cd.query()
+    want = np.array([2.0, 3.0, np.sqrt(2.0)], np.float32)
+    vertex, face, _ = cd.min_distances()
+    np.testing.assert_allclose(vertex[3:], want, rtol=1e-6)
+    np.testing.assert_allclose(face, [want.min()], rtol=1e-6)
+    vc, vr, _, _ = cd.results()
+    assert vc.tolist() == [0, 0, 0, 1, 1, 1] and (vr["face"][3:, 0] == 0).all()
+    cd.destroy()
+
+
 @pytest.mark.parametrize("name", list(CASES))
 @pytest.mark.parametrize("cap", [1, 8, 16])
 def test_wave_queries_equal_the_record_pass(gpu_ctx, name, cap):
