@@ -235,6 +235,7 @@ _SIGNATURES = {
     "gvbd_last_error": [_P],
     "gvbd_synchronize": [_P],
     "gvbd_context_memory": [_P, c_int64_p],
+    "gvbd_context_page_locked_transfers": [_P, _I],
     "gvbd_scene_device_bytes": [_P, _I, c_int64_p, c_int64_p],
     "gvbd_scene_create": [_P, ctypes.POINTER(PhysicsParams), c_int32_p],
     "gvbd_scene_destroy": [_P, _I],

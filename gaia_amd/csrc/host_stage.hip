@@ -63,9 +63,30 @@ void launch_piece(const Piece& p, char* slot, bool down, hipStream_t stream) {
 }  // namespace
 
 HostStage::~HostStage() {
+    release();
     for (hipEvent_t e : done_)
         if (e) (void)hipEventDestroy(e);
+}
+
+void HostStage::release() {
     if (buf_) (void)hipHostFree(buf_);
+    buf_ = nullptr;
+}
+
+void HostStage::usePageLocked(bool on) {
+    std::lock_guard<std::mutex> lock(mutex_);
+    pageLocked_ = on;
+    if (!on) release();  // no transfer is under way
+}
+
+bool HostStage::allocated() {
+    if (buf_) return true;
+    for (hipEvent_t& e : done_)
+        if (!e) hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "event create");
+    if (hipHostMalloc((void**)&buf_, kSlots * kSlotBytes, hipHostMallocDefault) == hipSuccess) return true;
+    (void)hipGetLastError();
+    buf_ = nullptr;
+    return false;
 }
 
 void HostStage::transfer(const std::vector<StagePart>& parts, bool down) {
@@ -73,15 +94,35 @@ void HostStage::transfer(const std::vector<StagePart>& parts, bool down) {
     int current = 0;
     hip_check(hipGetDevice(&current), "hipGetDevice");
     if (current != device_) hip_check(hipSetDevice(device_), "hipSetDevice");
-    if (!buf_) {
-        for (hipEvent_t& e : done_)
-            if (!e) hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "event create");
-        if (hipHostMalloc((void**)&buf_, kSlots * kSlotBytes, hipHostMallocDefault) != hipSuccess) {
-            (void)hipGetLastError();
-            buf_ = nullptr;
-            fail(GVBD_ERR_NOMEM, "pinned host allocation for transfers failed");
-        }
+    if (pageLocked_ && allocated())
+        staged(parts, down);
+    else
+        plain(parts, down);
+    if (current != device_) hip_check(hipSetDevice(current), "hipSetDevice");
+}
+
+void HostStage::plain(const std::vector<StagePart>& parts, bool down) {
+    std::vector<float4> wide;
+    for (const StagePart& p : parts) {
+        const bool vec = p.kind == StagePart::VEC3;
+        float* host = (float*)p.host;
+        if (vec) wide.resize(p.count);
+        if (vec && !down)
+            for (int64_t i = 0; i < p.count; ++i) wide[i] = make_float4(host[3 * i], host[3 * i + 1], host[3 * i + 2], 0.f);
+        void* mem = vec ? (void*)wide.data() : p.host;
+        const size_t bytes = (size_t)p.count * (vec ? sizeof(float4) : 4);
+        if (bytes)
+            hip_check(hipMemcpyAsync(down ? mem : p.device, down ? p.device : mem, bytes,
+                                     down ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice, stream_),
+                      "transfer");
+        hip_check(hipStreamSynchronize(stream_), "transfer wait");
+        if (vec && down)
+            for (int64_t i = 0; i < p.count; ++i) std::memcpy(host + 3 * i, &wide[i], 3 * sizeof(float));
     }
+    if (parts.empty()) hip_check(hipStreamSynchronize(stream_), "transfer wait");
+}
+
+void HostStage::staged(const std::vector<StagePart>& parts, bool down) {
     std::vector<Piece> pieces;
     for (const StagePart& p : parts) {
         const size_t hostSize = p.kind == StagePart::VEC3 ? 12 : 4, deviceSize = p.kind == StagePart::VEC3 ? 16 : 4;
@@ -118,7 +159,6 @@ void HostStage::transfer(const std::vector<StagePart>& parts, bool down) {
     }
     // also for an empty transfer: the work queued before it is complete
     if (!down || n == 0) hip_check(hipStreamSynchronize(stream_), "transfer wait");
-    if (current != device_) hip_check(hipSetDevice(current), "hipSetDevice");
 }
 
 }  // namespace gvbd

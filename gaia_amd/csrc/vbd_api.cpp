@@ -1928,6 +1928,13 @@ int gvbd_synchronize(gvbd_context* ctx) {
     });
 }
 
+int gvbd_context_page_locked_transfers(gvbd_context* ctx, int32_t enable) {
+    return guard(ctx, [&] {
+        require(ctx != nullptr, "ctx is NULL");
+        ctx->stage->usePageLocked(enable != 0);
+    });
+}
+
 int gvbd_context_memory(gvbd_context* ctx, int64_t* bytes) {
     return guard(ctx, [&] {
         require(ctx && bytes, "NULL argument");

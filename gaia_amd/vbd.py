@@ -176,6 +176,11 @@ class Context:
         self.check(lib().gvbd_context_memory(self.handle, ctypes.byref(b)))
         return b.value
 
+    def page_locked_transfers(self, enable):
+        """Whether state and result transfers go through the context's page-locked memory (the default)
+        or are plain copies."""
+        self.check(lib().gvbd_context_page_locked_transfers(self.handle, 1 if enable else 0))
+
     def stream_copy_ms(self, nbytes, reps=5, method=0):
         """Average time of a device copy of nbytes (measured copy bandwidth): method 0 the
         library's streaming kernel, 1 the runtime's device-to-device hipMemcpyAsync."""

@@ -237,6 +237,10 @@ GVBD_API const char* gvbd_last_error(const gvbd_context* ctx);
 GVBD_API int gvbd_synchronize(gvbd_context* ctx);
 /* device bytes currently held by scenes and plans of this context */
 GVBD_API int gvbd_context_memory(gvbd_context* ctx, int64_t* bytes);
+/* Transfers of states, detector positions and results use 4 MB of page-locked host memory per context (on by
+ * default; plain copies, 15 to 30 us slower each, where it cannot be allocated). 0 gives that memory back and uses
+ * plain copies from then on. */
+GVBD_API int gvbd_context_page_locked_transfers(gvbd_context* ctx, int32_t enable);
 /* device bytes of one scene as a server's memory budget counts them (no reference counterpart):
  * its arena (0 while not uploaded or copied out) and its contact detector (trees and detection
  * lists, resident while the scene exists); its launch plans are not included */
