@@ -225,8 +225,9 @@ class ContactDetector {
     hipStream_t stream() const { return stream_; }
 
   private:
-    // kind 0 faces, 1 edges, 3 tets, 4 faces over their path from `prev`
+    void read(std::vector<StagePart> parts);  // results to the caller's arrays
     void allocBuildScratch(const std::vector<int>& sizes);
+    // kind 0 faces, 1 edges, 3 tets, 4 faces over their path from `prev`
     void buildBvh(DeviceBvh& b, int kind, const float4* prev = nullptr);
     void refitBvh(DeviceBvh& b, int kind, hipStream_t stream, const float4* prev = nullptr,
                   const int* gate = nullptr);

@@ -3023,34 +3023,34 @@ void ContactDetector::eeContactsAll(int32_t* ee, float* mu, float* d) {
     }
 }
 
-void ContactDetector::vfContactsCapped(int32_t* count, VFContactRec* rec) {
+// The parts that have elements; nothing to read is no error, also before finalize().
+void ContactDetector::read(std::vector<StagePart> parts) {
+    parts.erase(std::remove_if(parts.begin(), parts.end(),
+                               [](const StagePart& p) { return p.host == nullptr || p.count == 0; }),
+                parts.end());
+    if (parts.empty()) return;
     if (!ready_) fail(GVBD_ERR_STATE, "detector not finalized");
-    std::vector<StagePart> parts;
-    if (count) parts.push_back({StagePart::WORDS, count, vfStored_, nv_});
-    if (rec) parts.push_back({StagePart::WORDS, rec, vfRec_, (int64_t)nv_ * vfCap_ * (int64_t)(sizeof(VFContactRec) / 4)});
-    if (!parts.empty()) stage_.download(parts);
+    stage_.download(parts);
+}
+
+void ContactDetector::vfContactsCapped(int32_t* count, VFContactRec* rec) {
+    read({{StagePart::WORDS, count, vfStored_, nv_},
+          {StagePart::WORDS, rec, vfRec_, (int64_t)nv_ * vfCap_ * (int64_t)(sizeof(VFContactRec) / 4)}});
 }
 
 void ContactDetector::eeContactsCapped(int32_t* count, EEContactRec* rec) {
-    if (!ready_) fail(GVBD_ERR_STATE, "detector not finalized");
-    std::vector<StagePart> parts;
-    if (count) parts.push_back({StagePart::WORDS, count, eeStored_, ne_});
-    if (rec) parts.push_back({StagePart::WORDS, rec, eeRec_, (int64_t)ne_ * eeCap_ * (int64_t)(sizeof(EEContactRec) / 4)});
-    if (!parts.empty()) stage_.download(parts);
+    read({{StagePart::WORDS, count, eeStored_, ne_},
+          {StagePart::WORDS, rec, eeRec_, (int64_t)ne_ * eeCap_ * (int64_t)(sizeof(EEContactRec) / 4)}});
 }
 
 void ContactDetector::minDistances(float* vf, float* face, float* edge) {
-    if (!ready_) fail(GVBD_ERR_STATE, "detector not finalized");
-    std::vector<StagePart> parts;
-    if (vf) parts.push_back({StagePart::WORDS, vf, vfMin_, nv_});
-    if (face) parts.push_back({StagePart::WORDS, face, faceMin_, nf_});
-    if (edge) parts.push_back({StagePart::WORDS, edge, eeMin_, ne_});
-    if (!parts.empty()) stage_.download(parts);
+    read({{StagePart::WORDS, vf, vfMin_, nv_},
+          {StagePart::WORDS, face, faceMin_, nf_},
+          {StagePart::WORDS, edge, eeMin_, ne_}});
 }
 
 void ContactDetector::boundsOut(float* b) {
-    if (!ready_) fail(GVBD_ERR_STATE, "detector not finalized");
-    stage_.download({{StagePart::WORDS, b, bounds_, nv_}});
+    read({{StagePart::WORDS, b, bounds_, nv_}});
 }
 
 }  // namespace gvbd
