@@ -74,20 +74,21 @@ struct DeviceBvh {
     RefitTop* top = nullptr;         // the tiers' lists
     int* topCount = nullptr;         // per list: its entries
     int topMost[4] = {0, 0, 0, 0};   // host: longest list per tier
+    uint64_t* keysAlt = nullptr;     // n (sorted Morton keys)
+    // Face trees of penetration contact: the mesh of every face below a node (2n - 1), -1 where faces of
+    // several meshes meet, set level by level at every build
+    int* mesh = nullptr;
     int* levelNodes = nullptr;       // internal nodes ordered by depth, deepest first
     std::vector<int> levelBegin;     // host: ranges of levelNodes per depth (deepest first)
     int* dLevelBegin = nullptr;      // the same ranges on the device
     std::vector<std::pair<int, int>> segments;  // launches over the levels: [first, last) level runs
-    uint64_t* keysAlt = nullptr;     // n (sorted Morton keys)
-    int* mesh = nullptr;             // 2n - 1 (face trees of penetration contact): the mesh of every
-                                     // face below the node, -1 where faces of several meshes meet
 };
 
 // Buffers of the tree builds (one set per detector).
 struct BvhScratch {
-    int* jump = nullptr;  // 4 (n - 1): depth / ancestor buffers of the depth computation
+    int* jump = nullptr;  // 2 (n - 1): lists and places of the refit's nodes; trees with levels 4 (n - 1):
+                          // depths and ancestors
     uint64_t *keys = nullptr, *depthKeys = nullptr, *depthKeysAlt = nullptr;
-    int* depth = nullptr;
     void* sortTemp = nullptr;
     size_t sortTempBytes = 0;
 };
@@ -226,9 +227,10 @@ class ContactDetector {
 
   private:
     void read(std::vector<StagePart> parts);  // results to the caller's arrays
-    void allocBuildScratch(const std::vector<int>& sizes);
+    void allocBuildScratch(const std::vector<int>& sizes, int levelled);
     // kind 0 faces, 1 edges, 3 tets, 4 faces over their path from `prev`
     void buildBvh(DeviceBvh& b, int kind, const float4* prev = nullptr);
+    void nodeMeshes(DeviceBvh& b);
     void refitBvh(DeviceBvh& b, int kind, hipStream_t stream, const float4* prev = nullptr,
                   const int* gate = nullptr);
     void allocBvh(DeviceBvh& b, int n, bool pairs);
@@ -289,7 +291,7 @@ class ContactDetector {
     float* recEEd_ = nullptr;
     bool recorded_ = false;
     int* error_ = nullptr;      // bit 0: traversal stack overflow, bit 1: tree too deep
-    int* depthHist_ = nullptr;  // per depth: first index of its run in the refit order (build)
+    int* depthHist_ = nullptr;  // per depth: first index of its run among levelNodes (build)
     unsigned int* boxPartial_ = nullptr;  // per-block centroid bounds (build)
     int boxPartialBlocks_ = 0;            // blocks boxPartial_ holds
     float4* external_ = nullptr;

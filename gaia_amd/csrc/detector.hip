@@ -4,7 +4,8 @@
 //   build   scene box of primitive centroids -> 30-bit Morton codes in the box (the 10-bit-per-
 //           axis interleave of BVH/MortonCode.h:9-31) with the primitive id in the low 32 bits ->
 //           device radix sort -> binary radix tree from the sorted keys (Karras 2012, HPG) ->
-//           lists of the nodes that cross blocks of leaves (the refit), node depths
+//           lists of the nodes that cross blocks of leaves (the refit); skip links (trees with a record
+//           pass) or the mesh of every node (penetration contact's face tree)
 //   refit   a block per 1,024 leaves: their boxes from the current positions and all nodes within
 //           them, climbing in LDS; then a launch per tier for nodes that cross blocks (no
 //           inter-block waits)
@@ -39,11 +40,12 @@ namespace gvbd {
 namespace {
 
 constexpr int kMaxCap = 16;       // largest per-query contact capacity
-// Traversal is stackless: every node's hi.w holds its skip link (the next node in depth-first
-// order after its subtree, -1 at the end), so a query visits left children first and follows
-// skip links; no per-thread stack lives in scratch memory.
+// Queries and the penetration searches traverse with a stack in LDS that a wave shares. The record pass
+// walks one thread per query without a stack: a node's hi.w holds its skip link (the next node in
+// depth-first order after its subtree, -1 at the end), so it visits left children first. No per-thread
+// stack lives in scratch memory.
 constexpr int kMaxDepth = 128;    // depth histogram size
-constexpr int kBlockLevel = 1024;  // refit levels of at most this many nodes share one-block launches
+constexpr int kBlockLevel = 1024;  // levels of at most this many nodes share one-block launches
 constexpr float kCmpEpsilon = 0.00001f;
 constexpr float kCmpEpsilon2 = kCmpEpsilon * kCmpEpsilon;
 constexpr float kAbsoluteRelaxation = 1e-6f;
@@ -1064,8 +1066,8 @@ __global__ __launch_bounds__(256) void depth_jump_kernel(const int* dIn, const i
 }
 
 // sort keys, deepest first: ascending (kMaxDepth - depth, node)
-__global__ __launch_bounds__(256) void depth_keys_kernel(const int* d, const int* anc, int nInternal, int* depth,
-                                                         uint64_t* keys, int* error) {
+__global__ __launch_bounds__(256) void depth_keys_kernel(const int* d, const int* anc, int nInternal, uint64_t* keys,
+                                                         int* error) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nInternal) return;
     int dpt = d[i];
@@ -1073,11 +1075,10 @@ __global__ __launch_bounds__(256) void depth_keys_kernel(const int* d, const int
         atomicOr(error, 2);
         dpt = kMaxDepth - 1;
     }
-    depth[i] = dpt;
     keys[i] = ((uint64_t)(kMaxDepth - dpt) << 32) | (uint32_t)i;
 }
 
-// node ids in refit order, and the first index of each depth's run (starts[depth], -1 if none)
+// node ids by level, deepest first, and the first index of each depth's run (starts[depth], -1 if none)
 __global__ __launch_bounds__(256) void level_nodes_kernel(const uint64_t* keys, int n, int* out, int* starts) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -2323,7 +2324,7 @@ void ContactDetector::finalize() {
     vfOffset_ = dalloc<int64_t>(nv_ + 1);
     eeOffset_ = dalloc<int64_t>(ne_ + 1);
     error_ = dalloc<int>(64);
-    depthHist_ = dalloc<int>(kMaxDepth);
+    if (pen_) depthHist_ = dalloc<int>(kMaxDepth);
     // per-block partial boxes of a tree build: the largest primitive count of any tree (faces,
     // edges, and with penetration contact the tets)
     boxPartialBlocks_ = blocks_for(std::max<int64_t>(std::max(nf_, ne_), pen_ ? (int64_t)penHost_.tetMesh.size() : 0));
@@ -2350,10 +2351,14 @@ void ContactDetector::finalize() {
         vSortTemp_ = dalloc<char>(vSortTempBytes_);
     }
     // BVH storage
-    allocBuildScratch({nf_, pen_ ? (int)penHost_.tetMesh.size() : ne_});
+    allocBuildScratch({nf_, pen_ ? (int)penHost_.tetMesh.size() : ne_}, pen_ ? nf_ : 0);
     allocBvh(fb_, nf_, !pen_);
     allocBvh(eb_, pen_ ? 0 : ne_, true);
-    if (pen_ && nf_ > 0) fb_.mesh = dalloc<int>(2 * (size_t)nf_ - 1);
+    if (pen_ && nf_ > 0) {
+        fb_.mesh = dalloc<int>(2 * (size_t)nf_ - 1);
+        fb_.levelNodes = dalloc<int>(std::max(nf_ - 1, 1));
+        fb_.dLevelBegin = dalloc<int>(kMaxDepth + 1);
+    }
     if (pen_) setupPenetrationDevice();
     hip_check(hipStreamSynchronize(stream_), "detector upload sync");
     ready_ = true;
@@ -2376,8 +2381,6 @@ void ContactDetector::allocBvh(DeviceBvh& B, int n, bool pairs) {
     B.parent = dalloc<int>(2 * (size_t)B.n - 1);
     B.right = dalloc<int>(std::max(B.n - 1, 1));
     B.keysAlt = dalloc<uint64_t>(B.n);
-    B.levelNodes = dalloc<int>(std::max(B.n - 1, 1));
-    B.dLevelBegin = dalloc<int>(kMaxDepth + 1);
     // refit lists: windows of kRefitLeaves * kRefitFan^(t + 1) leaves; a node in a window's list crosses
     // one of its inner borders, and at most kMaxRefitDepth nodes cross one border
     int64_t entries = 0;
@@ -2404,26 +2407,30 @@ void ContactDetector::allocBvh(DeviceBvh& B, int n, bool pairs) {
 }
 
 // Buffers of the tree builds, which run one after another on the detector's stream: one set, enough
-// for trees of any of the sizes.
-void ContactDetector::allocBuildScratch(const std::vector<int>& sizes) {
+// for trees of any of the sizes, one of `levelled` primitives (0: none) ordered by depth.
+void ContactDetector::allocBuildScratch(const std::vector<int>& sizes, int levelled) {
     const int n = *std::max_element(sizes.begin(), sizes.end());
     if (n == 0) return;
-    const size_t ni = (size_t)std::max(n - 1, 1);
-    scratch_.jump = dalloc<int>(4 * ni);
+    const size_t nl = (size_t)std::max(levelled - 1, 0);
+    scratch_.jump = dalloc<int>(std::max(2 * (size_t)std::max(n - 1, 1), 4 * nl));
     scratch_.keys = dalloc<uint64_t>(n);
-    scratch_.depthKeys = dalloc<uint64_t>(ni);
-    scratch_.depthKeysAlt = dalloc<uint64_t>(ni);
-    scratch_.depth = dalloc<int>(ni);
+    if (nl > 0) {
+        scratch_.depthKeys = dalloc<uint64_t>(nl);
+        scratch_.depthKeysAlt = dalloc<uint64_t>(nl);
+    }
     // a sort's temporary storage need not grow with its size: the largest over the trees
     for (int m : sizes) {
         if (m == 0) continue;
-        size_t s1 = 0, s2 = 0;
-        hip_check(rocprim::radix_sort_keys(nullptr, s1, scratch_.keys, scratch_.keys, (size_t)m, 0, 62, stream_),
+        size_t s = 0;
+        hip_check(rocprim::radix_sort_keys(nullptr, s, scratch_.keys, scratch_.keys, (size_t)m, 0, 62, stream_),
                   "sort size");
-        hip_check(rocprim::radix_sort_keys(nullptr, s2, scratch_.depthKeys, scratch_.depthKeysAlt,
-                                           (size_t)std::max(m - 1, 1), 0, 40, stream_),
+        scratch_.sortTempBytes = std::max(scratch_.sortTempBytes, s);
+    }
+    if (nl > 0) {
+        size_t s = 0;
+        hip_check(rocprim::radix_sort_keys(nullptr, s, scratch_.depthKeys, scratch_.depthKeysAlt, nl, 0, 40, stream_),
                   "sort size");
-        scratch_.sortTempBytes = std::max(scratch_.sortTempBytes, std::max(s1, s2));
+        scratch_.sortTempBytes = std::max(scratch_.sortTempBytes, s);
     }
     scratch_.sortTemp = dalloc<char>(scratch_.sortTempBytes);
 }
@@ -2473,12 +2480,31 @@ void ContactDetector::buildBvh(DeviceBvh& B, int kind, const float4* prev) {
     if (lists)
         hipLaunchKernelGGL(refit_top_entries_kernel, dim3(blocks_for(ni)), dim3(256), 0, stream_, B.nodes, B.parent,
                            B.right, ni, B.tiers, topList, topSlot, B.top);
-    hipLaunchKernelGGL(skip_kernel, dim3(blocks_for(2 * (int64_t)n - 1)), dim3(256), 0, stream_, B.nodes, B.parent,
-                       B.right, 2 * n - 1, error_);
+    if (!pen_)  // the record pass walks the skip links
+        hipLaunchKernelGGL(skip_kernel, dim3(blocks_for(2 * (int64_t)n - 1)), dim3(256), 0, stream_, B.nodes, B.parent,
+                           B.right, 2 * n - 1, error_);
     hip_check(hipGetLastError(), "bvh build launch");
-    // internal nodes by depth, deepest first
-    B.levelBegin.clear();
+    if (lists) {
+        std::vector<int> counts(lists);
+        hip_check(hipMemcpyAsync(counts.data(), B.topCount, lists * sizeof(int), hipMemcpyDeviceToHost, stream_),
+                  "list sizes");
+        hip_check(hipStreamSynchronize(stream_), "bvh build sync");
+        for (int t = 0; t < B.tiers.count; ++t) {
+            const int* c = counts.data() + B.tiers.firstList[t];
+            B.topMost[t] = *std::max_element(c, c + B.tiers.windows[t]);
+            if (B.topMost[t] > B.tiers.capacity[t]) fail(GVBD_ERR_STATE, "a refit list is longer than its bound");
+        }
+    }
+    refitBvh(B, kind, stream_, prev);
+    if (B.mesh) nodeMeshes(B);
+}
+
+// The mesh of every node of a face tree, level by level (it changes only with the tree's topology).
+void ContactDetector::nodeMeshes(DeviceBvh& B) {
+    const int n = B.n, ni = n - 1;
+    hipLaunchKernelGGL(node_mesh_leaf_kernel, dim3(blocks_for(n)), dim3(256), 0, stream_, faces_, B.nodes, n, B.mesh);
     if (ni > 0) {
+        BvhScratch& T = scratch_;
         int* d0 = T.jump;
         int* d1 = T.jump + ni;
         int* a0 = T.jump + 2 * (size_t)ni;
@@ -2489,10 +2515,10 @@ void ContactDetector::buildBvh(DeviceBvh& B, int kind, const float4* prev) {
             std::swap(d0, d1);
             std::swap(a0, a1);
         }
-        hipLaunchKernelGGL(depth_keys_kernel, dim3(blocks_for(ni)), dim3(256), 0, stream_, d0, a0, ni, T.depth,
-                           T.depthKeys, error_);
-        size_t tb2 = T.sortTempBytes;
-        hip_check(rocprim::radix_sort_keys(T.sortTemp, tb2, T.depthKeys, T.depthKeysAlt, (size_t)ni, 0, 40, stream_),
+        hipLaunchKernelGGL(depth_keys_kernel, dim3(blocks_for(ni)), dim3(256), 0, stream_, d0, a0, ni, T.depthKeys,
+                           error_);
+        size_t tb = T.sortTempBytes;
+        hip_check(rocprim::radix_sort_keys(T.sortTemp, tb, T.depthKeys, T.depthKeysAlt, (size_t)ni, 0, 40, stream_),
                   "depth sort");
         hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(256), 0, stream_, depthHist_, (int64_t)kMaxDepth, -1);
         hipLaunchKernelGGL(level_nodes_kernel, dim3(blocks_for(ni)), dim3(256), 0, stream_, T.depthKeysAlt, ni,
@@ -2500,17 +2526,9 @@ void ContactDetector::buildBvh(DeviceBvh& B, int kind, const float4* prev) {
         std::vector<int> starts(kMaxDepth, -1);
         hip_check(hipMemcpyAsync(starts.data(), depthHist_, kMaxDepth * sizeof(int), hipMemcpyDeviceToHost, stream_),
                   "level read");
-        std::vector<int> counts(lists);
-        if (lists)
-            hip_check(hipMemcpyAsync(counts.data(), B.topCount, lists * sizeof(int), hipMemcpyDeviceToHost, stream_),
-                      "list sizes");
-        hip_check(hipStreamSynchronize(stream_), "bvh build sync");
-        for (int t = 0; t < B.tiers.count; ++t) {
-            const int* c = counts.data() + B.tiers.firstList[t];
-            B.topMost[t] = *std::max_element(c, c + B.tiers.windows[t]);
-            if (B.topMost[t] > B.tiers.capacity[t]) fail(GVBD_ERR_STATE, "a refit list is longer than its bound");
-        }
+        hip_check(hipStreamSynchronize(stream_), "level sync");
         // runs are stored deepest first
+        B.levelBegin.clear();
         for (int d = kMaxDepth - 1; d >= 0; --d)
             if (starts[d] >= 0) B.levelBegin.push_back(starts[d]);
         B.levelBegin.push_back(ni);
@@ -2532,12 +2550,6 @@ void ContactDetector::buildBvh(DeviceBvh& B, int kind, const float4* prev) {
         hip_check(hipMemcpyAsync(B.dLevelBegin, B.levelBegin.data(), sizeof(int) * B.levelBegin.size(),
                                  hipMemcpyHostToDevice, stream_),
                   "level upload");
-    }
-    refitBvh(B, kind, stream_, prev);
-    if (B.mesh && kind == 0) {
-        // mesh membership changes only with the tree's topology: set at every build
-        hipLaunchKernelGGL(node_mesh_leaf_kernel, dim3(blocks_for(n)), dim3(256), 0, stream_, faces_, B.nodes, n,
-                           B.mesh);
         for (const auto& seg : B.segments) {
             const int b = B.levelBegin[seg.first], e = B.levelBegin[seg.first + 1];
             if (seg.second == seg.first + 1 && e - b > kBlockLevel)
@@ -2547,8 +2559,8 @@ void ContactDetector::buildBvh(DeviceBvh& B, int kind, const float4* prev) {
                 hipLaunchKernelGGL(node_mesh_levels_kernel, dim3(1), dim3(kBlockLevel), 0, stream_, B.levelNodes,
                                    B.dLevelBegin, seg.first, seg.second, B.nodes, B.right, B.mesh);
         }
-        hip_check(hipGetLastError(), "node mesh launch");
     }
+    hip_check(hipGetLastError(), "node mesh launch");
 }
 
 void ContactDetector::refitBvh(DeviceBvh& B, int kind, hipStream_t stream, const float4* prev, const int* gate) {
@@ -2948,7 +2960,7 @@ DetectorResultCounts ContactDetector::counts() {
     if (!ready_) fail(GVBD_ERR_STATE, "detector not finalized");
     const auto err = download(error_, 1, stream_);
     if (err[0] & 1) fail(GVBD_ERR_INTERNAL, "BVH traversal visited more nodes than the tree holds");
-    if (err[0] & 2) fail(GVBD_ERR_INTERNAL, "BVH deeper than the refit schedule supports");
+    if (err[0] & 2) fail(GVBD_ERR_INTERNAL, "BVH deeper than its keys allow");
     if (err[0] & 4) fail(GVBD_ERR_INTERNAL, "record pass found more contacts than the counting pass");
     const auto pc = download(vfPairCount_, nv_, stream_);
     const auto st = download(vfStored_, nv_, stream_);
