@@ -99,7 +99,7 @@ def solve_kernel_roofline(ctx, batch, schedule, reps=5):
         kernel = "group_solve_kernel"
     gbs = avg_bytes / (avg_ms * 1e-3) / 1e9
     out = dict(bound="hbm", achieved=round(gbs, 1), peak=HBM_PEAK_GBS, unit="GB/s",
-               frac=round(gbs / HBM_PEAK_GBS, 4), traffic=None,
+               frac=round(gbs / HBM_PEAK_GBS, 4), model="gather", traffic=None,
                kernel=kernel, avg_launch_us=round(avg_ms * 1e3, 2),
                algorithmic_bytes_per_launch=int(avg_bytes))
     if schedule["mode"] != "queue":
@@ -765,18 +765,18 @@ def main():
     log(f"batched: {batched_s / args.steps * 1e3:.2f} ms/step, {rate:.3e} vertex-solves/s")
 
     roof = solve_kernel_roofline(ctx, batch, sched)
-    # measured HBM bytes per launch (scaled PMC FETCH_SIZE + WRITE_SIZE) for this kernel,
-    # workload and schedule, from the committed profile summary
+    # `achieved` and `frac` are the gather model's, which counts neighbour positions that the caches serve
+    # (it can exceed the DRAM peak). Beside them the DRAM rate: measured HBM bytes per launch (scaled PMC
+    # FETCH_SIZE + WRITE_SIZE) of this kernel, workload and schedule from the committed profile summary over
+    # this run's launch time, left out where the summary was measured with other records
     side = os.path.join(REPO, "profiles", f"{roof['kernel']}_batched_256_scenes.traffic.json")
     if os.path.exists(side) and args.scenes == 256 and args.seed == 0:
-        t = json.load(open(side)).get("schedules", {}).get(key)
-        if t:
+        measured = json.load(open(side))
+        t = measured.get("schedules", {}).get(key)
+        if t and measured.get("algorithmic_bytes_per_launch") == roof["algorithmic_bytes_per_launch"]:
             roof["traffic"] = t["hbm_bytes_per_launch"]
-            # the gather model counts neighbour positions that the caches serve: the DRAM rate is the
-            # measured traffic's
-            roof["gather_model_gbs"] = roof["achieved"]
-            roof["achieved"] = round(t["hbm_bytes_per_launch"] / (roof["avg_launch_us"] * 1e-6) / 1e9, 1)
-            roof["frac"] = round(roof["achieved"] / HBM_PEAK_GBS, 4)
+            roof["dram_gbs"] = round(t["hbm_bytes_per_launch"] / (roof["avg_launch_us"] * 1e-6) / 1e9, 1)
+            roof["dram_frac"] = round(roof["dram_gbs"] / HBM_PEAK_GBS, 4)
     # achievable-bandwidth reference points: the library's streaming copy kernel and the runtime's
     # device-to-device copy (each moves 2 x copy_bytes per copy)
     copy_ms = ctx.stream_copy_ms(args.copy_bytes, reps=5)
