@@ -1,8 +1,8 @@
 """Small scenes stepped whole by one block each (group launches without staging) against the work
 queue, which solves the same vertices in the same order: the same bits, for every lane count, one tet,
 groups of several passes, cloth committed through positionsNext with attachments, damping, fixed
-vertices, substeps and the accelerator, scenes on both sides of the sizes that are stepped whole, alone,
-in a batch and captured."""
+vertices, substeps and the accelerator, scenes on both sides of the sizes that are stepped whole (which way a plan
+takes is asked of it), alone, in a batch and captured."""
 import numpy as np
 import pytest
 
@@ -40,9 +40,11 @@ def accelerated():
     return spec
 
 
-# 1,331 and 3,375 tet vertices and 1,600 of cloth are stepped whole with few lanes only
-SPECS = [lambda: tets(0), lambda: tets(3, iterations=0), multi_spec, accelerated, lambda: cloth(12),
-         hanging_pair_spec, lambda: tets(10, num_substeps=2), lambda: tets(14), lambda: cloth(40)]
+# scenes, and the most lanes per vertex with which they are stepped whole (1,331 and 3,375 tet vertices and 1,600 of
+# cloth: few, where their groups take one pass of a block's waves on average)
+SPECS = [(lambda: tets(0), 16), (lambda: tets(3, iterations=0), 16), (multi_spec, 16), (accelerated, 16),
+         (lambda: cloth(12), 16), (hanging_pair_spec, 16), (lambda: tets(10, num_substeps=2), 4), (lambda: tets(14), 2),
+         (lambda: cloth(40), 2)]
 
 
 def states(sims):
@@ -53,9 +55,10 @@ def states(sims):
 def test_whole_frames_equal_the_work_queue(gpu_ctx, lanes):
     runs = {}
     for mode, graph in (("queue", False), ("group", False), ("group", True)):
-        sims = [build_gpu(gpu_ctx, s()) for s in SPECS]
-        for s in sims:
+        sims = [build_gpu(gpu_ctx, s()) for s, _ in SPECS]
+        for s, (_, most) in zip(sims, SPECS):
             s.setSchedule(lanes, 256, mode=mode)
+            assert s.planInfo()[0] == (mode == "group" and lanes <= most)
             if graph:
                 s.recordVBDSolveGraph(True)
             for _ in range(3):
@@ -77,6 +80,7 @@ def test_batch_stepped_whole_equals_the_scenes_alone(gpu_ctx):
         if batched:
             b = Batch(gpu_ctx, sims)
             b.set_schedule(4, 256)
+            assert b.plan_info()[0]
             b.run_steps(3)
         else:
             for s in sims:
