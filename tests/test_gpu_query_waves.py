@@ -29,7 +29,8 @@ CASES = {
     "crowd of 3": lambda: crowd(3) + [(np.array([[9, 9, 9], [9.1, 9, 9], [9, 9.1, 9]], np.float32), np.array([[0, 1, 2]], np.int32))],
     "8 per wave": lambda: tori(2, 40, 20),
     "16 per wave": lambda: tori(2, 128, 63),  # 64,512 vertices, 193,536 edges
-    "32 per wave": lambda: tori(3, 120, 60),  # 194,400 vertices, 583,200 edges
+    "32 edges per wave": lambda: tori(3, 120, 60),  # 194,400 vertices (16 per wave), 583,200 edges
+    "32 per wave": lambda: tori(4, 66, 63),  # 266,112 vertices, 798,336 edges
 }
 
 
