@@ -634,7 +634,7 @@ struct RefChunk {
 // primitive each and find their pairs with shuffles, so the loads of a vertex's primitives overlap
 // and the pairs of a round are evaluated side by side. (Read in turn by every lane, two dependent
 // loads for each of a surface vertex's 12 or so primitives, they were half of the launch: 42 us per
-// launch before, 20 us now with 8 bodies of 5,000 tets on a 61 x 61 sheet, 22.4 us and 12.6 us with
+// launch before, 18.9 us now with 8 bodies of 5,000 tets on a 61 x 61 sheet, 22.4 us and 11.6 us with
 // 32 bodies of 8,640 tets and penetration contact; 16 lanes, 256 threads.) The LPV lanes of a vertex
 // are active together and take the same branches around the shuffles.
 template <int LPV, class Load, class Body>
