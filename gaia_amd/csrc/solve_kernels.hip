@@ -254,7 +254,7 @@ __device__ __forceinline__ void tet_block(const SceneView& S, float4* posInOut, 
         gzz += ag.z * t.g.z;
         cmu += Amu * t.mm;
     };
-    if (S.trow) {
+    if (CONTACT || S.trow) {  // (contact scenes always have rows)
         const float* __restrict__ tvol = S.tvol;
         for_lane_records<LPV, STAGE, 3>(S.trow.as<const float4>(), blockBegin, blockEnd, slot.y + sub,
                                         slot.z, lds, [&](const float4* r, int k) {
