@@ -399,6 +399,14 @@ struct TetRecords {
     std::vector<TetRow> row;
     std::vector<float> vol;  // per row record
     size_t size() const { return rows ? row.size() : inc.size(); }
+    void reserve(size_t n) {
+        if (rows) {
+            row.reserve(n);
+            vol.reserve(n);
+        } else {
+            inc.reserve(n);
+        }
+    }
 };
 
 void emit_tet_slot(const TetMeshHost& m, int32_t off, int32_t lv, int32_t mat, std::vector<int4>& slots,
@@ -556,6 +564,9 @@ void upload_scene(gvbd_context* ctx, SceneObj& s, const std::function<void(size_
     recs.rows = s.params.use_accelerator != 0 || s.params.handle_collision != 0;
     for (const TetMeshHost& m : s.tets)
         if (m.mat.dampingHydrostatic != 0.f || m.mat.dampingDeviatoric != 0.f) recs.rows = true;
+    size_t incidences = 0;
+    for (const TetMeshHost& m : s.tets) incidences += 4 * (size_t)m.nt;
+    recs.reserve(incidences);
     std::vector<ClothSlot> cslots;
     std::vector<FaceInc> cface;
     std::vector<BendInc> cbend;
